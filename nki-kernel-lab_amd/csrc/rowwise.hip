@@ -7,12 +7,20 @@
 // Outputs are written with non-temporal (streaming) stores, which reach HBM
 // faster than write-back stores for data the kernel never reads again.
 //
-// Layout: one 64-lane wavefront owns one row; a 256-thread workgroup owns 4
-// rows.  Each lane keeps NV 16-byte vectors of its row in registers, so a row
-// is read from HBM exactly once and the reductions are wavefront shuffles.
-// Rows too long for the register cache, or not 16-byte aligned, take the
-// looped kernels, which re-read the row (from L2) once per pass.
+// Layout: a row is held in registers by 1, 4 or 16 wavefronts (pick_row), each
+// lane with NV 16-byte vectors, so it is read from HBM exactly once and the
+// reductions are wavefront shuffles (and one LDS exchange per reduction when
+// several wavefronts share the row).  Rows whose length, stride or base is off
+// 16 bytes are read and written with the same 16-byte instructions at the
+// element's own alignment (gfx950 takes them at any address); the elements
+// ahead of the row's first 64-byte boundary and its last ones go one to a
+// lane.  One wavefront per row with element loads and three sweeps took 316 us
+// at 1000 x 20000 fp32 and 252 at 66 x 31363; sixteen wavefronts holding the
+// row take 35.3 (4.5 TB/s) and 6.8.  Rows past 65536 elements take the looped
+// kernels, which re-read the row (from L2) once per pass.
 #include <math.h>
+
+#include <type_traits>
 
 #include "common.h"
 
@@ -20,36 +28,138 @@ namespace nkl {
 
 constexpr int kRowsPerBlock = 4;
 
+// 16 bytes at the alignment of T only.
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+typedef u32x4 u32x4_a4 __attribute__((aligned(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
+
+__device__ __forceinline__ u32x4 ld16_any(const float* p) { return *reinterpret_cast<const u32x4_a4*>(p); }
+__device__ __forceinline__ u32x4 ld16_any(const bf16* p) { return *reinterpret_cast<const u32x4_a2*>(p); }
+__device__ __forceinline__ void unpack16(u32x4 t, float (&v)[4]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = __uint_as_float(t[i]);
+}
+__device__ __forceinline__ void unpack16(u32x4 t, float (&v)[8]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[2 * i] = bf16lo(t[i]), v[2 * i + 1] = bf16hi(t[i]);
+}
+
+// E elements at p as fp32 values (AL: p is 16-byte aligned).
+template <bool AL, typename T, int E>
+__device__ __forceinline__ void load_row_vec(const T* p, float (&v)[E]) {
+  if constexpr (AL)
+    load16(p, v);
+  else
+    unpack16(ld16_any(p), v);
+}
+
+// E fp32 values to p as T (E = 4 or 8), streaming.
+template <bool AL, typename T, int E>
+__device__ __forceinline__ void store_row_vec(T* p, const float (&v)[E]) {
+  if constexpr (AL) {
+    store_vec_nt<E>(p, v);
+  } else if constexpr (sizeof(T) == 4) {
+#pragma unroll
+    for (int i = 0; i < E; i += 4) {
+      const u32x4 t = {__float_as_uint(v[i]), __float_as_uint(v[i + 1]), __float_as_uint(v[i + 2]),
+                       __float_as_uint(v[i + 3])};
+      __builtin_nontemporal_store(t, reinterpret_cast<u32x4_a4*>(p + i));
+    }
+  } else {
+    auto pack = [](float a, float b) {
+      if constexpr (std::is_same<T, bf16>::value)
+        return pack_bf16x2(a, b);
+      else
+        return pack_f16x2(a, b);
+    };
+    if constexpr (E == 8) {
+      const u32x4 t = {pack(v[0], v[1]), pack(v[2], v[3]), pack(v[4], v[5]), pack(v[6], v[7])};
+      __builtin_nontemporal_store(t, reinterpret_cast<u32x4_a2*>(p));
+    } else {
+      const u32x2 t = {pack(v[0], v[1]), pack(v[2], v[3])};
+      __builtin_nontemporal_store(t, reinterpret_cast<u32x2_a2*>(p));
+    }
+  }
+}
+
+// Elements of a row ahead of its first 64-byte boundary in y: the vectors start
+// there, so that whole-vector stores do not straddle lines (4097 x 2049 bf16
+// softmax 7.6 us, 8.0 with vectors from the row's first element; 500 x 20001
+// fp32 17.3, 17.8 from the first 16-byte boundary).
+template <typename T>
+__device__ __forceinline__ int row_head(const T* y, int cols) {
+  return min(cols, (int)((0u - (unsigned)(uintptr_t)y) % 64 / sizeof(T)));
+}
+
+// max / sum over the WPR wavefronts of a row (WPR > 1: the whole workgroup;
+// `red` is one of the kernel's LDS arrays, used once).
+template <int WPR>
+__device__ __forceinline__ float row_max(float v, float* red) {
+  v = wave_max(v);
+  if constexpr (WPR > 1) {
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = red[0];
+#pragma unroll
+    for (int i = 1; i < WPR; ++i) v = fmaxf(v, red[i]);
+  }
+  return v;
+}
+template <int WPR>
+__device__ __forceinline__ float row_sum(float v, float* red) {
+  v = wave_sum(v);
+  if constexpr (WPR > 1) {
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = red[0];
+#pragma unroll
+    for (int i = 1; i < WPR; ++i) v += red[i];
+  }
+  return v;
+}
+
 // ------------------------------------------------------------- softmax --
 // nkilab/kernels/norm.py:65-89: neg_max = -max(x); e = exp(x + neg_max) with
 // the row sum in fp32; rinv = 1 / sum; y = e * rinv rounded once.
-template <typename T, int NV>
-__global__ __launch_bounds__(256) void softmax_vec_kernel(const T* __restrict__ x, T* __restrict__ y,
-                                                          int rows, int cols, long ldx, long ldy) {
+template <typename T, int WPR, int NV, bool AL>
+__global__ __launch_bounds__(WPR == 1 ? 256 : 64 * WPR) void softmax_vec_kernel(const T* __restrict__ x,
+                                                                                T* __restrict__ y, int rows, int cols,
+                                                                                long ldx, long ldy) {
   constexpr int E = VecE<T>::value;
-  const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
-  if (row >= rows) return;
+  __shared__ float red[2][WPR];
+  const int t = WPR == 1 ? threadIdx.x & 63 : threadIdx.x;
+  const int row = WPR == 1 ? blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6) : blockIdx.x;
+  if (row >= rows) return;  // WPR > 1: one row per workgroup, never taken
   const T* xr = x + (long)row * ldx;
   T* yr = y + (long)row * ldy;
-  const int nvec = cols / E;
+  const int head = AL ? 0 : row_head(yr, cols);
+  const int nvec = (cols - head) / E, edge = AL ? 0 : cols - nvec * E;
+  // Edge element of lane t < edge: the row's first head, then its last ones.
+  const int te = t < head ? t : nvec * E + t;
   float v[NV][E];
-  float mx = -INFINITY;
 #pragma unroll
   for (int n = 0; n < NV; ++n) {
-    const int vi = n * kWave + lane;
+    const int vi = n * 64 * WPR + t;
     if (vi < nvec) {
-      load16(xr + (long)vi * E, v[n]);
+      load_row_vec<AL>(xr + head + vi * E, v[n]);
     } else {
 #pragma unroll
       for (int e = 0; e < E; ++e) v[n][e] = -INFINITY;
     }
+  }
+  float tv = -INFINITY;
+  if (t < edge) tv = to_f32(xr[te]);
+  float mx = tv;
+#pragma unroll
+  for (int n = 0; n < NV; ++n)
 #pragma unroll
     for (int e = 0; e < E; ++e) mx = fmaxf(mx, v[n][e]);
-  }
-  mx = wave_max(mx);
+  mx = row_max<WPR>(mx, red[0]);
   const float mx2 = mx * kLog2e;
   float sum = 0.f;
+  if constexpr (!AL) sum = tv = fast_exp2(fmaf(tv, kLog2e, -mx2));
 #pragma unroll
   for (int n = 0; n < NV; ++n)
 #pragma unroll
@@ -57,39 +167,57 @@ __global__ __launch_bounds__(256) void softmax_vec_kernel(const T* __restrict__ 
       v[n][e] = fast_exp2(fmaf(v[n][e], kLog2e, -mx2));
       sum += v[n][e];
     }
-  sum = wave_sum(sum);
+  sum = row_sum<WPR>(sum, red[1]);
   const float rinv = 1.0f / sum;
 #pragma unroll
   for (int n = 0; n < NV; ++n) {
-    const int vi = n * kWave + lane;
+    const int vi = n * 64 * WPR + t;
     if (vi < nvec) {
       float o[E];
 #pragma unroll
       for (int e = 0; e < E; ++e) o[e] = v[n][e] * rinv;
-      store_vec_nt<E>(yr + (long)vi * E, o);
+      store_row_vec<AL>(yr + head + vi * E, o);
     }
   }
+  if (t < edge) yr[te] = from_f32<T>(tv * rinv);
 }
 
-// Any length / alignment: one wavefront per row, three sweeps over the row.
+// Rows too long for registers: one 1024-thread workgroup per row, three sweeps
+// over the row.
 template <typename T>
-__global__ __launch_bounds__(256) void softmax_loop_kernel(const T* __restrict__ x, T* __restrict__ y,
-                                                           int rows, int cols, long ldx, long ldy) {
-  const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const T* xr = x + (long)row * ldx;
-  T* yr = y + (long)row * ldy;
-  float mx = -INFINITY;
-  for (int c = lane; c < cols; c += kWave) mx = fmaxf(mx, to_f32(xr[c]));
-  mx = wave_max(mx);
+__global__ __launch_bounds__(1024) void softmax_loop_kernel(const T* __restrict__ x, T* __restrict__ y, int cols,
+                                                            long ldx, long ldy) {
+  constexpr int E = VecE<T>::value;
+  __shared__ float red[2][16];
+  const T* xr = x + (long)blockIdx.x * ldx;
+  T* yr = y + (long)blockIdx.x * ldy;
+  const int t = threadIdx.x, nvec = cols / E, tail = cols - nvec * E;
+  float v[E];
+  float tv = -INFINITY;
+  if (t < tail) tv = to_f32(xr[(long)nvec * E + t]);
+  float mx = tv;
+  for (int vi = t; vi < nvec; vi += 1024) {
+    load_row_vec<false>(xr + (long)vi * E, v);
+#pragma unroll
+    for (int e = 0; e < E; ++e) mx = fmaxf(mx, v[e]);
+  }
+  mx = row_max<16>(mx, red[0]);
   const float mx2 = mx * kLog2e;
-  float sum = 0.f;
-  for (int c = lane; c < cols; c += kWave) sum += fast_exp2(fmaf(to_f32(xr[c]), kLog2e, -mx2));
-  sum = wave_sum(sum);
+  float sum = tv = fast_exp2(fmaf(tv, kLog2e, -mx2));
+  for (int vi = t; vi < nvec; vi += 1024) {
+    load_row_vec<false>(xr + (long)vi * E, v);
+#pragma unroll
+    for (int e = 0; e < E; ++e) sum += fast_exp2(fmaf(v[e], kLog2e, -mx2));
+  }
+  sum = row_sum<16>(sum, red[1]);
   const float rinv = 1.0f / sum;
-  for (int c = lane; c < cols; c += kWave)
-    yr[c] = from_f32<T>(fast_exp2(fmaf(to_f32(xr[c]), kLog2e, -mx2)) * rinv);
+  for (int vi = t; vi < nvec; vi += 1024) {
+    load_row_vec<false>(xr + (long)vi * E, v);
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = fast_exp2(fmaf(v[e], kLog2e, -mx2)) * rinv;
+    store_row_vec<false>(yr + (long)vi * E, v);
+  }
+  if (t < tail) yr[(long)nvec * E + t] = from_f32<T>(tv * rinv);
 }
 
 // ---------------------------------------------------- three-pass softmax --
@@ -143,86 +271,108 @@ __global__ __launch_bounds__(256) void softmax_pass3_kernel(const float* __restr
 // ------------------------------------------------------------- RMSNorm --
 // nkilab/kernels/norm.py:92-118: ssq = sum(x^2) (fp32); ms = ssq * (1/D) + eps;
 // rstd = rsqrt(ms); xn = x * rstd (fp32); y = xn * w rounded once.
-// E weight elements of type TW (16-byte aligned) as fp32 values.
-template <int E>
+// E weight elements of type TW as fp32 values.
+template <bool AL, int E>
 __device__ __forceinline__ void load_w(const float* p, float (&v)[E]) {
 #pragma unroll
   for (int i = 0; i < E; i += 4) {
     float t[4];
-    load16(p + i, t);
+    load_row_vec<AL>(p + i, t);
 #pragma unroll
     for (int k = 0; k < 4; ++k) v[i + k] = t[k];
   }
 }
-template <int E>
+template <bool AL, int E>
 __device__ __forceinline__ void load_w(const bf16* p, float (&v)[E]) {
   if constexpr (E == 8) {
-    load16(p, v);
+    load_row_vec<AL>(p, v);
   } else {
     static_assert(E == 4, "4 or 8 weights per vector");
-    const uint2 t = *reinterpret_cast<const uint2*>(p);
-    v[0] = bf16lo(t.x), v[1] = bf16hi(t.x), v[2] = bf16lo(t.y), v[3] = bf16hi(t.y);
+    const u32x2 t = AL ? *reinterpret_cast<const u32x2*>(p) : *reinterpret_cast<const u32x2_a2*>(p);
+    v[0] = bf16lo(t[0]), v[1] = bf16hi(t[0]), v[2] = bf16lo(t[1]), v[3] = bf16hi(t[1]);
   }
 }
 
-template <typename TI, typename TW, typename TO, int NV>
-__global__ __launch_bounds__(256) void rmsnorm_vec_kernel(const TI* __restrict__ x, const TW* __restrict__ w,
-                                                          TO* __restrict__ y, int rows, int cols, long ldx,
-                                                          long ldy, float inv_d, float eps) {
+template <typename TI, typename TW, typename TO, int WPR, int NV, bool AL>
+__global__ __launch_bounds__(WPR == 1 ? 256 : 64 * WPR) void rmsnorm_vec_kernel(
+    const TI* __restrict__ x, const TW* __restrict__ w, TO* __restrict__ y, int rows, int cols, long ldx, long ldy,
+    float inv_d, float eps) {
   constexpr int E = VecE<TI>::value;
-  const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
-  if (row >= rows) return;
+  __shared__ float red[WPR];
+  const int t = WPR == 1 ? threadIdx.x & 63 : threadIdx.x;
+  const int row = WPR == 1 ? blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6) : blockIdx.x;
+  if (row >= rows) return;  // WPR > 1: one row per workgroup, never taken
   const TI* xr = x + (long)row * ldx;
   TO* yr = y + (long)row * ldy;
-  const int nvec = cols / E;
+  const int head = AL ? 0 : row_head(yr, cols);
+  const int nvec = (cols - head) / E, edge = AL ? 0 : cols - nvec * E;
+  // Edge element of lane t < edge: the row's first head, then its last ones.
+  const int te = t < head ? t : nvec * E + t;
   float v[NV][E];
-  float ssq = 0.f;
 #pragma unroll
   for (int n = 0; n < NV; ++n) {
-    const int vi = n * kWave + lane;
+    const int vi = n * 64 * WPR + t;
     if (vi < nvec) {
-      load16(xr + (long)vi * E, v[n]);
+      load_row_vec<AL>(xr + head + vi * E, v[n]);
     } else {
 #pragma unroll
       for (int e = 0; e < E; ++e) v[n][e] = 0.f;
     }
+  }
+  float tv = 0.f;
+  if (t < edge) tv = to_f32(xr[te]);
+  float ssq = tv * tv;
+#pragma unroll
+  for (int n = 0; n < NV; ++n)
 #pragma unroll
     for (int e = 0; e < E; ++e) ssq = fmaf(v[n][e], v[n][e], ssq);
-  }
-  ssq = wave_sum(ssq);
+  ssq = row_sum<WPR>(ssq, red);
   const float rstd = __frsqrt_rn(fmaf(ssq, inv_d, eps));
 #pragma unroll
   for (int n = 0; n < NV; ++n) {
-    const int vi = n * kWave + lane;
+    const int vi = n * 64 * WPR + t;
     if (vi < nvec) {
       float wv[E];
-      load_w<E>(w + (long)vi * E, wv);
+      load_w<AL>(w + head + vi * E, wv);
       float o[E];
 #pragma unroll
       for (int e = 0; e < E; ++e) o[e] = (v[n][e] * rstd) * wv[e];
-      store_vec_nt<E>(yr + (long)vi * E, o);
+      store_row_vec<AL>(yr + head + vi * E, o);
     }
   }
+  if (t < edge) yr[te] = from_f32<TO>((tv * rstd) * to_f32(w[te]));
 }
 
+// Rows too long for registers: one 1024-thread workgroup per row, two sweeps.
 template <typename TI, typename TW, typename TO>
-__global__ __launch_bounds__(256) void rmsnorm_loop_kernel(const TI* __restrict__ x, const TW* __restrict__ w,
-                                                           TO* __restrict__ y, int rows, int cols, long ldx,
-                                                           long ldy, float inv_d, float eps) {
-  const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const TI* xr = x + (long)row * ldx;
-  TO* yr = y + (long)row * ldy;
-  float ssq = 0.f;
-  for (int c = lane; c < cols; c += kWave) {
-    const float t = to_f32(xr[c]);
-    ssq = fmaf(t, t, ssq);
+__global__ __launch_bounds__(1024) void rmsnorm_loop_kernel(const TI* __restrict__ x, const TW* __restrict__ w,
+                                                            TO* __restrict__ y, int cols, long ldx, long ldy,
+                                                            float inv_d, float eps) {
+  constexpr int E = VecE<TI>::value;
+  __shared__ float red[16];
+  const TI* xr = x + (long)blockIdx.x * ldx;
+  TO* yr = y + (long)blockIdx.x * ldy;
+  const int t = threadIdx.x, nvec = cols / E, tail = cols - nvec * E;
+  float v[E];
+  float tv = 0.f;
+  if (t < tail) tv = to_f32(xr[(long)nvec * E + t]);
+  float ssq = tv * tv;
+  for (int vi = t; vi < nvec; vi += 1024) {
+    load_row_vec<false>(xr + (long)vi * E, v);
+#pragma unroll
+    for (int e = 0; e < E; ++e) ssq = fmaf(v[e], v[e], ssq);
   }
-  ssq = wave_sum(ssq);
+  ssq = row_sum<16>(ssq, red);
   const float rstd = __frsqrt_rn(fmaf(ssq, inv_d, eps));
-  for (int c = lane; c < cols; c += kWave) yr[c] = from_f32<TO>((to_f32(xr[c]) * rstd) * to_f32(w[c]));
+  for (int vi = t; vi < nvec; vi += 1024) {
+    float wv[E];
+    load_row_vec<false>(xr + (long)vi * E, v);
+    load_w<false>(w + (long)vi * E, wv);
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = (v[e] * rstd) * wv[e];
+    store_row_vec<false>(yr + (long)vi * E, v);
+  }
+  if (t < tail) yr[(long)nvec * E + t] = from_f32<TO>((tv * rstd) * to_f32(w[(long)nvec * E + t]));
 }
 
 // -------------------------------------------------------------- SwiGLU --
@@ -267,56 +417,104 @@ __global__ __launch_bounds__(256) void swiglu_tail_kernel(const T* __restrict__ 
 // ------------------------------------------------------------ dispatch --
 static bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
-// Smallest register-cache depth (vectors per lane) that holds a row of nvec
-// 16-byte vectors; 0 when the row is longer than the deepest variant.
-static int pick_nv(int nvec) {
-  for (int nv = 1; nv <= 16; nv *= 2)
-    if (nvec <= nv * kWave) return nv;
-  return 0;
+// Wavefronts per row and vectors per lane (a power of two) that hold a row of
+// nvec 16-byte vectors in registers; nv = 0 when it is longer than 16
+// wavefronts hold (64 values a lane).
+//
+// One wavefront holds up to 16 vectors a lane; four share the row when that
+// fills the chip sooner: from 4 vectors a lane while every row's workgroup
+// fits one round (2048 of 256 threads; rotated inputs, us, one wavefront /
+// four: softmax 1536 x 2048 bf16 5.2 / 4.7, RMSNorm 5.2 / 4.3, 2048 x 2048
+// fp32 -> fp16 6.3 / 5.7; past one round one wavefront is level or ahead: 3000
+// x 2048 bf16 softmax 5.7 / 6.3).  Sixteen vectors a lane turn at `deep_rows`
+// (fp32 softmax 1024 x 4096 7.6 / 6.0 but 1536 x 4096 9.0 / 9.7), and in 16
+// bits, 128 values a lane, always go to four (4096 x 8192 26.0 / 22.1).
+struct RowPlan {
+  int wpr, nv;
+};
+template <typename T>
+static RowPlan pick_row(int rows, int cols, int deep_rows) {
+  constexpr int E = VecE<T>::value;
+  const int nvec = cols / E;  // full vectors: the edges of an unaligned row ride in one more register
+  for (int wpr : {1, 4, 16}) {
+    const int cap = wpr == 16 ? 64 / E : 16;
+    for (int nv = 1; nv <= cap; nv *= 2) {
+      if (nvec > nv * 64 * wpr) continue;
+      if (wpr == 1 && nv >= 4 && (rows <= (nv == 16 ? deep_rows : 2048) || nv * E > 64)) return RowPlan{4, nv / 4};
+      return RowPlan{wpr, nv};
+    }
+  }
+  return RowPlan{16, 0};
+}
+
+// Calls f(wpr, nv) with the plan's values as compile-time constants; false
+// when the plan is the looped kernel's.
+template <typename T, typename F>
+static bool with_row_plan(RowPlan p, F f) {
+#define NKL_ROW(W, N)                                                        \
+  if (p.wpr == W && p.nv == N) {                                             \
+    f(std::integral_constant<int, W>{}, std::integral_constant<int, N>{});   \
+    return true;                                                             \
+  }
+  NKL_ROW(1, 1) NKL_ROW(1, 2) NKL_ROW(1, 4) NKL_ROW(1, 8)
+  if constexpr (VecE<T>::value == 4) { NKL_ROW(1, 16) }
+  NKL_ROW(4, 1) NKL_ROW(4, 2) NKL_ROW(4, 4) NKL_ROW(4, 8) NKL_ROW(4, 16)
+  NKL_ROW(16, 8)
+  if constexpr (VecE<T>::value == 4) { NKL_ROW(16, 16) }
+#undef NKL_ROW
+  return false;
 }
 
 template <typename T>
-static int softmax_launch(const void* x, void* y, int rows, int cols, long ldx, long ldy, hipStream_t st) {
+static int softmax_launch_plan(RowPlan plan, const void* x, void* y, int rows, int cols, long ldx, long ldy,
+                               hipStream_t st) {
   constexpr int E = VecE<T>::value;
-  const dim3 grid((rows + kRowsPerBlock - 1) / kRowsPerBlock), block(256);
   const T* xp = static_cast<const T*>(x);
   T* yp = static_cast<T*>(y);
-  const bool vec = cols % E == 0 && ldx % E == 0 && ldy % E == 0 && aligned16(x) && aligned16(y);
-  const int nv = vec ? pick_nv(cols / E) : 0;
-  switch (nv) {
-    case 1: softmax_vec_kernel<T, 1><<<grid, block, 0, st>>>(xp, yp, rows, cols, ldx, ldy); break;
-    case 2: softmax_vec_kernel<T, 2><<<grid, block, 0, st>>>(xp, yp, rows, cols, ldx, ldy); break;
-    case 4: softmax_vec_kernel<T, 4><<<grid, block, 0, st>>>(xp, yp, rows, cols, ldx, ldy); break;
-    case 8: softmax_vec_kernel<T, 8><<<grid, block, 0, st>>>(xp, yp, rows, cols, ldx, ldy); break;
-    case 16: softmax_vec_kernel<T, 16><<<grid, block, 0, st>>>(xp, yp, rows, cols, ldx, ldy); break;
-    default: softmax_loop_kernel<T><<<grid, block, 0, st>>>(xp, yp, rows, cols, ldx, ldy); break;
-  }
+  const bool al = cols % E == 0 && ldx % E == 0 && ldy % E == 0 && aligned16(x) && aligned16(y);
+  const bool done = with_row_plan<T>(plan, [&](auto W, auto N) {
+    constexpr int WPR = decltype(W)::value, NV = decltype(N)::value;
+    const dim3 grid(WPR == 1 ? (rows + kRowsPerBlock - 1) / kRowsPerBlock : rows), block(WPR == 1 ? 256 : 64 * WPR);
+    if (al)
+      softmax_vec_kernel<T, WPR, NV, true><<<grid, block, 0, st>>>(xp, yp, rows, cols, ldx, ldy);
+    else
+      softmax_vec_kernel<T, WPR, NV, false><<<grid, block, 0, st>>>(xp, yp, rows, cols, ldx, ldy);
+  });
+  if (!done) softmax_loop_kernel<T><<<dim3(rows), dim3(1024), 0, st>>>(xp, yp, cols, ldx, ldy);
   return check_launch("nkl_softmax");
+}
+template <typename T>
+static int softmax_launch(const void* x, void* y, int rows, int cols, long ldx, long ldy, hipStream_t st) {
+  return softmax_launch_plan<T>(pick_row<T>(rows, cols, 1280), x, y, rows, cols, ldx, ldy, st);
 }
 
 template <typename TI, typename TW, typename TO>
-static int rmsnorm_launch(const void* x, const void* w, void* y, int rows, int cols, long ldx, long ldy,
-                          float eps, hipStream_t st) {
+static int rmsnorm_launch_plan(RowPlan plan, const void* x, const void* w, void* y, int rows, int cols, long ldx,
+                               long ldy, float eps, hipStream_t st) {
   constexpr int E = VecE<TI>::value;
-  const dim3 grid((rows + kRowsPerBlock - 1) / kRowsPerBlock), block(256);
   const TI* xp = static_cast<const TI*>(x);
   const TW* wp = static_cast<const TW*>(w);
   TO* yp = static_cast<TO*>(y);
   // The multiplier 1/D is the fp32 value nearest the exact quotient.
   const float inv_d = (float)(1.0 / (double)cols);
-  const bool out_vec = (E * sizeof(TO)) % 8 == 0;
-  const bool vec = out_vec && cols % E == 0 && ldx % E == 0 && ldy % E == 0 && aligned16(x) &&
-                   aligned16(w) && aligned16(y);
-  const int nv = vec ? pick_nv(cols / E) : 0;
-  switch (nv) {
-    case 1: rmsnorm_vec_kernel<TI, TW, TO, 1><<<grid, block, 0, st>>>(xp, wp, yp, rows, cols, ldx, ldy, inv_d, eps); break;
-    case 2: rmsnorm_vec_kernel<TI, TW, TO, 2><<<grid, block, 0, st>>>(xp, wp, yp, rows, cols, ldx, ldy, inv_d, eps); break;
-    case 4: rmsnorm_vec_kernel<TI, TW, TO, 4><<<grid, block, 0, st>>>(xp, wp, yp, rows, cols, ldx, ldy, inv_d, eps); break;
-    case 8: rmsnorm_vec_kernel<TI, TW, TO, 8><<<grid, block, 0, st>>>(xp, wp, yp, rows, cols, ldx, ldy, inv_d, eps); break;
-    case 16: rmsnorm_vec_kernel<TI, TW, TO, 16><<<grid, block, 0, st>>>(xp, wp, yp, rows, cols, ldx, ldy, inv_d, eps); break;
-    default: rmsnorm_loop_kernel<TI, TW, TO><<<grid, block, 0, st>>>(xp, wp, yp, rows, cols, ldx, ldy, inv_d, eps); break;
-  }
+  const bool al = cols % E == 0 && ldx % E == 0 && ldy % E == 0 && aligned16(x) && aligned16(w) && aligned16(y);
+  const bool done = with_row_plan<TI>(plan, [&](auto W, auto N) {
+    constexpr int WPR = decltype(W)::value, NV = decltype(N)::value;
+    const dim3 grid(WPR == 1 ? (rows + kRowsPerBlock - 1) / kRowsPerBlock : rows), block(WPR == 1 ? 256 : 64 * WPR);
+    if (al)
+      rmsnorm_vec_kernel<TI, TW, TO, WPR, NV, true><<<grid, block, 0, st>>>(xp, wp, yp, rows, cols, ldx, ldy, inv_d,
+                                                                            eps);
+    else
+      rmsnorm_vec_kernel<TI, TW, TO, WPR, NV, false><<<grid, block, 0, st>>>(xp, wp, yp, rows, cols, ldx, ldy, inv_d,
+                                                                             eps);
+  });
+  if (!done) rmsnorm_loop_kernel<TI, TW, TO><<<dim3(rows), dim3(1024), 0, st>>>(xp, wp, yp, cols, ldx, ldy, inv_d, eps);
   return check_launch("nkl_rmsnorm");
+}
+template <typename TI, typename TW, typename TO>
+static int rmsnorm_launch(const void* x, const void* w, void* y, int rows, int cols, long ldx, long ldy, float eps,
+                          hipStream_t st) {
+  return rmsnorm_launch_plan<TI, TW, TO>(pick_row<TI>(rows, cols, 2048), x, w, y, rows, cols, ldx, ldy, eps, st);
 }
 
 template <typename T>
@@ -353,7 +551,6 @@ static int swiglu_launch(const void* g, const void* u, void* y, long n, hipStrea
 // (and of per-workgroup contiguous chunks) at 16 - 128 MiB on MI355X.  It
 // measures the HBM ceiling the row kernels' roofline is read against at the
 // same size.
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kCopyUnroll = 2;
 __global__ __launch_bounds__(256) void stream_copy_kernel(const u32x4* __restrict__ x, u32x4* __restrict__ y, long n) {
   const long base = (long)blockIdx.x * 256 + threadIdx.x, span = (long)gridDim.x * 256;

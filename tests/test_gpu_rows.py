@@ -243,3 +243,55 @@ def test_stream_copy_is_exact(nbytes):
     torch.cuda.synchronize()
     assert torch.equal(y[:nbytes], x[:nbytes])
     assert bool((y[nbytes:] == 7).all())
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("R,D", [(1, 1), (3, 7), (2049, 257), (5, 1025), (2048, 1024), (2049, 2048), (7, 4097),
+                                 (1281, 4096), (3, 8191), (5, 16384), (2, 16389), (9, 31363), (2, 65536), (2, 70003)])
+def test_row_kernels_at_every_plan(dt, R, D):
+    """softmax and RMSNorm on rows held by 1, 4 and 16 wavefronts and by the
+    looped kernels, contiguous and as views whose rows start off 16 bytes
+    (another offset for x than for y), against float64.  fp32: 1e-5 relative
+    (row sums of up to 7e4 positive terms in a tree: below 40 roundings of
+    2^-24 and the exponential's 2^-22); bf16: one ulp of the exact value."""
+    from nkilab import ops
+
+    g = torch.Generator(device="cuda").manual_seed(R * 100003 + D)
+    for off_x, off_y in ((0, 0), (3, 1)):
+        xb = (torch.randn(R, D + 9, generator=g, device="cuda") * 3).to(dt)
+        x = xb[:, off_x:off_x + D] if off_x else xb[:, :D].contiguous()
+        yb = torch.full((R, D + 5), 7.0, dtype=dt, device="cuda")
+        y = yb[:, off_y:off_y + D] if off_y else torch.empty(R, D, dtype=dt, device="cuda")
+        ops.softmax_into(x, y)
+        ref = torch.softmax(x.double(), -1)
+        w = (torch.randn(D + 1, generator=g, device="cuda") * 0.1 + 1).to(dt)[off_y:off_y + D]
+        n = torch.empty(R, D, dtype=dt, device="cuda")
+        ops.rmsnorm_into(x, w, n)
+        xd = x.double()
+        nref = xd * torch.rsqrt(xd.pow(2).mean(-1, keepdim=True) + 1e-6) * w.double()
+        if dt == torch.float32:
+            assert ((y.double() - ref).abs() <= 1e-5 * ref).all()
+            assert ((n.double() - nref).abs() <= 1e-5 * nref.abs()).all()
+        else:
+            assert_within_bf16_ulps(_np(y), ref.cpu().numpy())
+            assert_within_bf16_ulps(_np(n), nref.cpu().numpy())
+        if off_y:  # nothing outside the view is written
+            assert (yb[:, :off_y] == 7).all() and (yb[:, off_y + D:] == 7).all()
+
+
+def test_softmax_of_infinite_and_masked_rows():
+    """Masked entries (-inf, the type's lowest value) get probability 0, a row
+    of them and a row with +inf or NaN is NaN, at every plan."""
+    from nkilab import ops
+
+    for D in (5, 1000, 5000, 20001, 70003):
+        x = torch.randn(5, D, device="cuda")
+        x[0, ::2] = -float("inf")
+        x[1, 1:] = torch.finfo(torch.float32).min
+        x[2] = -float("inf")
+        x[3, D // 2] = float("inf")
+        x[4, D - 1] = float("nan")
+        y = ops.softmax(x)
+        assert (y[0, ::2] == 0).all() and abs(y[0].double().sum().item() - 1) < 1e-5
+        assert y[1, 0] == 1 and (y[1, 1:] == 0).all()
+        assert torch.isnan(y[2]).all() and torch.isnan(y[3, D // 2]) and torch.isnan(y[4]).all()
