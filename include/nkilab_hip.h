@@ -73,10 +73,11 @@ const char* nkl_last_error_string(void);
  *      NULL for none.
  * Products accumulate in fp32; C is rounded once (round-to-nearest-even) to
  * dtype_out.  dtype_in in {F32, BF16, F16}; dtype_out in {F32, dtype_in}.
- * BF16 and F16 operands take the LDS-DMA kernel when A and B are 16-byte
- * aligned, K, lda, ldb (and N when b_trans == 0) are multiples of 8 and the
- * operands are under 2 GiB; other shapes, and variant NKL_GEMM_NAIVE, take a
- * one-tile-per-wavefront kernel (the same fp32 accumulation).
+ * The LDS-DMA kernel takes operands of 16-byte chunks: A and B 16-byte
+ * aligned, K, lda, ldb (and N when b_trans == 0) multiples of 8 (F32: 4), and
+ * the operands under 2 GiB; others are staged through registers.  Variant
+ * NKL_GEMM_NAIVE takes a one-tile-per-wavefront kernel (the same fp32
+ * accumulation).
  * The work is enqueued on `stream` as one kernel launch, or as two over
  * column ranges when the large tiles would leave a partial last round of
  * workgroups; nothing is allocated, and the call can be captured in a graph.
@@ -86,6 +87,24 @@ int nkl_gemm(const void* A, const void* B, void* C, const void* R,
              int b_trans, int batch, long strideA, long strideB, long strideC,
              long strideR, int dtype_in, int dtype_out, int variant,
              void* stream);
+
+/*
+ * One product of nkl_gemm (batch 1, NKL_GEMM_BLOCKED) with a workspace of
+ * nkl_gemm_workspace_bytes(...) bytes (16-byte aligned, no initialisation
+ * needed), which some shapes use: products of few tiles split a long K over
+ * workgroups (fp32 partial sums, added in a fixed order by a second launch),
+ * and large unaligned 16-bit products first copy their operands into aligned
+ * rows.  Where the size is 0 the call is nkl_gemm's and a null workspace will
+ * do; a workspace that is too small gets NKL_EWORKSPACE and nothing launched.
+ * The size depends on what it is given, the alignment of A and B included.
+ */
+size_t nkl_gemm_workspace_bytes(const void* A, const void* B, int M, int N,
+                                int K, long lda, long ldb, int b_trans,
+                                int dtype_in, int dtype_out);
+int nkl_gemm_ws(const void* A, const void* B, void* C, const void* R,
+                void* workspace, size_t workspace_bytes, int M, int N, int K,
+                long lda, long ldb, long ldc, long ldr, int b_trans,
+                int dtype_in, int dtype_out, void* stream);
 
 /*
  * C = silu(A . Wg^T) * (A . Wu^T): the decoder's gate and up projections and

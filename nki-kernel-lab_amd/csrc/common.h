@@ -306,6 +306,14 @@ __device__ __forceinline__ shortx4 ds_read_tr16_b64_async(const void* lds_ptr) {
   asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(r) : "v"(a));
   return r;
 }
+// The compiler's own form of the read, for kernels that fill their LDS with
+// ordinary stores.
+__device__ __forceinline__ shortx4 ds_read_tr16_b64_tracked(const void* lds_ptr) {
+  typedef short s4 __attribute__((vector_size(8)));
+  typedef __attribute__((address_space(3))) s4* lp;
+  return __builtin_bit_cast(shortx4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(size_t)(
+      const __attribute__((address_space(3))) void*)lds_ptr));
+}
 // ds_read_b128 in the same untracked form (so that the compiler's lgkmcnt
 // waits for its own reads do not count across untracked ones).
 __device__ __forceinline__ bf16x8 ds_read_b128_async(const void* lds_ptr) {

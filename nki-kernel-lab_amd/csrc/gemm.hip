@@ -1,23 +1,15 @@
 // GEMM: C = A . op(B) (+ R) on 32x32 MFMA tiles with fp32 accumulation.
 //
-// bf16 operands take the LDS-DMA kernel further down (gemm_dma_kernel: the
-// hot path, tiles from 64x64 to 256x256).
+// gemm_dma_kernel, the hot path: operands of 16-byte chunks (bf16, fp16 and
+// fp32) staged by the buffer unit, tiles from 32x32 to 256x256.
+// gemm_reg_kernel: any alignment, staged through registers.
+// gemm_pack_kernel, gemm_reduce_kernel: with a workspace (nkl_gemm_ws), large
+// unaligned 16-bit products copy their operands into aligned rows for the
+// first kernel, and few-tile products with a long K split it over workgroups.
 //
-// Register-staged blocked kernel (fp32 operands, and bf16 operands the DMA
-// kernel's buffer offsets cannot address): a 256-thread workgroup owns a
-// BM x BN tile of C; its four wavefronts are laid out 2 x 2 and each owns a
-// (BM/2) x (BN/2) sub-tile of 32x32 MFMA accumulators.  Per K step of BK
-// elements (64 bytes of each operand row) the workgroup stages an A tile
-// [BM][BK] and a B tile [BN][BK] in LDS, both K-contiguous so that every MFMA
-// operand fragment is one 16-byte LDS read.  B given as [K, N] (the
-// reference's `rhs`) is transposed while it is written to LDS; B given as
-// [N, K] (nn.Linear.weight) is copied as is.  LDS is double-buffered and the
-// next K step's global loads are in flight while the current one computes.
-//
-// Naive kernel (variant "naive", and the fallback for shapes the blocked
-// kernel's 16-byte loads cannot address): each wavefront computes one 32x32
-// tile of C reading its operands straight from global memory at every K step
-// -- no on-chip reuse, like the reference's matmul_naive.
+// Naive kernel (variant "naive"): each wavefront computes one 32x32 tile of C
+// reading its operands straight from global memory at every K step -- no
+// on-chip reuse, like the reference's matmul_naive.
 #include <atomic>
 #include <cstdlib>
 #include <cstring>
@@ -43,10 +35,10 @@ struct GemmArgs {
   long lda, ldb, ldc, ldr;
   long sA, sB, sC, sR;
   int epi;  // Epi (the LDS-DMA kernel; the other kernels store elements)
+  int Nc;   // columns stored: N, or fewer when packed operands pad N
+  int Kall; // 0, or the whole K of a product split over the batch index: entry z takes K columns from z K
+  int padded;  // rows along K hold zeros up to a multiple of 16 bytes past K
 };
-
-template <typename T>
-struct GemmBK { static constexpr int value = 64 / sizeof(T); };
 
 // Workgroup tile index -> (tile_m, tile_n).  Consecutive workgroup ids are
 // dispatched round-robin over the 8 XCDs; the remap gives each XCD a
@@ -64,138 +56,6 @@ __device__ __forceinline__ void tile_coords(int bid, int tiles_m, int tiles_n, i
   const int in_group = id - group * group_size;
   tm = first_m + in_group % gm;
   tn = in_group / gm;
-}
-
-template <typename T, typename TO, int BM, int BN, bool BT>
-__global__ __launch_bounds__(256) void gemm_blocked_kernel(GemmArgs p) {
-  using MF = Mfma32<T>;
-  constexpr int E = VecE<T>::value;           // elements per 16-byte chunk
-  constexpr int BK = GemmBK<T>::value;        // K elements per stage (64 bytes)
-  constexpr int PAD = E;                      // 16 bytes of row padding
-  constexpr int LDK = BK + PAD;               // LDS row stride (elements)
-  constexpr int CPR = BK / E;                 // 16-byte chunks per LDS row (4)
-  constexpr int WM = BM / 2, WN = BN / 2;     // wave sub-tile
-  constexpr int TM = WM / 32, TN = WN / 32;   // 32x32 MFMA tiles per wave
-  constexpr int A_CH = BM * CPR / 256;        // A chunks per thread
-  constexpr int B_CH = BN * CPR / 256;        // B chunks per thread
-  static_assert(A_CH >= 1 && B_CH >= 1, "tile too small for 256 threads");
-
-  __shared__ T As[2][BM * LDK];
-  __shared__ T Bs[2][BN * LDK];
-
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int wm = wid >> 1, wn = wid & 1;
-  const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
-  int tm, tn;
-  tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
-  const int bz = blockIdx.z;
-  const T* A = static_cast<const T*>(p.A) + (long)bz * p.sA;
-  const T* B = static_cast<const T*>(p.B) + (long)bz * p.sB;
-  TO* C = static_cast<TO*>(p.C) + (long)bz * p.sC;
-  const TO* R = p.R ? static_cast<const TO*>(p.R) + (long)bz * p.sR : nullptr;
-
-  uint4 ra[A_CH], rb[B_CH];
-  auto gload = [&](int k0) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < A_CH; ++i) {
-      const int c = tid + 256 * i, row = c / CPR, kc = (c % CPR) * E;
-      const int gm = m0 + row, gk = k0 + kc;
-      ra[i] = ld16_or_zero(A, (long)gm * p.lda + gk, gm < p.M && gk < p.K);
-    }
-    if constexpr (BT) {
-#pragma unroll
-      for (int i = 0; i < B_CH; ++i) {
-        const int c = tid + 256 * i, row = c / CPR, kc = (c % CPR) * E;
-        const int gn = n0 + row, gk = k0 + kc;
-        rb[i] = ld16_or_zero(B, (long)gn * p.ldb + gk, gn < p.N && gk < p.K);
-      }
-    } else {
-      constexpr int NCH = BN / E;  // 16-byte chunks per B row of the tile
-#pragma unroll
-      for (int i = 0; i < B_CH; ++i) {
-        const int c = tid + 256 * i, kr = c / NCH, nc = (c % NCH) * E;
-        const int gk = k0 + kr, gn = n0 + nc;
-        rb[i] = ld16_or_zero(B, (long)gk * p.ldb + gn, gk < p.K && gn < p.N);
-      }
-    }
-  };
-
-  auto lstore = [&](int buf) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < A_CH; ++i) {
-      const int c = tid + 256 * i, row = c / CPR, kc = (c % CPR) * E;
-      *reinterpret_cast<uint4*>(&As[buf][row * LDK + kc]) = ra[i];
-    }
-    if constexpr (BT) {
-#pragma unroll
-      for (int i = 0; i < B_CH; ++i) {
-        const int c = tid + 256 * i, row = c / CPR, kc = (c % CPR) * E;
-        *reinterpret_cast<uint4*>(&Bs[buf][row * LDK + kc]) = rb[i];
-      }
-    } else {
-      constexpr int NCH = BN / E;
-#pragma unroll
-      for (int i = 0; i < B_CH; ++i) {
-        const int c = tid + 256 * i, kr = c / NCH, nc = (c % NCH) * E;
-        const T* v = reinterpret_cast<const T*>(&rb[i]);
-#pragma unroll
-        for (int e = 0; e < E; ++e) Bs[buf][(nc + e) * LDK + kr] = v[e];
-      }
-    }
-  };
-
-  floatx16 acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-
-  const int nk = (p.K + BK - 1) / BK;
-  gload(0);
-  lstore(0);
-  __syncthreads();
-  const int lr = lane & 31, lg = lane >> 5;
-  for (int kt = 0; kt < nk; ++kt) {
-    const int buf = kt & 1;
-    if (kt + 1 < nk) gload((kt + 1) * BK);
-#pragma unroll
-    for (int ks = 0; ks < BK / MF::MK; ++ks) {
-      const int kk = ks * MF::MK + lg * MF::KPER;
-      typename MF::frag af[TM], bfr[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) af[i] = load_frag(&As[buf][(wm * WM + i * 32 + lr) * LDK + kk]);
-#pragma unroll
-      for (int j = 0; j < TN; ++j) bfr[j] = load_frag(&Bs[buf][(wn * WN + j * 32 + lr) * LDK + kk]);
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = MF::mma(af[i], bfr[j], acc[i][j]);
-    }
-    if (kt + 1 < nk) lstore(buf ^ 1);
-    __syncthreads();
-  }
-
-  // Epilogue: accumulator element e of tile (i, j) is C[row][col] with
-  // row = 8 * (e / 4) + 4 * (lane / 32) + e % 4, col = lane % 32.
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int col = n0 + wn * WN + j * 32 + lr;
-      if (col >= p.N) continue;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int row = m0 + wm * WM + i * 32 + 8 * (e / 4) + 4 * lg + (e % 4);
-        if (row < p.M) {
-          float vv = acc[i][j][e];
-          if (R) vv += to_f32(R[(long)row * p.ldr + col]);
-          C[(long)row * p.ldc + col] = from_f32<TO>(vv);
-        }
-      }
-    }
 }
 
 // One wavefront per 32x32 tile of C, four per workgroup; operands are read
@@ -256,9 +116,14 @@ __global__ __launch_bounds__(256) void gemm_naive_kernel(GemmArgs p) {
   }
 }
 
-// ------------------------------------------------ bf16 GEMM, LDS-DMA staged --
+// 16 bytes at the alignment of their element only.
+typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+typedef u32x4_t u32x4_al2 __attribute__((aligned(2)));
+typedef u32x4_t u32x4_al4 __attribute__((aligned(4)));
+
+// ----------------------------------------------------- GEMM, LDS-DMA staged --
 //
-// The bf16 path.  Operand tiles are copied global -> LDS by the buffer unit
+// Operand tiles are copied global -> LDS by the buffer unit
 // (buffer_load ... lds, lane l's 16 bytes at the instruction's LDS base + 16 l)
 // into a ring of NS stages, NS - 1 K-steps ahead of use, so that even a small
 // GEMM (1024^3, 256 workgroups of 64x64) keeps enough loads in flight to cover
@@ -270,6 +135,15 @@ __global__ __launch_bounds__(256) void gemm_naive_kernel(GemmArgs p) {
 // read with ds_read_b64_tr_b16) free of bank conflicts.  One barrier per
 // K-step; WGM x WGN wavefronts of 32x32x16 MFMA tiles.
 //
+// fp32 runs the same pipeline over the same bytes: a 16-byte fragment is 4
+// elements of K for four 32x32x2 MFMAs (lane group lg supplies k = 4 lg + j to
+// MFMA j, the same order in A and B), and B as [K, N] stays row-major in LDS
+// and is read 4 bytes at a time.  Its MFMAs take 64 cycles each, so the loop is
+// bound by them: 2048^3 222 -> 131 us (B^T; [K, N] 141) against 111 us of MFMA
+// time, 128x128 tiles in two K groups; a 64 x 64 wavefront tile without the
+// copies, or without the fragment reads, takes 125 and 128.  The register-staged
+// kernel takes 150 to 160 there.
+//
 // 2 x 2 wavefronts (256 threads, one per SIMD) for tiles up to 128 x 128;
 // 2 x 4 (512 threads, two per SIMD) for 256-row tiles.  A 128 x 128 tile
 // stages 32 KB per K-step for 2 MFLOP, ~64 B/clk per CU at the MFMA rate --
@@ -279,7 +153,9 @@ __global__ __launch_bounds__(256) void gemm_naive_kernel(GemmArgs p) {
 
 namespace {
 
-constexpr int G_BK = 64;  // K elements per stage
+// K elements per stage (128-byte rows).
+template <typename T>
+constexpr int kBK = 128 / (int)sizeof(T);
 
 __device__ __forceinline__ int g_swz(int r) { return (((r >> 1) & 1) << 2) | (((r >> 2) & 1) << 1) | ((r >> 3) & 1); }
 // Byte offset of 16-byte chunk c of row r in a tile of 128-byte rows.
@@ -299,14 +175,16 @@ constexpr unsigned kOOB = 0x80000000u;  // a buffer offset past every range: the
 
 template <typename TI, typename TO, int BM, int BN, bool BT, int NS, int WGM = 2, int WGN = 2, int KG = 1>
 __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_dma_kernel(GemmArgs p) {
-  // TI: the 16-bit operand format (bf16 or fp16); operands move as raw 16-bit
-  // values, the format only picks the MFMA.
+  // TI: the operand format (bf16, fp16 or fp32); operands move as raw 16-byte
+  // chunks, the format only picks the MFMA.
   // KG > 1: KG groups of WGM x WGN wavefronts share the tile; group g takes
   // K-steps g, g + KG, ... through its own part of each stage, and the groups'
   // accumulators are added in group order at the end.  Each SIMD then runs KG
   // wavefronts whose copy and fragment-read latencies hide each other's.
   constexpr bool H = std::is_same<TI, f16>::value;
-  static_assert(H || std::is_same<TI, bf16>::value, "16-bit operands");
+  constexpr bool F32 = std::is_same<TI, float>::value;
+  static_assert(H || F32 || std::is_same<TI, bf16>::value, "operand format");
+  constexpr int E = VecE<TI>::value, SZ = sizeof(TI), BK = kBK<TI>;
   constexpr int NW = WGM * WGN;
   constexpr int A_BYTES = BM * 128;
   constexpr int B_BYTES = BN * 128;  // BN rows of 128 B (B^T) or BN / 64 sub-tiles of 64 x 128 B
@@ -331,11 +209,12 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_dma_kernel(GemmArgs 
   tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
   const int bz = blockIdx.z;
-  const bf16* A = static_cast<const bf16*>(p.A) + (long)bz * p.sA;
-  const bf16* B = static_cast<const bf16*>(p.B) + (long)bz * p.sB;
+  const TI* A = static_cast<const TI*>(p.A) + (long)bz * p.sA;
+  const TI* B = static_cast<const TI*>(p.B) + (long)bz * p.sB;
   TO* C = static_cast<TO*>(p.C) + (long)bz * p.sC;
   const TO* R = p.R ? static_cast<const TO*>(p.R) + (long)bz * p.sR : nullptr;
-  const int K = p.K;
+  const int K = p.Kall ? min(p.K, p.Kall - bz * p.K) : p.K;
+  const int Kr = (K + E - 1) / E * E;  // readable (K unless the rows are padded)
 
   // ---- DMA: instruction q of a 128-byte-row tile covers rows 8 q .. 8 q + 7;
   // lane l fills row 8 q + l / 8, physical chunk l % 8.
@@ -343,15 +222,15 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_dma_kernel(GemmArgs 
   // A rows m (B^T rows n): byte offset of the lane's chunk at K-step 0, or kOOB.
   const int rows_a = min(BM, p.M - m0);
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(A + (long)m0 * p.lda), (short)0, (int)min(2L * ((rows_a - 1) * p.lda + K), 0x7fffffffL), 0x00020000);
+      (void*)(A + (long)m0 * p.lda), (short)0, (int)min((long)SZ * ((rows_a - 1) * p.lda + Kr), 0x7fffffffL), 0x00020000);
   unsigned aoff[A_PW];
   int akc[A_PW];
 #pragma unroll
   for (int u = 0; u < A_PW; ++u) {
     const int row = 8 * (wid * A_PW + u) + dr;
     const int lc = dpc ^ g_swz(row);
-    akc[u] = 8 * lc;
-    aoff[u] = row < rows_a ? (unsigned)(2 * ((long)row * p.lda + 8 * lc)) : kOOB;
+    akc[u] = E * lc;
+    aoff[u] = row < rows_a ? (unsigned)(SZ * ((long)row * p.lda + E * lc)) : kOOB;
   }
   __amdgpu_buffer_rsrc_t rb;
   unsigned boff[B_PW];
@@ -359,46 +238,47 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_dma_kernel(GemmArgs 
   if constexpr (BT) {
     const int rows_b = min(BN, p.N - n0);
     rb = __builtin_amdgcn_make_buffer_rsrc((void*)(B + (long)n0 * p.ldb), (short)0,
-                                           (int)min(2L * ((rows_b - 1) * p.ldb + K), 0x7fffffffL), 0x00020000);
+                                           (int)min((long)SZ * ((rows_b - 1) * p.ldb + Kr), 0x7fffffffL), 0x00020000);
 #pragma unroll
     for (int u = 0; u < B_PW; ++u) {
       const int row = 8 * (wid * B_PW + u) + dr;
       const int lc = dpc ^ g_swz(row);
-      bkc[u] = 8 * lc;
+      bkc[u] = E * lc;
       brow[u] = 0;
-      boff[u] = row < rows_b ? (unsigned)(2 * ((long)row * p.ldb + 8 * lc)) : kOOB;
+      boff[u] = row < rows_b ? (unsigned)(SZ * ((long)row * p.ldb + E * lc)) : kOOB;
     }
   } else {
-    // [K, N]: instruction q -> sub-tile q / 8 (64 columns), k rows 8 (q % 8) + dr.
+    // [K, N]: 16-bit instruction q -> sub-tile q / 8 (64 columns), k rows
+    // 8 (q % 8) + dr; fp32: 1024 bytes of the row-major [BK][BN] tile.
     const int cols_b = min(BN, p.N - n0);
     rb = __builtin_amdgcn_make_buffer_rsrc((void*)(B + n0), (short)0,
-                                           (int)min(2L * ((long)(K - 1) * p.ldb + cols_b), 0x7fffffffL), 0x00020000);
+                                           (int)min((long)SZ * ((long)(K - 1) * p.ldb + cols_b), 0x7fffffffL), 0x00020000);
 #pragma unroll
     for (int u = 0; u < B_PW; ++u) {
       const int q = wid * B_PW + u;
-      const int sub = q / 8, row = 8 * (q % 8) + dr;
-      const int col = 64 * sub + 8 * (dpc ^ g_swz(row));
+      const int sub = q / 8, row = F32 ? (256 * q + 4 * lane) / BN : 8 * (q % 8) + dr;
+      const int col = F32 ? (256 * q + 4 * lane) % BN : 64 * sub + 8 * (dpc ^ g_swz(row));
       brow[u] = row;
       bkc[u] = 0;
-      boff[u] = col < cols_b ? (unsigned)(2 * ((long)row * p.ldb + col)) : kOOB;
+      boff[u] = col < cols_b ? (unsigned)(SZ * ((long)row * p.ldb + col)) : kOOB;
     }
   }
   // Copy instruction u (A for u < A_PW, then B) of K-step s into stage st
   // (K-steps past K copy zeros).
   auto dma1 = [&](int s, int st, int u) __attribute__((always_inline)) {
-    const int k0 = (KG * s + kg) * G_BK;
+    const int k0 = (KG * s + kg) * BK;
     unsigned char* sb = lds + st * SSET + kg * STAGE;
     if (u < A_PW) {
-      const unsigned off = (aoff[u] != kOOB && k0 + akc[u] < K) ? aoff[u] + 2u * k0 : kOOB;
+      const unsigned off = (aoff[u] != kOOB && k0 + akc[u] < K) ? aoff[u] + (unsigned)SZ * k0 : kOOB;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (__attribute__((address_space(3))) void*)(sb + (wid * A_PW + u) * 1024),
                                                16, (int)off, 0, 0, 0);
     } else {
       const int w = u - A_PW;
       unsigned off;
       if constexpr (BT)
-        off = (boff[w] != kOOB && k0 + bkc[w] < K) ? boff[w] + 2u * k0 : kOOB;
+        off = (boff[w] != kOOB && k0 + bkc[w] < K) ? boff[w] + (unsigned)SZ * k0 : kOOB;
       else
-        off = (boff[w] != kOOB && k0 + brow[w] < K) ? boff[w] + (unsigned)(2L * k0 * p.ldb) : kOOB;
+        off = (boff[w] != kOOB && k0 + brow[w] < K) ? boff[w] + (unsigned)((long)SZ * k0 * p.ldb) : kOOB;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           rb, (__attribute__((address_space(3))) void*)(sb + A_BYTES + (wid * B_PW + w) * 1024), 16, (int)off, 0, 0,
           0);
@@ -419,7 +299,9 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_dma_kernel(GemmArgs 
     afo[ks] = g_pos(wm * WM + lr, 2 * ks + lg);
     bto[ks] = A_BYTES + g_pos(wn * WN + lr, 2 * ks + lg);
   }
-  if constexpr (!BT) {
+  // fp32 B as [K, N]: element e of sub-step ks is row 8 ks + 4 lg + e.
+  const int bf32 = A_BYTES + 16 * lg * BN + 4 * (wn * WN + lr);
+  if constexpr (!BT && !F32) {
     const int i16 = lane & 15, g2 = (lane >> 4) & 1;
 #pragma unroll
     for (int j = 0; j < TN; ++j)
@@ -444,19 +326,25 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_dma_kernel(GemmArgs 
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
-  // Fragments of sub-step ks (16 K) of the stage at sb.
+  // Fragments of sub-step ks (32 bytes of K) of the stage at sb.
   auto frags = [&](const unsigned char* sb, int ks, bf16x8 (&af)[TM], bf16x8 (&bfr)[TN])
                    __attribute__((always_inline)) {
-    // With B as [K, N] every fragment read is untracked (see
+    // With 16-bit B as [K, N] every fragment read is untracked (see
     // ds_read_tr16_b64_async); lds_wait_tie on the B fragments orders them all.
 #pragma unroll
     for (int i = 0; i < TM; ++i)
-      af[i] = BT ? *reinterpret_cast<const bf16x8*>(sb + afo[ks] + 4096 * i)
-                 : ds_read_b128_async(sb + afo[ks] + 4096 * i);
+      af[i] = BT || F32 ? *reinterpret_cast<const bf16x8*>(sb + afo[ks] + 4096 * i)
+                        : ds_read_b128_async(sb + afo[ks] + 4096 * i);
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       if constexpr (BT) {
         bfr[j] = *reinterpret_cast<const bf16x8*>(sb + bto[ks] + 4096 * j);
+      } else if constexpr (F32) {
+        floatx4 t;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          t[e] = *reinterpret_cast<const float*>(sb + bf32 + 4 * ((8 * ks + e) * BN + 32 * j));
+        bfr[j] = __builtin_bit_cast(bf16x8, t);
       } else {
         // (untracked reads: tied by lds_wait_tie before the MFMAs use them)
         const shortx4 x = ds_read_tr16_b64_async(sb + bfo[j][ks][0]);
@@ -465,11 +353,17 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_dma_kernel(GemmArgs 
       }
     }
   };
-  auto mmas = [&](const bf16x8 (&af)[TM], const bf16x8 (&bfr)[TN]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] = mma32_16b<H>(af[i], bfr[j], acc[i][j]);
+  // MFMA k of a sub-step: one per tile in 16 bits; four per tile in fp32, the
+  // tiles in turn so that consecutive ones are independent.
+  constexpr int NMMA = TM * TN * (F32 ? 4 : 1);
+  auto mma1 = [&](const bf16x8 (&af)[TM], const bf16x8 (&bfr)[TN], int k) __attribute__((always_inline)) {
+    const int t = k % (TM * TN), i = t / TN, j = t % TN;
+    if constexpr (F32)
+      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__builtin_bit_cast(floatx4, af[i])[k / (TM * TN)],
+                                                       __builtin_bit_cast(floatx4, bfr[j])[k / (TM * TN)], acc[i][j],
+                                                       0, 0, 0);
+    else
+      acc[i][j] = mma32_16b<H>(af[i], bfr[j], acc[i][j]);
   };
   // Every wavefront's copies of a stage have landed once each waited for its
   // own (vmcnt) and all passed the barrier.  A bare s_barrier, not
@@ -495,7 +389,6 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_dma_kernel(GemmArgs 
   // right after the barrier that frees their stage, the rest with the first
   // sub-step of step s+1, and must land by the end of step s+1.
   constexpr bool SPREAD = NS >= 3;
-  constexpr int NMMA = TM * TN;
   constexpr int Q = (LPT + 3) / 4;  // copies per sub-step when spread
   constexpr int H2 = (LPT + 1) / 2;  // two stages: copies issued right after the barrier
   // Copies issued after K-step s+1's last one when step s waits for it: with
@@ -504,20 +397,25 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_dma_kernel(GemmArgs 
   // takes every copy in flight).
   constexpr int WAITN = SPREAD ? (NS - 3) * LPT + 3 * Q : (NS - 2) * LPT;
   static_assert(!SPREAD || 3 * Q <= LPT, "the last sub-step's share of the copies is not negative");
-  // The MFMAs of one sub-step with copies u0 .. u1-1 of K-step sd between them.
-  auto mma_copy = [&](const bf16x8 (&af)[TM], const bf16x8 (&bfr)[TN], int sd, int u0, int u1)
+  bf16x8 fa[2][TM], fb[2][TN];
+  // The fragment reads of sub-step nks of the stage at nsb, then the MFMAs of
+  // the current one with copies u0 .. u1-1 of K-step sd between them.
+  auto sub_step = [&](int cur, const unsigned char* nsb, int nks, int sd, int u0, int u1)
                       __attribute__((always_inline)) {
-    const int per = (u1 - u0 + NMMA - 1) / NMMA;
+    frags(nsb, nks, fa[cur ^ 1], fb[cur ^ 1]);
+    __builtin_amdgcn_sched_barrier(0);  // the reads stay ahead of the MFMAs
+    const int nc = u1 - u0, per = (nc + NMMA - 1) / NMMA;
 #pragma unroll
     for (int k = 0; k < NMMA; ++k) {
-      acc[k / TN][k % TN] = mma32_16b<H>(af[k / TN], bfr[k % TN], acc[k / TN][k % TN]);
+      mma1(fa[cur], fb[cur], k);
 #pragma unroll
       for (int u = u0 + k * per; u < u0 + (k + 1) * per && u < u1; ++u) dma1(sd, sd % NS, u);
-      __builtin_amdgcn_sched_barrier(0);
+      if (nc > 0) __builtin_amdgcn_sched_barrier(0);
     }
+    __builtin_amdgcn_sched_barrier(0);
   };
   // Steps of the loop: KG K-steps each (a group's K-steps past K copy zeros).
-  const int nk = ((K + G_BK - 1) / G_BK + KG - 1) / KG;
+  const int nk = ((K + BK - 1) / BK + KG - 1) / KG;
   const unsigned char* const glds = lds + kg * STAGE;  // this group's part of stage 0
   // K-steps 0 .. NS-2, and with two stages the first H2 copies of K-step
   // NS-1 (step 0 issues the rest, as every step does for the K-step after it).
@@ -529,42 +427,35 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_dma_kernel(GemmArgs 
   }
   g_wait_vm<(NS - 2) * LPT + (SPREAD ? 0 : H2)>();  // K-step 0 has landed
   barrier();
-  bf16x8 fa[2][TM], fb[2][TN];
   frags(glds, 0, fa[0], fb[0]);
 #pragma unroll 1
   for (int s = 0; s < nk; ++s) {
     const unsigned char* sb = glds + (s % NS) * SSET;
 #pragma unroll
     for (int ks = 0; ks < 3; ++ks) {
-      if constexpr (!BT) {  // B^T fragments of sub-step ks have landed (read one sub-step ago)
+      if constexpr (!BT && !F32) {  // B^T fragments of sub-step ks have landed (read one sub-step ago)
 #pragma unroll
         for (int j = 0; j < TN; ++j) lds_wait_tie(fb[ks & 1][j]);
       }
-      frags(sb, ks + 1, fa[(ks + 1) & 1], fb[(ks + 1) & 1]);
-      __builtin_amdgcn_sched_barrier(0);  // the reads stay ahead of the MFMAs
       if constexpr (SPREAD)
-        mma_copy(fa[ks & 1], fb[ks & 1], s + NS - 1, ks * Q, min((ks + 1) * Q, LPT));
-      else if (ks == 0)
-        mma_copy(fa[0], fb[0], s + NS - 1, H2, LPT);  // the rest of K-step s+1
+        sub_step(ks & 1, sb, ks + 1, s + NS - 1, ks * Q, min((ks + 1) * Q, LPT));
       else
-        mmas(fa[ks & 1], fb[ks & 1]);
-      __builtin_amdgcn_sched_barrier(0);
+        sub_step(ks & 1, sb, ks + 1, s + NS - 1, H2, ks == 0 ? LPT : H2);  // the rest of K-step s+1
     }
     g_wait_vm<WAITN>();  // K-step s+1 has landed
     g_wait_lgkm0();      // this wavefront's reads of K-step s are done
-    if constexpr (!BT) {
+    if constexpr (!BT && !F32) {
 #pragma unroll
       for (int j = 0; j < TN; ++j) lds_wait_tie(fb[1][j]);
     }
     barrier();                    // ... for every wavefront
-    // The next K-step's first fragment reads come first in program order
-    // (the copies may alias them), then the last sub-step's MFMAs, whose
-    // fragments are already in registers.
-    frags(glds + ((s + 1) % NS) * SSET, 0, fa[0], fb[0]);
+    // The last sub-step's MFMAs (fragments in registers), with the next
+    // K-step's first fragment reads.
+    const unsigned char* nsb = glds + ((s + 1) % NS) * SSET;
     if constexpr (SPREAD)
-      mma_copy(fa[1], fb[1], s + NS - 1, 3 * Q, LPT);
+      sub_step(1, nsb, 0, s + NS - 1, 3 * Q, LPT);
     else
-      mma_copy(fa[1], fb[1], s + NS, 0, H2);  // into K-step s's stage
+      sub_step(1, nsb, 0, s + NS, 0, H2);  // into K-step s's stage
   }
   __builtin_amdgcn_s_waitcnt(0);  // the copies of K-steps past K have landed
 
@@ -572,7 +463,8 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_dma_kernel(GemmArgs 
   constexpr int OE = 16 / sizeof(TO);  // output elements per 16-byte store
   constexpr int WC_MAX = WN;           // staged columns per wavefront (SwiGLU: WN / 2)
   constexpr int PITCH = WC_MAX + 4;    // staged row pitch, floats
-  constexpr int RP = NW * WM * PITCH * 4 <= NS * SSET ? WM : 32;  // rows per pass
+  constexpr int RED = (KG - 1) * NW * TM * TN * 4096;  // the K groups' partial sums, bytes
+  constexpr int RP = NW * WM * PITCH * 4 + RED <= NS * SSET ? WM : 32;  // rows per pass
   constexpr int TP = RP / 32;                                      // tiles per pass
   static_assert(NW * RP * PITCH * 4 <= NS * SSET, "the staged rows fit the stages");
   if constexpr (KG > 1) {
@@ -625,7 +517,7 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_dma_kernel(GemmArgs 
     const int wc = sw ? WN / 2 : WN;
     // Rows of the block go to rows m0 + wm WM ..; columns to c0 ...
     const int c0 = sw ? (n0 + wn * WN) / 2 : n0 + wn * WN;
-    const int ncols = sw ? p.N / 2 : p.N;
+    const int ncols = sw ? p.N / 2 : p.Nc;
     const int cpr = wc / OE;  // 16-byte chunks per staged row
 #pragma unroll
     for (int ip = 0; ip < TM / TP; ++ip) {
@@ -682,7 +574,308 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_dma_kernel(GemmArgs 
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       const int col = n0 + wn * WN + j * 32 + lr;
-      if (col >= p.N) continue;
+      if (col >= p.Nc) continue;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int row = m0 + wm * WM + i * 32 + 8 * (e / 4) + 4 * lg + (e % 4);
+        if (row < p.M) {
+          float vv = acc[i][j][e];
+          if (R) vv += to_f32(R[(long)row * p.ldr + col]);
+          C[(long)row * p.ldc + col] = from_f32<TO>(vv);
+        }
+      }
+    }
+}
+
+// ----------------------------------------- register-staged GEMM, unaligned --
+//
+// Operands the buffer unit's copies cannot take (bases, K or leading dimensions
+// off 16 bytes, N off 16 bytes with B as [K, N], 2 GiB or more).  Operand tiles
+// go global -> registers -> LDS, PF K-steps ahead, with 16-byte loads at the
+// element's own alignment (gfx950 takes them at any address); the last K-steps,
+// and those with rows of a [K, N] B whose loads would end past it, are loaded
+// with a check per chunk and the chunk that straddles K or N element by
+// element.  Rows and columns past M and N repeat the last one (their products
+// are never stored); K is padded with zeros in both operands.
+//
+// Bound by the K-step's chain (LDS reads, stores and a barrier, ~0.4 us with one
+// workgroup on a CU) on small grids and by LDS traffic on large ones.  One
+// wavefront per tile reading elements from global memory, as before, took 74 us
+// at 1000 x 777 x 1301 bf16; this takes 14.5 (rows at an odd address cost ~20%:
+// 12.2 at 1000 x 784 x 1304).
+//
+// LDS tiles are the LDS-DMA kernel's: 128-byte rows (32 fp32 or 64 16-bit
+// elements of K; B as [K, N] in 16 bits in sub-tiles of 64 columns), 16-byte
+// chunks swizzled, and one b128 read per operand fragment: 8 elements of K for
+// one 16-bit MFMA, or 4 for four fp32 MFMAs (32x32x2; lane group lg supplies
+// k = 4 lg + j to MFMA j of the four, the same order in A and B).  fp32 B as
+// [K, N] stays row-major and is read 4 bytes at a time, 32 columns a row.
+//
+// KG groups of WGM x WGN wavefronts share the tile as in the LDS-DMA kernel:
+// group g takes K-steps g, g + KG, ... and the groups' accumulators are added
+// in group order at the end, so that a GEMM of few tiles still has its K range
+// spread over a CU's SIMDs.
+__device__ __forceinline__ u32x4_t ld16_unaligned(const float* p) { return *reinterpret_cast<const u32x4_al4*>(p); }
+template <typename T>
+__device__ __forceinline__ u32x4_t ld16_unaligned(const T* p) {
+  static_assert(sizeof(T) == 2, "16-bit elements");
+  return *reinterpret_cast<const u32x4_al2*>(p);
+}
+// The first n elements at p, zeros after them.
+template <typename T>
+__device__ __forceinline__ u32x4_t ld16_first(const T* p, int n) {
+  constexpr int E = VecE<T>::value;
+  if (n >= E) return ld16_unaligned(p);
+  u32x4_t r = {0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if (e < n) {
+      if constexpr (sizeof(T) == 4)
+        r[e] = __float_as_uint(p[e]);
+      else
+        r[e / 2] |= (uint32_t)__builtin_bit_cast(uint16_t, p[e]) << (16 * (e & 1));
+    }
+  return r;
+}
+
+template <typename TI, typename TO, int BM, int BN, bool BT, int WGM, int WGN, int KG, int PF>
+__global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_reg_kernel(GemmArgs p) {
+  constexpr bool F32 = sizeof(TI) == 4;
+  constexpr bool H = std::is_same<TI, f16>::value;
+  constexpr int E = VecE<TI>::value;  // elements per 16-byte chunk
+  constexpr int BK = 128 / sizeof(TI);
+  constexpr int NT = 64 * WGM * WGN;  // threads of a K group
+  constexpr int A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128, SSET = KG * STAGE;
+  constexpr int A_CH = BM * 8 / NT, B_CH = BN * 8 / NT;  // chunks per thread and K-step
+  constexpr int WM = BM / WGM, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
+  static_assert(A_CH * NT == BM * 8 && B_CH * NT == BN * 8, "chunks split over the group");
+  static_assert(F32 || BT || BN % 64 == 0, "16-bit [K, N] tiles are made of 64-column sub-tiles");
+  __shared__ __align__(16) unsigned char lds[2 * SSET];
+
+  const int tid = threadIdx.x % NT, lane = tid & 63;
+  const int wall = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kg = wall / (WGM * WGN), wid = wall % (WGM * WGN);
+  const int wm = wid / WGN, wn = wid % WGN;
+  const int lr = lane & 31, lg = lane >> 5;
+  const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
+  int tm, tn;
+  tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int bz = blockIdx.z;
+  const TI* A = static_cast<const TI*>(p.A) + (long)bz * p.sA;
+  const TI* B = static_cast<const TI*>(p.B) + (long)bz * p.sB;
+  TO* C = static_cast<TO*>(p.C) + (long)bz * p.sC;
+  const TO* R = p.R ? static_cast<const TO*>(p.R) + (long)bz * p.sR : nullptr;
+  const int K = p.Kall ? min(p.K, p.Kall - bz * p.K) : p.K, N = p.N;
+
+  // Chunk i of the thread: LDS byte, K offset within a K-step and address at
+  // K-step 0.
+  const TI* pa[A_CH];
+  const TI* pb[B_CH];
+  int la[A_CH], lb[B_CH], ka[A_CH], kb[B_CH], nb[B_CH];
+#pragma unroll
+  for (int i = 0; i < A_CH; ++i) {
+    const int c = tid + NT * i, row = c / 8, pc = c % 8;
+    la[i] = g_pos(row, pc);
+    ka[i] = pc * E;
+    pa[i] = A + (long)min(m0 + row, p.M - 1) * p.lda + ka[i];
+  }
+#pragma unroll
+  for (int i = 0; i < B_CH; ++i) {
+    const int c = tid + NT * i;
+    if constexpr (BT) {
+      const int row = c / 8, pc = c % 8;
+      lb[i] = A_BYTES + g_pos(row, pc);
+      kb[i] = pc * E;
+      nb[i] = E;
+      pb[i] = B + (long)min(n0 + row, N - 1) * p.ldb + kb[i];
+    } else {
+      constexpr int CPR = BN / E;  // chunks per K row
+      const int kr = c / CPR, nc = c % CPR;
+      const int n = min(n0 + nc * E, (N - 1) / E * E);  // columns past N repeat the last chunk
+      lb[i] = A_BYTES + (F32 ? kr * BN * 4 + nc * 16 : nc / 8 * 8192 + g_pos(kr, nc % 8));
+      kb[i] = kr;
+      nb[i] = N - n;  // columns the chunk may read
+      pb[i] = B + (long)kr * p.ldb + n;
+    }
+  }
+  const long b_step = BT ? BK : (long)BK * p.ldb;
+  // The leading K-steps whose loads all end within K and, with B as [K, N],
+  // before B's last element.
+  int kfast = K / BK;
+  if constexpr (!BT) {
+    const long end = (long)(K - 1) * p.ldb + N - min(n0 + BN, (N + E - 1) / E * E);  // last row a chunk fits in
+    kfast = end < 0 ? 0 : (int)min((long)kfast, (end / p.ldb + 1) / BK);
+  }
+
+  // Registers of K-steps in flight: K-step s in slot s % PF.
+  u32x4_t rra[PF][A_CH], rrb[PF][B_CH];
+  auto gload = [&](int s, u32x4_t (&ra)[A_CH], u32x4_t (&rb)[B_CH])
+                   __attribute__((always_inline)) {  // K-step s of this group, a leading one
+    const int ks = KG * s + kg;
+#pragma unroll
+    for (int i = 0; i < A_CH; ++i) ra[i] = ld16_unaligned(pa[i] + ks * BK);
+#pragma unroll
+    for (int i = 0; i < B_CH; ++i) rb[i] = ld16_unaligned(pb[i] + ks * b_step);
+  };
+  auto gload_checked = [&](int s, u32x4_t (&ra)[A_CH], u32x4_t (&rb)[B_CH]) __attribute__((always_inline)) {
+    const int ks = KG * s + kg, k0 = ks * BK;
+#pragma unroll
+    for (int i = 0; i < A_CH; ++i) ra[i] = ld16_first(pa[i] + k0, K - k0 - ka[i]);
+#pragma unroll
+    for (int i = 0; i < B_CH; ++i) {
+      if constexpr (BT)
+        rb[i] = ld16_first(pb[i] + k0, K - k0 - kb[i]);
+      else
+        rb[i] = ld16_first(pb[i] + ks * b_step, k0 + kb[i] < K ? nb[i] : 0);
+    }
+  };
+  auto lstore = [&](int st, const u32x4_t (&ra)[A_CH], const u32x4_t (&rb)[B_CH]) __attribute__((always_inline)) {
+    unsigned char* sb = lds + st * SSET + kg * STAGE;
+#pragma unroll
+    for (int i = 0; i < A_CH; ++i) *reinterpret_cast<u32x4_t*>(sb + la[i]) = ra[i];
+#pragma unroll
+    for (int i = 0; i < B_CH; ++i) *reinterpret_cast<u32x4_t*>(sb + lb[i]) = rb[i];
+  };
+  // The LDS stores and reads of every wavefront are done; the next K-step's
+  // global loads stay in flight (__syncthreads() would wait for them).
+  auto lds_barrier = [&]() __attribute__((always_inline)) {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    g_wait_lgkm0();
+    __builtin_amdgcn_s_barrier();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  };
+
+  floatx16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+
+  const int nk = ((K + BK - 1) / BK + KG - 1) / KG;
+  // Every fragment of the K-step in stage st is read in flight together, then
+  // `mid` runs behind the reads, then the MFMAs.
+  auto compute = [&](int st, auto mid) __attribute__((always_inline)) {
+    const unsigned char* sb = lds + st * SSET + kg * STAGE;
+    bf16x8 af[4][TM], bfr[4][TN];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+        af[ks][i] = *reinterpret_cast<const bf16x8*>(sb + g_pos(wm * WM + lr, 2 * ks + lg) + 4096 * i);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        if constexpr (BT) {
+          bfr[ks][j] = *reinterpret_cast<const bf16x8*>(sb + A_BYTES + g_pos(wn * WN + lr, 2 * ks + lg) + 4096 * j);
+        } else if constexpr (F32) {
+          const float* bp =
+              reinterpret_cast<const float*>(sb + A_BYTES) + (8 * ks + 4 * lg) * BN + wn * WN + 32 * j + lr;
+          bfr[ks][j] = __builtin_bit_cast(bf16x8, floatx4{bp[0], bp[BN], bp[2 * BN], bp[3 * BN]});
+        } else {
+          // Two transposed reads of 4 K rows: lane i of a 16-lane group
+          // reads row i / 4, columns 4 (i % 4) .. + 3 of its 16.
+          const int i16 = lane & 15, g2 = (lane >> 4) & 1;
+          const int n = wn * WN + j * 32 + 16 * g2 + 4 * (i16 & 3), nc = n % 64;
+          const unsigned char* bp = sb + A_BYTES + n / 64 * 8192 + (nc % 8) * 2;
+          const shortx4 x = ds_read_tr16_b64_tracked(bp + g_pos(16 * ks + 8 * lg + (i16 >> 2), nc / 8));
+          const shortx4 y = ds_read_tr16_b64_tracked(bp + g_pos(16 * ks + 8 * lg + 4 + (i16 >> 2), nc / 8));
+          bfr[ks][j] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    mid();
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      if constexpr (F32) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__builtin_bit_cast(floatx4, af[ks][i])[e],
+                                                               __builtin_bit_cast(floatx4, bfr[ks][j])[e], acc[i][j], 0,
+                                                               0, 0);
+      } else {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = mma32_16b<H>(af[ks][i], bfr[ks][j], acc[i][j]);
+      }
+    }
+  };
+  // Leading steps (every group's K-step a leading one): no branch around a
+  // load, so that each wait counts the loads issued after the one it waits
+  // for.  The last steps' loads past nfast repeat the last leading step.
+  const int nfast = kfast / KG;
+  if (nfast > 0) {
+#pragma unroll
+    for (int u = 0; u < PF; ++u) gload(min(u, nfast - 1), rra[u], rrb[u]);
+    lstore(0, rra[0], rrb[0]);
+    gload(min(PF, nfast - 1), rra[0], rrb[0]);
+    lds_barrier();
+#pragma unroll 1
+    for (int s0 = 0; s0 < nfast; s0 += PF)
+#pragma unroll
+      for (int u = 0; u < PF; ++u) {
+        const int s = s0 + u;
+        if (s >= nfast) break;
+        compute(s & 1, [&]() __attribute__((always_inline)) {
+          // The next K-step's LDS stores (its stage was read last in step
+          // s - 1) and the global loads PF steps after it.
+          lstore((s + 1) & 1, rra[(u + 1) % PF], rrb[(u + 1) % PF]);
+          gload(min(s + 1 + PF, nfast - 1), rra[(u + 1) % PF], rrb[(u + 1) % PF]);
+        });
+        lds_barrier();
+      }
+  }
+#pragma unroll 1
+  for (int s = nfast; s < nk; ++s) {
+    gload_checked(s, rra[0], rrb[0]);
+    lstore(s & 1, rra[0], rrb[0]);
+    lds_barrier();
+    compute(s & 1, []() {});
+    lds_barrier();
+  }
+
+  if constexpr (KG > 1) {
+    // Groups 1 .. KG-1 leave their accumulators in LDS (lane-major float4
+    // chunks); group 0 adds them in group order and writes the tile.
+    constexpr int NCH = TM * TN * 4;
+    static_assert((KG - 1) * WGM * WGN * NCH * 1024 <= 2 * SSET, "the partial sums fit the stages");
+    floatx4* red = reinterpret_cast<floatx4*>(lds);
+    if (kg > 0) {
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) {
+        const floatx16& a = acc[c / 4 / TN][c / 4 % TN];
+        red[(((kg - 1) * WGM * WGN + wid) * NCH + c) * 64 + lane] =
+            floatx4{a[4 * (c % 4)], a[4 * (c % 4) + 1], a[4 * (c % 4) + 2], a[4 * (c % 4) + 3]};
+      }
+    }
+    lds_barrier();
+    if (kg > 0) return;
+#pragma unroll
+    for (int g = 1; g < KG; ++g)
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) {
+        const floatx4 v = red[(((g - 1) * WGM * WGN + wid) * NCH + c) * 64 + lane];
+        floatx16& a = acc[c / 4 / TN][c / 4 % TN];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[4 * (c % 4) + e] += v[e];
+      }
+  }
+
+  // Accumulator element e of tile (i, j) is C[row][col] with
+  // row = 8 * (e / 4) + 4 * (lane / 32) + e % 4, col = lane % 32.
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int col = n0 + wn * WN + j * 32 + lr;
+      if (col >= N) continue;
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const int row = m0 + wm * WM + i * 32 + 8 * (e / 4) + 4 * lg + (e % 4);
@@ -702,7 +895,7 @@ static bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 template <typename TO>
 static bool staged_ok(const GemmArgs& a) {
   constexpr long OE = 16 / sizeof(TO);
-  const bool c_ok = aligned16(a.C) && a.ldc % OE == 0 && a.sC % OE == 0 && a.N % OE == 0;
+  const bool c_ok = aligned16(a.C) && a.ldc % OE == 0 && a.sC % OE == 0 && a.Nc % OE == 0;
   const bool r_ok = !a.R || (aligned16(a.R) && a.ldr % OE == 0 && a.sR % OE == 0);
   return c_ok && r_ok;
 }
@@ -829,7 +1022,7 @@ static TilePlan plan_tiles(const GemmArgs& a, DmaTile t, int batch, bool swiglu)
   TilePlan best{t, 0, t};
   if (batch != 1 || forced_tile() >= 0 || round_step_us(t) == 0.0) return best;
   const long cus = gemm_cus();
-  const double nk = (a.K + G_BK - 1) / G_BK;
+  const double nk = (a.K + 63) / 64;
   auto cost = [&](DmaTile x, int n) {
     int bm, bn;
     tile_dims(x, bm, bn);
@@ -865,9 +1058,10 @@ static void launch_dma_cols(DmaTile t, const GemmArgs& g, int batch, bool swiglu
     return;
   }
   GemmArgs g1 = g, g2 = g;
-  g1.N = pl.n1;
+  g1.N = g1.Nc = pl.n1;
   g2.N = g.N - pl.n1;
-  const uint16_t* B = static_cast<const uint16_t*>(g.B);
+  g2.Nc = g.Nc - pl.n1;
+  const TI* B = static_cast<const TI*>(g.B);
   g2.B = BT ? B + (long)pl.n1 * g.ldb : B + pl.n1;
   const long coff = swiglu ? pl.n1 / 2 : pl.n1;
   g2.C = static_cast<TO*>(g.C) + coff;
@@ -876,64 +1070,256 @@ static void launch_dma_cols(DmaTile t, const GemmArgs& g, int batch, bool swiglu
   launch_dma<TI, TO, BT>(pl.t2, g2, 1, st);
 }
 
-template <typename T, typename TO, bool BT>
-static int gemm_dispatch(const GemmArgs& a, int batch, int variant, hipStream_t st) {
+template <typename T, typename TO, bool BT, int BM, int BN, int WGM, int WGN, int KG, int PF>
+static void launch_reg(const GemmArgs& a, int batch, hipStream_t st) {
+  const dim3 grid((unsigned)tiles_of(a, BM, BN, 1), 1, (unsigned)batch);
+  gemm_reg_kernel<T, TO, BM, BN, BT, WGM, WGN, KG, PF><<<grid, dim3(64 * WGM * WGN * KG), 0, st>>>(a);
+}
+
+// fp32 tiles of the LDS-DMA kernel (two or four K groups each).
+enum F32Tile { kF128x128, kF64x128, kF64x64, kF32x64, kF32x32 };
+
+template <typename TO, bool BT>
+static void launch_f32(int t, const GemmArgs& g, int batch, hipStream_t st) {
+  auto grid = [&](int bm, int bn) { return dim3((unsigned)tiles_of(g, bm, bn, 1), 1, (unsigned)batch); };
+  switch (t) {
+    case kF128x128: gemm_dma_kernel<float, TO, 128, 128, BT, 2, 2, 2, 2><<<grid(128, 128), dim3(512), 0, st>>>(g); break;
+    case kF64x128: gemm_dma_kernel<float, TO, 64, 128, BT, 3, 2, 2, 2><<<grid(64, 128), dim3(512), 0, st>>>(g); break;
+    case kF64x64: gemm_dma_kernel<float, TO, 64, 64, BT, 4, 2, 2, 2><<<grid(64, 64), dim3(512), 0, st>>>(g); break;
+    case kF32x64: gemm_dma_kernel<float, TO, 32, 64, BT, 3, 1, 2, 4><<<grid(32, 64), dim3(512), 0, st>>>(g); break;
+    default: gemm_dma_kernel<float, TO, 32, 32, BT, 4, 1, 1, 4><<<grid(32, 32), dim3(256), 0, st>>>(g); break;
+  }
+}
+
+// The LDS-DMA kernel takes 16-byte chunks at 32-bit buffer offsets.
+template <typename T, bool BT>
+static bool dma_ok(const GemmArgs& a) {
   constexpr int E = VecE<T>::value;
-  const bool vec = aligned16(a.A) && aligned16(a.B) && a.K % E == 0 && a.lda % E == 0 && a.ldb % E == 0 &&
-                   a.sA % E == 0 && a.sB % E == 0 && (BT || a.N % E == 0);
-  constexpr bool half = std::is_same<T, f16>::value;
-  if constexpr (half) {
-    // fp16 operands: the LDS-DMA kernel, or for the naive variant, unaligned
-    // operands, K or leading dimensions off a multiple of 8 and operands over
-    // 2 GiB, the one-tile-per-wavefront kernel.
-    const long a_bytes = 2L * ((long)(a.M - 1) * a.lda + a.K), b_bytes = BT ? 2L * ((long)(a.N - 1) * a.ldb + a.K)
-                                                                        : 2L * ((long)(a.K - 1) * a.ldb + a.N);
-    if (variant == NKL_GEMM_NAIVE || !vec || a_bytes >= (1L << 31) || b_bytes >= (1L << 31)) {
-      const long tiles = (long)((a.M + 31) / 32) * ((a.N + 31) / 32);
-      gemm_naive_kernel<T, TO, BT><<<dim3((unsigned)((tiles + 3) / 4), 1, batch), dim3(256), 0, st>>>(a);
-      return check_launch("nkl_gemm(naive)");
-    }
+  constexpr long SZ = sizeof(T);
+  const int K = a.Kall ? a.Kall : a.K;
+  const long a_bytes = SZ * ((long)(a.M - 1) * a.lda + K),
+             b_bytes = SZ * (BT ? (long)(a.N - 1) * a.ldb + K : (long)(K - 1) * a.ldb + a.N);
+  return aligned16(a.A) && aligned16(a.B) && (K % E == 0 || a.padded) && a.lda % E == 0 && a.ldb % E == 0 && a.sA % E == 0 &&
+         a.sB % E == 0 && (BT || a.N % E == 0) && a_bytes < (1L << 31) && b_bytes < (1L << 31);
+}
+
+// The smallest tile that needs one round of workgroups (us: 512^3 7.2 with
+// 32x32, 9.4 32x64, 13.5 64x64; 300 x 1024 x K 256 5.6 / 6.9 / 8.6 at N 768,
+// 9.5 / 7.0 / 8.6 at N 1024, whose 320 tiles of 32x32 make two rounds;
+// 1000^3 39 / 30 / 25.7), else the least of rounds times the time per 32
+// elements of K of a round.
+static F32Tile choose_f32_tile(const GemmArgs& a, int batch) {
+  if (tiles_of(a, 32, 32, batch) <= 256) return kF32x32;
+  if (tiles_of(a, 32, 64, batch) <= 256) return kF32x64;
+  auto rounds = [&](int bm, int bn) { return (double)((tiles_of(a, bm, bn, batch) + 255) / 256); };
+  const double c64 = 0.69 * rounds(64, 64), c64x128 = 1.2 * rounds(64, 128), c128 = 2.0 * rounds(128, 128);
+  return c128 <= c64x128 && c128 <= c64 ? kF128x128 : c64x128 < c64 ? kF64x128 : kF64x64;
+}
+
+// One product (or a batch of them) into C, by the kernel its operands allow.
+template <typename T, typename TO, bool BT>
+static void gemm_launch(const GemmArgs& a, int batch, hipStream_t st) {
+  if (dma_ok<T, BT>(a)) {
     GemmArgs g = a;
     g.epi = staged_ok<TO>(a) ? kEpiStaged : kEpiElem;
-    launch_dma_cols<f16, TO, BT>(choose_tile(a, batch), g, batch, false, st);
-    return check_launch("nkl_gemm(blocked)");
-  } else {
-  if (variant == NKL_GEMM_NAIVE || !vec) {
+    if constexpr (sizeof(T) == 4)
+      launch_f32<TO, BT>(choose_f32_tile(a, batch), g, batch, st);
+    else
+      launch_dma_cols<T, TO, BT>(choose_tile(a, batch), g, batch, false, st);
+    return;
+  }
+  // 128x128 from one such tile per CU (4001 x 4099 x 3999 bf16 225 us, 64x64
+  // 395; level at 1501 x 2049 x 2047); fp32 grids that 32x64 tiles of four K
+  // groups cover in one round take those (300 x 256 x 1024 7.2 us, 64x64 8.9).
+  if (tiles_of(a, 128, 128, batch) >= 256)
+    launch_reg<T, TO, BT, 128, 128, 2, 2, 1, 1>(a, batch, st);
+  else if (sizeof(T) == 4 && tiles_of(a, 32, 64, batch) <= 256)
+    launch_reg<T, TO, BT, 32, 64, 1, 2, 4, 2>(a, batch, st);
+  else
+    launch_reg<T, TO, BT, 64, 64, 2, 2, 1, 1>(a, batch, st);
+}
+
+// -------------------------------------- workspace: packed operands, split K --
+// Copies rows of `cols` elements (source stride ld) to rows of ldp elements (a
+// multiple of 16 bytes, zeros past cols): one 16-byte chunk per thread, A's
+// chunks first, then B's.
+struct PackArgs {
+  const void* src[2];
+  void* dst[2];
+  long ld[2], ldp[2];
+  int cols[2];
+  long chunks[2];  // 16-byte chunks of each destination (0: not packed)
+};
+template <typename T>
+__global__ __launch_bounds__(256) void gemm_pack_kernel(PackArgs p) {
+  constexpr int E = VecE<T>::value;
+  long c = (long)blockIdx.x * 256 + threadIdx.x;
+  const int w = c >= p.chunks[0];
+  if (w) c -= p.chunks[0];
+  if (c >= p.chunks[w]) return;
+  const long cpr = p.ldp[w] / E;
+  const long r = c / cpr;
+  const int k = (int)(c - r * cpr) * E;
+  const u32x4_t v = ld16_first(static_cast<const T*>(p.src[w]) + r * p.ld[w] + k, p.cols[w] - k);
+  *reinterpret_cast<u32x4_t*>(static_cast<T*>(p.dst[w]) + r * p.ldp[w] + k) = v;
+}
+
+// C = sum over z < splits of P[z] (+ R), in the order of z; P: [splits][M][N] fp32.
+template <typename TO>
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restrict__ P, int splits, GemmArgs p) {
+  const long mn = (long)p.M * p.Nc;
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= mn) return;
+  const long r = i / p.Nc, c = i - r * p.Nc;
+  float v = 0.f;
+#pragma unroll 8
+  for (int z = 0; z < splits; ++z) v += P[z * mn + i];
+  if (p.R) v += to_f32(static_cast<const TO*>(p.R)[r * p.ldr + c]);
+  static_cast<TO*>(p.C)[r * p.ldc + c] = from_f32<TO>(v);
+}
+
+// What one product does beyond a plain launch, and the workspace it takes.
+struct WsPlan {
+  bool pack;           // copy the operands the LDS-DMA kernel cannot take into aligned rows
+  bool pack_a, pack_b;
+  long kp, np;         // packed K (A, B^T) and N (B as [K, N])
+  int splits, kc;      // parts of K, and K elements of a part
+  size_t a_off, b_off, p_off, bytes;
+};
+template <typename T, bool BT>
+static WsPlan plan_ws(const GemmArgs& a) {
+  constexpr int E = VecE<T>::value;
+  constexpr int BK = 128 / (int)sizeof(T);
+  WsPlan w{};
+  auto up = [](size_t x) { return (x + 255) / 256 * 256; };
+  w.kp = a.K;
+  w.np = a.N;
+  // Packing pays from two rounds of 128x128 tiles on (bf16 4001 x 4099 x 3999
+  // 225 -> 159 us; 1501 x 2049 x 2047, 192 tiles, 40 -> 44); the fp32 kernels
+  // are close enough to each other that it does not.
+  if (sizeof(T) == 2 && !dma_ok<T, BT>(a) && tiles_of(a, 128, 128, 1) >= 512) {
+    w.pack_a = !aligned16(a.A) || a.K % E || a.lda % E;  // (K off a vector: zeros in A, and in B^T)
+    w.pack_b = !aligned16(a.B) || a.ldb % E || (BT ? a.K % E : a.N % E);
+    w.pack = w.pack_a || w.pack_b;
+    w.kp = (a.K + E - 1) / E * E;
+    if (!BT) w.np = (a.N + E - 1) / E * E;
+    if (w.pack_a) w.a_off = w.bytes, w.bytes += up(sizeof(T) * (size_t)a.M * w.kp);
+    if (w.pack_b) w.b_off = w.bytes, w.bytes += up(sizeof(T) * (BT ? (size_t)a.N * w.kp : (size_t)a.K * w.np));
+  }
+  // K is split over workgroups when their tiles leave half the CUs idle and K
+  // is long: parts of at least 8 K-steps, up to one workgroup per CU (bf16
+  // 8 x 8064 x 64 23.9 -> 7.2 us, 16 x 4096 x 4096 15.3 -> 12.4, 1 x 8192 x
+  // 8192 39 -> 31; 304 x 1024 x 256 6.4 -> 7.9, so not below 48 K-steps).
+  const bool dma = w.pack || dma_ok<T, BT>(a);
+  const long tiles = sizeof(T) == 2 ? tiles_of(a, 64, 64, 1) : dma ? tiles_of(a, 32, 32, 1) : tiles_of(a, 32, 64, 1);
+  const int steps = (a.K + BK - 1) / BK;
+  w.splits = 1;
+  if (tiles <= 128 && steps >= 48) {
+    const int want = (int)min(256 / tiles, (long)steps / 8), per = (steps + want - 1) / want;
+    w.kc = per * BK;
+    w.splits = (steps + per - 1) / per;
+    if (w.splits > 1) w.p_off = w.bytes, w.bytes += up(4 * (size_t)w.splits * a.M * a.Nc);
+  }
+  return w;
+}
+
+// A call's workspace: whether it may use one, and `need` to ask for its size
+// instead of launching.
+struct Workspace {
+  bool use;
+  void* p;
+  size_t bytes;
+  size_t* need;
+};
+
+template <typename T, typename TO, bool BT>
+static int gemm_dispatch(const GemmArgs& a, int batch, int variant, Workspace ws, hipStream_t st) {
+  if (variant == NKL_GEMM_NAIVE) {
     const long tiles = (long)((a.M + 31) / 32) * ((a.N + 31) / 32);
     gemm_naive_kernel<T, TO, BT><<<dim3((unsigned)((tiles + 3) / 4), 1, batch), dim3(256), 0, st>>>(a);
     return check_launch("nkl_gemm(naive)");
   }
-  const long t128 = (long)((a.M + 127) / 128) * ((a.N + 127) / 128) * batch;
-  const long t64x128 = (long)((a.M + 63) / 64) * ((a.N + 127) / 128) * batch;
-  if constexpr (std::is_same<T, bf16>::value) {
-    // bf16: the LDS-DMA kernel, whose buffer offsets need operands under 2 GB.
-    const long a_bytes = 2L * ((long)(a.M - 1) * a.lda + a.K), b_bytes = BT ? 2L * ((long)(a.N - 1) * a.ldb + a.K)
-                                                                        : 2L * ((long)(a.K - 1) * a.ldb + a.N);
-    if (a_bytes < (1L << 31) && b_bytes < (1L << 31)) {
+  if (ws.use) {  // (batch 1)
+    const WsPlan w = plan_ws<T, BT>(a);
+    if (ws.need) return *ws.need = w.bytes, NKL_OK;
+    if (w.bytes > 0) {
+      if (!ws.p || ws.bytes < w.bytes)
+        return set_error(NKL_EWORKSPACE, "nkl_gemm_ws: workspace of %zu bytes needed, %zu given", w.bytes, ws.bytes);
       GemmArgs g = a;
-      g.epi = staged_ok<TO>(a) ? kEpiStaged : kEpiElem;
-      launch_dma_cols<bf16, TO, BT>(choose_tile(a, batch), g, batch, false, st);
-      return check_launch("nkl_gemm(blocked)");
+      char* base = static_cast<char*>(ws.p);
+      if (w.pack) {
+        constexpr int E = VecE<T>::value;
+        PackArgs k{};
+        if (w.pack_a) {
+          k.src[0] = a.A, k.dst[0] = base + w.a_off, k.ld[0] = a.lda, k.ldp[0] = w.kp, k.cols[0] = a.K;
+          k.chunks[0] = (long)a.M * (w.kp / E);
+          g.A = k.dst[0], g.lda = w.kp;
+        }
+        if (w.pack_b) {
+          k.src[1] = a.B, k.dst[1] = base + w.b_off, k.ld[1] = a.ldb, k.ldp[1] = BT ? w.kp : w.np;
+          k.cols[1] = BT ? a.K : a.N;
+          k.chunks[1] = BT ? (long)a.N * (w.kp / E) : (long)a.K * (w.np / E);
+          g.B = k.dst[1], g.ldb = k.ldp[1];
+        }
+        gemm_pack_kernel<T><<<dim3((unsigned)((k.chunks[0] + k.chunks[1] + 255) / 256)), dim3(256), 0, st>>>(k);
+        g.N = (int)w.np, g.padded = 1;
+      }
+      if (w.splits > 1) {
+        GemmArgs part = g;
+        part.Kall = g.K;
+        part.K = w.kc;
+        part.sA = w.kc;
+        part.sB = BT ? w.kc : w.kc * g.ldb;
+        part.C = base + w.p_off;
+        part.ldc = a.Nc;
+        part.sC = (long)a.M * a.Nc;
+        part.R = nullptr;
+        gemm_launch<T, float, BT>(part, w.splits, st);
+        const long mn = (long)a.M * a.Nc;
+        gemm_reduce_kernel<TO><<<dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, st>>>(
+            reinterpret_cast<const float*>(base + w.p_off), w.splits, a);
+      } else {
+        gemm_launch<T, TO, BT>(g, 1, st);
+      }
+      return check_launch("nkl_gemm_ws");
     }
   }
-  if (t128 >= 256) {
-    const long tiles = (long)((a.M + 127) / 128) * ((a.N + 127) / 128);
-    gemm_blocked_kernel<T, TO, 128, 128, BT><<<dim3((unsigned)tiles, 1, batch), dim3(256), 0, st>>>(a);
-  } else if (t64x128 >= 256) {
-    const long tiles = (long)((a.M + 63) / 64) * ((a.N + 127) / 128);
-    gemm_blocked_kernel<T, TO, 64, 128, BT><<<dim3((unsigned)tiles, 1, batch), dim3(256), 0, st>>>(a);
-  } else {
-    const long tiles = (long)((a.M + 63) / 64) * ((a.N + 63) / 64);
-    gemm_blocked_kernel<T, TO, 64, 64, BT><<<dim3((unsigned)tiles, 1, batch), dim3(256), 0, st>>>(a);
-  }
+  gemm_launch<T, TO, BT>(a, batch, st);
   return check_launch("nkl_gemm(blocked)");
-  }
 }
 
 template <typename T, typename TO>
-static int gemm_layout(const GemmArgs& a, int b_trans, int batch, int variant, hipStream_t st) {
-  return b_trans ? gemm_dispatch<T, TO, true>(a, batch, variant, st)
-                 : gemm_dispatch<T, TO, false>(a, batch, variant, st);
+static int gemm_layout(const GemmArgs& a, int b_trans, int batch, int variant, Workspace ws,
+                       hipStream_t st) {
+  return b_trans ? gemm_dispatch<T, TO, true>(a, batch, variant, ws, st)
+                 : gemm_dispatch<T, TO, false>(a, batch, variant, ws, st);
+}
+
+// Checks the arguments, then launches (need null) or asks for the workspace.
+static int gemm_entry(const char* fn, const void* A, const void* B, void* C, const void* R, int M, int N, int K,
+                      long lda, long ldb, long ldc, long ldr, int b_trans, int batch, long strideA, long strideB,
+                      long strideC, long strideR, int dtype_in, int dtype_out, int variant, Workspace ws,
+                      void* stream) {
+  if (M < 0 || N < 0 || K < 0 || batch < 0)
+    return set_error(NKL_EINVAL, "%s: negative shape M=%d N=%d K=%d batch=%d", fn, M, N, K, batch);
+  if (variant != NKL_GEMM_BLOCKED && variant != NKL_GEMM_NAIVE)
+    return set_error(NKL_EINVAL, "%s: unknown variant %d", fn, variant);
+  if (M == 0 || N == 0 || batch == 0) return NKL_OK;
+  if (lda < K || ldc < N || (R && ldr < N) || (b_trans ? ldb < K : ldb < N))
+    return set_error(NKL_EINVAL, "%s: leading dimension too small (lda=%ld ldb=%ld ldc=%ld)", fn, lda, ldb, ldc);
+  if (!A || !B || (!C && !ws.need)) return set_error(NKL_EINVAL, "%s: null operand pointer", fn);
+  GemmArgs a{A, B, C, R, M, N, K, lda, ldb, ldc, ldr, strideA, strideB, strideC, strideR, kEpiElem, N, 0, 0};
+  hipStream_t st = (hipStream_t)stream;
+#define NKL_GEMM_TYPES(ti, TI, to, TO)  \
+  if (dtype_in == ti && dtype_out == to) \
+  return gemm_layout<TI, TO>(a, b_trans, batch, variant, ws, st)
+  NKL_GEMM_TYPES(NKL_F32, float, NKL_F32, float);
+  NKL_GEMM_TYPES(NKL_BF16, bf16, NKL_BF16, bf16);
+  NKL_GEMM_TYPES(NKL_BF16, bf16, NKL_F32, float);
+  NKL_GEMM_TYPES(NKL_F16, f16, NKL_F16, f16);
+  NKL_GEMM_TYPES(NKL_F16, f16, NKL_F32, float);
+#undef NKL_GEMM_TYPES
+  return set_error(NKL_EDTYPE, "%s: unsupported dtype pair (%d -> %d)", fn, dtype_in, dtype_out);
 }
 
 }  // namespace nkl
@@ -943,22 +1329,24 @@ using namespace nkl;
 extern "C" int nkl_gemm(const void* A, const void* B, void* C, const void* R, int M, int N, int K, long lda,
                         long ldb, long ldc, long ldr, int b_trans, int batch, long strideA, long strideB,
                         long strideC, long strideR, int dtype_in, int dtype_out, int variant, void* stream) {
-  if (M < 0 || N < 0 || K < 0 || batch < 0)
-    return set_error(NKL_EINVAL, "nkl_gemm: negative shape M=%d N=%d K=%d batch=%d", M, N, K, batch);
-  if (variant != NKL_GEMM_BLOCKED && variant != NKL_GEMM_NAIVE)
-    return set_error(NKL_EINVAL, "nkl_gemm: unknown variant %d", variant);
-  if (M == 0 || N == 0 || batch == 0) return NKL_OK;
-  if (lda < K || ldc < N || (R && ldr < N) || (b_trans ? ldb < K : ldb < N))
-    return set_error(NKL_EINVAL, "nkl_gemm: leading dimension too small (lda=%ld ldb=%ld ldc=%ld)", lda, ldb, ldc);
-  if (!A || !B || !C) return set_error(NKL_EINVAL, "nkl_gemm: null operand pointer");
-  GemmArgs a{A, B, C, R, M, N, K, lda, ldb, ldc, ldr, strideA, strideB, strideC, strideR};
-  hipStream_t st = (hipStream_t)stream;
-  if (dtype_in == NKL_F32 && dtype_out == NKL_F32) return gemm_layout<float, float>(a, b_trans, batch, variant, st);
-  if (dtype_in == NKL_BF16 && dtype_out == NKL_BF16) return gemm_layout<bf16, bf16>(a, b_trans, batch, variant, st);
-  if (dtype_in == NKL_BF16 && dtype_out == NKL_F32) return gemm_layout<bf16, float>(a, b_trans, batch, variant, st);
-  if (dtype_in == NKL_F16 && dtype_out == NKL_F16) return gemm_layout<f16, f16>(a, b_trans, batch, variant, st);
-  if (dtype_in == NKL_F16 && dtype_out == NKL_F32) return gemm_layout<f16, float>(a, b_trans, batch, variant, st);
-  return set_error(NKL_EDTYPE, "nkl_gemm: unsupported dtype pair (%d -> %d)", dtype_in, dtype_out);
+  return gemm_entry("nkl_gemm", A, B, C, R, M, N, K, lda, ldb, ldc, ldr, b_trans, batch, strideA, strideB, strideC,
+                    strideR, dtype_in, dtype_out, variant, Workspace{}, stream);
+}
+
+extern "C" size_t nkl_gemm_workspace_bytes(const void* A, const void* B, int M, int N, int K, long lda, long ldb,
+                                           int b_trans, int dtype_in, int dtype_out) {
+  size_t need = 0;
+  const int rc = gemm_entry("nkl_gemm_workspace_bytes", A, B, nullptr, nullptr, M, N, K, lda, ldb, N, 0, b_trans, 1, 0,
+                            0, 0, 0, dtype_in, dtype_out, NKL_GEMM_BLOCKED, Workspace{true, nullptr, 0, &need},
+                            nullptr);
+  return rc == NKL_OK ? need : 0;
+}
+
+extern "C" int nkl_gemm_ws(const void* A, const void* B, void* C, const void* R, void* workspace,
+                           size_t workspace_bytes, int M, int N, int K, long lda, long ldb, long ldc, long ldr,
+                           int b_trans, int dtype_in, int dtype_out, void* stream) {
+  return gemm_entry("nkl_gemm_ws", A, B, C, R, M, N, K, lda, ldb, ldc, ldr, b_trans, 1, 0, 0, 0, 0, dtype_in, dtype_out,
+                    NKL_GEMM_BLOCKED, Workspace{true, workspace, workspace_bytes, nullptr}, stream);
 }
 
 extern "C" int nkl_gemm_swiglu(const void* A, const void* Bgu, void* C, int M, int N, int K, long lda, long ldb,
@@ -980,7 +1368,7 @@ extern "C" int nkl_gemm_swiglu(const void* A, const void* Bgu, void* C, int M, i
   const long a_bytes = 2L * ((long)(M - 1) * lda + K), b_bytes = 2L * ((long)(2L * N - 1) * ldb + K);
   if (a_bytes >= (1L << 31) || b_bytes >= (1L << 31))
     return set_error(NKL_EINVAL, "nkl_gemm_swiglu: operands must be under 2 GiB");
-  GemmArgs a{A, Bgu, C, nullptr, M, 2 * N, K, lda, ldb, ldc, 0, 0, 0, 0, 0, kEpiSwiglu};
+  GemmArgs a{A, Bgu, C, nullptr, M, 2 * N, K, lda, ldb, ldc, 0, 0, 0, 0, 0, kEpiSwiglu, 2 * N, 0, 0};
   hipStream_t st = (hipStream_t)stream;
   // A tile whose wavefronts own 64 columns (one gate/up pair), summing the
   // K-steps in the order the separate M x N gate and up GEMMs would: in two

@@ -13,6 +13,7 @@ LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
 
 F32, BF16, F16 = 0, 1, 2
 GEMM_BLOCKED, GEMM_NAIVE = 0, 1
+EWORKSPACE = -4
 ABI_VERSION = 1
 
 _c_int, _c_long, _c_float, _c_size = ctypes.c_int, ctypes.c_long, ctypes.c_float, ctypes.c_size_t
@@ -24,6 +25,9 @@ SIGNATURES = {
     "nkl_last_error_string": (ctypes.c_char_p, []),
     "nkl_gemm": (_c_int, [_vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _c_long, _c_long, _c_long, _c_long,
                           _c_int, _c_int, _c_long, _c_long, _c_long, _c_long, _c_int, _c_int, _c_int, _vp]),
+    "nkl_gemm_workspace_bytes": (_c_size, [_vp, _vp, _c_int, _c_int, _c_int, _c_long, _c_long, _c_int, _c_int, _c_int]),
+    "nkl_gemm_ws": (_c_int, [_vp, _vp, _vp, _vp, _vp, _c_size, _c_int, _c_int, _c_int, _c_long, _c_long, _c_long,
+                             _c_long, _c_int, _c_int, _c_int, _vp]),
     "nkl_gemm_swiglu": (_c_int, [_vp, _vp, _vp, _c_int, _c_int, _c_int, _c_long, _c_long, _c_long, _c_int, _vp]),
     "nkl_check_blocks": (_c_int, [_c_int, _c_int]),
     "nkl_softmax": (_c_int, [_vp, _vp, _c_int, _c_int, _c_long, _c_long, _c_int, _vp]),
@@ -120,13 +124,16 @@ def flash_plan_check(H: int, S: int, d: int, f16: bool = False) -> tuple[int, in
     return tuple(info)
 
 
-def call(name: str, *args) -> int:
-    """Call a status-returning entry point and raise on failure."""
-    L = lib()
-    rc = getattr(L, name)(*args)
+def check(name: str, rc: int) -> int:
+    """Raise on a failure status of entry point `name`."""
     if rc != 0:
-        msg = L.nkl_last_error_string().decode(errors="replace")
+        msg = lib().nkl_last_error_string().decode(errors="replace")
         if rc == -1 and "PSUM" not in msg:
             raise ValueError(f"{name}: {msg}")
         raise NklError(name, rc, msg)
     return rc
+
+
+def call(name: str, *args) -> int:
+    """Call a status-returning entry point and raise on failure."""
+    return check(name, getattr(lib(), name)(*args))

@@ -91,9 +91,20 @@ def _gemm(a: torch.Tensor, bmat: torch.Tensor, ldb: int, b_trans: bool, c: torch
     if K == 0:
         c.copy_(residual if residual is not None else torch.zeros_like(c))
         return c
-    _lib.call("nkl_gemm", ptr(a), ptr(bmat), ptr(c), ptr(residual), M, N, K, lda, ldb, ldc, ldr,
-              int(b_trans), 1, 0, 0, 0, 0, dtype_code(a.dtype), dtype_code(c.dtype),
-              _MATMUL_VARIANTS[variant], stream_handle())
+    pa, pb, pc, pr, st = ptr(a), ptr(bmat), ptr(c), ptr(residual), stream_handle()
+    dt_in, dt_out, bt = dtype_code(a.dtype), dtype_code(c.dtype), int(b_trans)
+    if _MATMUL_VARIANTS[variant] == _lib.GEMM_NAIVE:
+        _lib.call("nkl_gemm", pa, pb, pc, pr, M, N, K, lda, ldb, ldc, ldr, bt, 1, 0, 0, 0, 0, dt_in, dt_out,
+                  _lib.GEMM_NAIVE, st)
+        return c
+    # Most shapes need no workspace; the call says so before it launches anything.
+    rc = _lib.lib().nkl_gemm_ws(pa, pb, pc, pr, None, 0, M, N, K, lda, ldb, ldc, ldr, bt, dt_in, dt_out, st)
+    if rc == _lib.EWORKSPACE:
+        nbytes = _lib.lib().nkl_gemm_workspace_bytes(pa, pb, M, N, K, lda, ldb, bt, dt_in, dt_out)
+        ws = workspace(nbytes, c.device)
+        rc = _lib.lib().nkl_gemm_ws(pa, pb, pc, pr, ptr(ws), nbytes, M, N, K, lda, ldb, ldc, ldr, bt, dt_in, dt_out,
+                                    st)
+    _lib.check("nkl_gemm_ws", rc)
     return c
 
 

@@ -265,3 +265,59 @@ def test_batched_gemm_on_large_tiles(rng, layout):
         bt = b[i].double().cpu() if layout == "nn" else b[i].double().cpu().t()
         ref = (a[i].double().cpu() @ bt + r[i].double().cpu()).numpy()
         assert_within_bf16_ulps(_np(c[i]), ref, 1, floor=2e-3)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,N,off", [
+    (1, 1, 1, 0), (1, 7, 3, 1), (33, 5, 2, 0), (31, 63, 65, 3), (64, 64, 64, 1), (65, 129, 33, 0),  # K and N tails
+    (300, 256, 1024, 0), (300, 1024, 256, 0), (1000, 1000, 1000, 0), (2000, 96, 1000, 0),           # fp32 tile choice
+    (130, 515, 2050, 1), (2049, 71, 2051, 0), (8, 8021, 64, 0), (16, 4096, 260, 0), (9, 3333, 31, 5),  # K split
+    (2945, 137, 2947, 0)])                                                                           # packed operands
+def test_gemm_any_shape_and_alignment(dt, M, K, N, off):
+    """Every staging path, tile choice, K split and operand copy, both layouts
+    and a residual, as views `off` elements into wider rows of NaN (so that
+    anything read past K or N would show), against float64: within K roundings
+    of 2^-24 of the sum of |a b|, plus one rounding to the output type."""
+    from nkilab import ops
+
+    g = torch.Generator(device="cuda").manual_seed(M * 31 + K * 7 + N)
+
+    def operand(r, c):
+        buf = torch.full((r, c + (9 if off else 0)), float("nan"), dtype=dt, device="cuda")
+        v = buf[:, off:off + c]
+        v.copy_(torch.randn(r, c, generator=g, device="cuda"))
+        return v
+
+    u = {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dt]
+    for bt in (False, True):
+        a, b, r = operand(M, K), operand(N, K) if bt else operand(K, N), operand(M, N)
+        bd = b.double().t() if bt else b.double()
+        ref, mag = a.double() @ bd, a.double().abs() @ bd.abs()
+        run = ops.linear_into if bt else ops.gemm_into
+        for res in (None, r):
+            cb = torch.full((M, N + 3), 5.0, dtype=dt, device="cuda")
+            c = cb[:, 1:N + 1]
+            run(a, b, c, residual=res)
+            want = ref if res is None else ref + res.double()
+            bound = (K + 2) * 2.0 ** -24 * (mag + want.abs()) + u * want.abs() + 2.0 ** -24
+            assert ((c.double() - want).abs() <= bound).all(), (bt, res is not None)
+            assert (cb[:, 0] == 5).all() and (cb[:, N + 1:] == 5).all()
+            again = torch.empty(M, N, dtype=dt, device="cuda")
+            run(a, b, again, residual=res)
+            assert torch.equal(again, c)
+
+
+def test_gemm_workspace_is_for_the_shapes_that_use_it():
+    """No workspace where one launch serves (the common aligned shapes); the K
+    split and the packed operands ask for one, and refuse a smaller one."""
+    from nkilab import _lib
+
+    L = _lib.lib()
+    a = torch.empty(1 << 24, dtype=torch.bfloat16, device="cuda")
+    p = a.data_ptr()
+    assert L.nkl_gemm_workspace_bytes(p, p, 1024, 1024, 1024, 1024, 1024, 0, 1, 1) == 0
+    assert L.nkl_gemm_workspace_bytes(p, p, 1000, 1301, 777, 777, 1301, 0, 1, 1) == 0
+    need = L.nkl_gemm_workspace_bytes(p, p, 8, 64, 8064, 8064, 64, 0, 1, 1)
+    assert need >= 2 * 8 * 64 * 4
+    assert L.nkl_gemm_workspace_bytes(p, p, 2945, 2947, 137, 137, 2947, 0, 1, 1) > 0
+    assert L.nkl_gemm_ws(p, p, p, None, p, need - 1, 8, 64, 8064, 8064, 64, 64, 0, 0, 1, 1, None) == -4
