@@ -27,6 +27,9 @@ size_t flash_bf16_counter_bytes(int H, int S);
 int flash_bf16_launch(const AttnArgs& a, void* workspace, size_t workspace_bytes, int* counters,
                       size_t counter_bytes, hipStream_t st);
 
+// fp32 flash attention (flash_f32.hip): d up to 128, no scratch.
+int flash_f32_launch(const AttnArgs& a, hipStream_t st);
+
 namespace fsched {
 struct Work;
 }

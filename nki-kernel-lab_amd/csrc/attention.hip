@@ -1,22 +1,7 @@
 // Causal attention on gfx950.
 //
-// flash_fwd_kernel -- the hot path.  One 256-thread workgroup owns BM = 64
-// consecutive queries of one head; each of its four wavefronts owns 16 of
-// them.  Key/value tiles of BN keys stream through double-buffered LDS and
-// the running softmax state (max, sum, output) stays in registers, so
-// scores never leave the chip.  Key tiles entirely above the diagonal are
-// never visited; the tiles that straddle it are masked element-wise.
-//
-// Everything is computed transposed so that each lane always works on a
-// single query:
-//     S^T = K . Q^T      (A = K rows from LDS, B = Q^T fragments in VGPRs)
-//     O^T = V^T . P^T    (A = V^T from LDS,    B = P^T straight from S^T)
-// With 16x16 MFMAs, lane l holds query l % 16 of its wavefront in both the
-// S^T and O^T accumulators, so the running max / sum / correction factor are
-// per-lane scalars, and the probabilities produced by the exp are already in
-// the B-operand layout of the P.V MFMA (no shuffle, no LDS round trip).
-// For bf16 the V tile is written to LDS transposed and key-permuted so that
-// the V^T operand is one 16-byte read per MFMA.
+// Argument checks, workspaces and C entries of the flash kernels (flash_*.hip;
+// fp32: flash_f32.hip).
 //
 // attention_naive -- the reference's unfused variant: scores and
 // probabilities are materialised in a caller-provided workspace, using the
@@ -27,262 +12,6 @@
 
 namespace nkl {
 
-
-template <typename T>
-struct FlashCfg;
-template <>
-struct FlashCfg<bf16> { static constexpr int BN = 64; };
-template <>
-struct FlashCfg<float> { static constexpr int BN = 32; };
-
-// bf16 V^T layout: within a tile of 64 keys, key kk = 16 * kb + 4 * g + i
-// (kb < 4, g < 4, i < 4) is stored at column 32 * (kb / 2) + 8 * g +
-// 4 * (kb % 2) + i, so that lane group g's eight keys of MFMA t = kb / 2 are
-// contiguous -- the same order in which the lane holds their probabilities.
-__device__ __forceinline__ int vt_col(int kk) {
-  const int kb = kk >> 4, g = (kk >> 2) & 3, i = kk & 3;
-  return 32 * (kb >> 1) + 8 * g + 4 * (kb & 1) + i;
-}
-
-template <typename T, int D>
-__global__ __launch_bounds__(256) void flash_fwd_kernel(AttnArgs p) {
-  using MF = Mfma16<T>;
-  constexpr bool BF = sizeof(T) == 2;
-  constexpr int BM = 64;
-  constexpr int BN = FlashCfg<T>::BN;
-  constexpr int E = VecE<T>::value;      // elements per 16-byte chunk
-  constexpr int CPR = D / E;             // 16-byte chunks per K/V row
-  constexpr int LDK = D + E;             // K (and f32 V) LDS row stride, padded
-  constexpr int LDV = BN + 8;            // bf16 V^T LDS row stride, padded
-  constexpr int K_CH = BN * CPR / 256;   // K chunks per thread
-  constexpr int NKB = BN / 16;           // 16-key sub-blocks per tile
-  constexpr int ND = D / 16;             // 16-wide d blocks of O^T
-  constexpr int NQF = D / MF::MK;        // Q fragments per lane
-  static_assert(K_CH >= 1 && (BN * CPR) % 256 == 0, "tile does not split over 256 threads");
-
-  constexpr int V_ELEMS = BF ? D * LDV : BN * LDK;
-  __shared__ T Ks[2][BN * LDK];
-  __shared__ T Vs[2][V_ELEMS];
-
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int g = lane >> 4, r = lane & 15;
-  const int S = p.S, dlim = p.d;
-
-  // Heavy-first: the first workgroups dispatched take the query blocks with
-  // the most key tiles; consecutive ids walk the heads, so with 8 heads head
-  // h always lands on XCD h and its K/V stay in one L2.
-  const int nqb = (S + BM - 1) / BM;
-  const int h = blockIdx.x % p.H;
-  const int qb = nqb - 1 - blockIdx.x / p.H;
-  const int q0 = qb * BM;
-  const int qw = q0 + 16 * w;   // first query of this wavefront
-  const int myq = qw + r;       // this lane's query
-
-  const T* Q = static_cast<const T*>(p.q) + (long)h * p.q_sh;
-  const T* K = static_cast<const T*>(p.k) + (long)(h / p.group) * p.k_sh;  // shared K/V head (GQA)
-  const T* V = static_cast<const T*>(p.v) + (long)(h / p.group) * p.v_sh;
-  T* O = static_cast<T*>(p.o) + (long)h * p.o_sh;
-
-  // Q^T fragments: lane (r, g) holds Q[myq][MK * f + KPER * g + j].
-  typename MF::frag qf[NQF];
-#pragma unroll
-  for (int f = 0; f < NQF; ++f) {
-    const int dd = f * MF::MK + g * MF::KPER;
-    if constexpr (BF) {
-      if (myq < S && dd < dlim)
-        qf[f] = load_frag(Q + (long)myq * p.q_ss + dd);
-      else
-#pragma unroll
-        for (int j = 0; j < 8; ++j) qf[f][j] = (bf16)0.f;
-    } else {
-      qf[f] = (myq < S && dd < dlim) ? Q[(long)myq * p.q_ss + dd] : 0.f;
-    }
-  }
-
-  // ---- K/V staging: global -> registers -> LDS.
-  uint4 rk[K_CH];
-  // bf16 V: a thread moves 4 consecutive keys x 8 d values.
-  constexpr int V_GRP = BF ? (BN / 4) * (D / 8) : 0;
-  constexpr int V_IT = BF ? (V_GRP + 255) / 256 : K_CH;
-  uint4 rv[BF ? V_IT * 4 : K_CH];
-  auto gload = [&](int k0) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < K_CH; ++i) {
-      const int c = tid + 256 * i, row = c / CPR, cc = (c % CPR) * E;
-      const int key = k0 + row;
-      rk[i] = ld16_or_zero(K, (long)key * p.k_ss + cc, key < S && cc < dlim);
-      if constexpr (!BF)
-        rv[i] = ld16_or_zero(V, (long)key * p.v_ss + cc, key < S && cc < dlim);
-    }
-    if constexpr (BF) {
-#pragma unroll
-      for (int it = 0; it < V_IT; ++it) {
-        const int grp = tid + 256 * it;
-        const int kg = grp % (BN / 4), dc = (grp / (BN / 4)) * 8;
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-          const int key = k0 + 4 * kg + rr;
-          rv[it * 4 + rr] = ld16_or_zero(V, (long)key * p.v_ss + dc, grp < V_GRP && key < S && dc < dlim);
-        }
-      }
-    }
-  };
-
-  auto lstore = [&](int buf) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < K_CH; ++i) {
-      const int c = tid + 256 * i, row = c / CPR, cc = (c % CPR) * E;
-      *reinterpret_cast<uint4*>(&Ks[buf][row * LDK + cc]) = rk[i];
-      if constexpr (!BF) *reinterpret_cast<uint4*>(&Vs[buf][row * LDK + cc]) = rv[i];
-    }
-    if constexpr (BF) {
-#pragma unroll
-      for (int it = 0; it < V_IT; ++it) {
-        const int grp = tid + 256 * it;
-        if (grp < V_GRP) {
-          const int kg = grp % (BN / 4), dc = (grp / (BN / 4)) * 8;
-          const int col = vt_col(4 * kg);
-          const uint32_t* a0 = reinterpret_cast<const uint32_t*>(&rv[it * 4 + 0]);
-          const uint32_t* a1 = reinterpret_cast<const uint32_t*>(&rv[it * 4 + 1]);
-          const uint32_t* a2 = reinterpret_cast<const uint32_t*>(&rv[it * 4 + 2]);
-          const uint32_t* a3 = reinterpret_cast<const uint32_t*>(&rv[it * 4 + 3]);
-#pragma unroll
-          for (int jj = 0; jj < 8; ++jj) {
-            const int wd = jj >> 1;
-            uint2 t;
-            if (jj & 1) {
-              t.x = (a0[wd] >> 16) | (a1[wd] & 0xffff0000u);
-              t.y = (a2[wd] >> 16) | (a3[wd] & 0xffff0000u);
-            } else {
-              t.x = (a0[wd] & 0xffffu) | (a1[wd] << 16);
-              t.y = (a2[wd] & 0xffffu) | (a3[wd] << 16);
-            }
-            *reinterpret_cast<uint2*>(&Vs[buf][(dc + jj) * LDV + col]) = t;
-          }
-        }
-      }
-    }
-  };
-
-  // ---- running state for query myq
-  float m_run = -INFINITY;  // running max of s * c
-  float l_run = 0.f;        // this lane's share of the running sum
-  floatx4 oacc[ND];
-#pragma unroll
-  for (int db = 0; db < ND; ++db) oacc[db] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-  const int q_last = min(q0 + BM, S) - 1;
-  const int nkt = q_last / BN + 1;  // key tiles 0 .. nkt-1 (the rest are above the diagonal)
-  const int wq_last = qw + 15;
-
-  gload(0);
-  lstore(0);
-  __syncthreads();
-
-  for (int jt = 0; jt < nkt; ++jt) {
-    const int buf = jt & 1;
-    const int k0 = jt * BN;
-    if (jt + 1 < nkt) gload(k0 + BN);
-
-    // S^T = K . Q^T for this wavefront's 16 queries.
-    floatx4 sacc[NKB];
-#pragma unroll
-    for (int kb = 0; kb < NKB; ++kb) {
-      sacc[kb] = floatx4{0.f, 0.f, 0.f, 0.f};
-      if (k0 + 16 * kb <= wq_last) {
-#pragma unroll
-        for (int f = 0; f < NQF; ++f) {
-          const typename MF::frag a = load_frag(&Ks[buf][(16 * kb + r) * LDK + f * MF::MK + g * MF::KPER]);
-          sacc[kb] = MF::mma(a, qf[f], sacc[kb]);
-        }
-      }
-    }
-
-    // Online softmax.  Element i of sacc[kb] is key k0 + 16 kb + 4 g + i.
-    const bool diag = k0 + BN - 1 > qw;
-    float mloc = -INFINITY;
-#pragma unroll
-    for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float s = sacc[kb][i] * p.c;
-        if (diag && k0 + 16 * kb + 4 * g + i > myq) s = -INFINITY;
-        sacc[kb][i] = s;
-        mloc = fmaxf(mloc, s);
-      }
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 16, kWave));
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 32, kWave));
-    const float m_new = fmaxf(m_run, mloc);
-    const float corr = fast_exp2(m_run - m_new);
-    m_run = m_new;
-    float rsum = 0.f;
-#pragma unroll
-    for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float e = fast_exp2(sacc[kb][i] - m_new);
-        sacc[kb][i] = e;
-        rsum += e;
-      }
-    l_run = fmaf(l_run, corr, rsum);
-#pragma unroll
-    for (int db = 0; db < ND; ++db)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) oacc[db][i] *= corr;
-
-    // O^T += V^T . P^T
-    if constexpr (BF) {
-#pragma unroll
-      for (int t = 0; t < BN / 32; ++t) {
-        if (k0 + 32 * t > wq_last) continue;
-        bf16x8 pf;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          pf[i] = (bf16)sacc[2 * t][i];
-          pf[4 + i] = (bf16)sacc[2 * t + 1][i];
-        }
-#pragma unroll
-        for (int db = 0; db < ND; ++db) {
-          const bf16x8 a = load_frag(&Vs[buf][(16 * db + r) * LDV + 32 * t + 8 * g]);
-          oacc[db] = MF::mma(a, pf, oacc[db]);
-        }
-      }
-    } else {
-#pragma unroll
-      for (int kb = 0; kb < NKB; ++kb) {
-        if (k0 + 16 * kb > wq_last) continue;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int db = 0; db < ND; ++db) {
-            const float a = Vs[buf][(16 * kb + 4 * g + i) * LDK + 16 * db + r];
-            oacc[db] = MF::mma(a, sacc[kb][i], oacc[db]);
-          }
-      }
-    }
-
-    if (jt + 1 < nkt) lstore(buf ^ 1);
-    __syncthreads();
-  }
-
-  // Finish: l = sum over the four lane groups; O = O^T / l rounded once.
-  float l = l_run + __shfl_xor(l_run, 16, kWave);
-  l += __shfl_xor(l, 32, kWave);
-  const float linv = 1.0f / l;
-  if (myq < S) {
-    T* orow = O + (long)myq * p.o_ss;
-#pragma unroll
-    for (int db = 0; db < ND; ++db) {
-      const int dd = 16 * db + 4 * g;
-      if (dd < dlim) {
-        float ov[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ov[i] = oacc[db][i] * linv;
-        store_vec<4>(orow + dd, ov);
-      }
-    }
-  }
-}
 
 // ------------------------------------------------ naive (unfused) path --
 // nkilab/kernels/attention.py:35-89, pass 2: scores (already Q.K^T) are
@@ -311,22 +40,6 @@ __global__ __launch_bounds__(256) void masked_softmax_kernel(float* __restrict__
 }
 
 static bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
-
-template <int D>
-static void flash_f32_launch(const AttnArgs& a, hipStream_t st) {
-  const int nqb = (a.S + 63) / 64;
-  flash_fwd_kernel<float, D><<<dim3((unsigned)(nqb * a.H)), dim3(256), 0, st>>>(a);
-}
-
-static int flash_f32_dispatch(const AttnArgs& a, hipStream_t st) {
-  if (a.d <= 32)
-    flash_f32_launch<32>(a, st);
-  else if (a.d <= 64)
-    flash_f32_launch<64>(a, st);
-  else
-    flash_f32_launch<128>(a, st);
-  return check_launch("nkl_flash_attn_causal");
-}
 
 }  // namespace nkl
 
@@ -378,7 +91,7 @@ static int flash_entry(const char* fn, const void* q, const void* k, const void*
       return set_error(NKL_EWORKSPACE, "%s: null workspace", fn);
     return flash_bf16_launch(a, workspace, workspace_bytes, counters, counter_bytes, st);
   }
-  return flash_f32_dispatch(a, st);
+  return flash_f32_launch(a, st);
 }
 
 extern "C" int nkl_flash_attn_causal(const void* q, const void* k, const void* v, void* o, int H, int S, int d,

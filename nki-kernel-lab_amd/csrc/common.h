@@ -197,30 +197,6 @@ __device__ __forceinline__ float wave_sum(float v) {
 }
 
 // ------------------------------------------------------- MFMA operands --
-// A 16x16 (M x N) MFMA with K = 4 * KPER: lane l holds
-//   A[m = l % 16][k = KPER * (l / 16) + j], B[k = KPER * (l / 16) + j][n = l % 16]
-// for j < KPER, and the accumulator C[4 * (l / 16) + i][l % 16], i < 4.
-template <typename T>
-struct Mfma16;
-template <>
-struct Mfma16<bf16> {
-  static constexpr int KPER = 8;
-  static constexpr int MK = 32;
-  typedef bf16x8 frag;
-  static __device__ __forceinline__ floatx4 mma(frag a, frag b, floatx4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-  }
-};
-template <>
-struct Mfma16<float> {
-  static constexpr int KPER = 1;
-  static constexpr int MK = 4;
-  typedef float frag;
-  static __device__ __forceinline__ floatx4 mma(frag a, frag b, floatx4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-};
-
 // A 32x32 MFMA with K = 2 * KPER: lane l holds
 //   A[m = l % 32][k = KPER * (l / 32) + j], B[k = KPER * (l / 32) + j][n = l % 32]
 // and the accumulator C[8 * (i / 4) + 4 * (l / 32) + i % 4][l % 32], i < 16.

@@ -1,0 +1,326 @@
+// Causal flash attention in fp32: 16x16x4 fp32 MFMA, every sum, score and
+// probability in 32 bits.
+//
+// One 512-thread workgroup per 64-query block of a head (heaviest blocks
+// first: the dispatcher hands the light ones to the CUs that end early).  Its
+// eight wavefronts are 2 query groups x 4 key groups: wavefront (qg, kg) owns
+// queries 32 qg .. + 31 and keys 16 kg .. + 15 of every step of 64 keys, with a
+// running state (max, sum, O) of its own; the four key groups of a query group
+// are merged through LDS at the end.  Each SIMD so holds two wavefronts, one's
+// softmax beside the other's MFMAs, on a grid of twice the 128-query blocks.
+//
+// K and V rows are copied global -> LDS by the buffer unit, one step ahead,
+// into two stages.  Everything is computed transposed, so that a lane works on
+// two queries (halves h of its group) and nothing is shuffled between the
+// products:
+//     S^T = K . Q^T    a K fragment is one b128 read, 4 elements of d for four
+//                      MFMAs (lane group g supplies d = 16 ks + 4 g + j to MFMA
+//                      j) and both halves; Q^T is held in registers.
+//     O^T = V^T . P^T  MFMA i takes key 4 g + i from lane group g, which is
+//                      where S^T left its probability; a V fragment is one b128
+//                      read of a key's row, d = 4 r .. 4 r + 3 of lane r for
+//                      four 16-row blocks of O^T (row r of block b is d = 4 r +
+//                      b), so that a lane ends up with contiguous runs of O.
+// K rows are swizzled by 16-byte chunks (chunk c of row r at c ^ swz(r)), which
+// keeps the 16-row reads free of bank conflicts; V reads are whole rows.
+//
+// Bound by the fp32 MFMAs (256 flop per clock and CU; a step is 8192 cycles of
+// them per SIMD, 3.5 of its 4.5 us): 16 x 2048 x 128 281 -> 171 us (101 TFLOP/s),
+// 8/2 x 4096 x 128 551 -> 320, 4 x 300 x 64 24.5 -> 17.8, against 64-query
+// workgroups of four 16-query wavefronts that read one 4-byte operand per MFMA.
+// Of the rest, the copies take 0.3 us a step and the softmax, which the second
+// wavefront hides only in part, 0.3.
+#include <math.h>
+
+#include "attention.h"
+
+namespace nkl {
+
+namespace {
+
+constexpr int kQB = 64, kKB = 64;           // queries of a block, keys of a step
+constexpr unsigned kPastEnd = 0x80000000u;  // a buffer offset past every range: the lane reads zeros
+
+template <int D>
+__device__ __forceinline__ int k_swz(int row) {
+  return D == 32 ? (row >> 1) & 7 : row & 15;
+}
+
+__device__ __forceinline__ float max_xor16(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float sum_xor16(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+}  // namespace
+
+template <int D>
+__global__ __launch_bounds__(512) void flash_f32_kernel(AttnArgs p) {
+  constexpr int ROWB = D * 4, TILEB = kKB * ROWB, STAGEB = 2 * TILEB;  // K then V
+  constexpr int CPT = TILEB / 1024 / 8;                                // copies per wavefront and tile
+  constexpr int NKS = D / 16;                                          // K fragments (and 16-row blocks of O^T)
+  constexpr int NB = D >= 64 ? 4 : 2, NH = NKS / NB;                   // blocks per V read, V reads per key
+  __shared__ __align__(16) unsigned char lds[2 * STAGEB];
+  __shared__ float ml[8][2][16][2];  // (max, sum) per wavefront, half and query
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int qg = w & 1, kg = w >> 1;
+  const int g = lane >> 4, r = lane & 15;
+  const int S = p.S;
+
+  const int nqb = (S + kQB - 1) / kQB;
+  const int h = blockIdx.x % p.H;
+  const int q0 = (nqb - 1 - blockIdx.x / p.H) * kQB;
+  const int qw = q0 + 32 * qg;  // first query of this wavefront
+  const float* Q = static_cast<const float*>(p.q) + (long)h * p.q_sh;
+  const float* K = static_cast<const float*>(p.k) + (long)(h / p.group) * p.k_sh;  // shared K/V head (GQA)
+  const float* V = static_cast<const float*>(p.v) + (long)(h / p.group) * p.v_sh;
+  float* O = static_cast<float*>(p.o) + (long)h * p.o_sh;
+
+  // Copy u of this wavefront, 1024 bytes of a tile, lane l's 16 bytes at 16 l:
+  // u < CPT of a K tile, then of a V tile.
+  unsigned off[2 * CPT];
+  int crow[CPT];
+#pragma unroll
+  for (int u = 0; u < CPT; ++u) {
+    const int b = (w * CPT + u) * 1024 + lane * 16;
+    const int row = b / ROWB, pc = b % ROWB / 16, kc = pc ^ k_swz<D>(row);
+    crow[u] = row;
+    off[u] = 4 * kc < p.d ? (unsigned)(4 * ((long)row * p.k_ss + 4 * kc)) : kPastEnd;
+    off[CPT + u] = 4 * pc < p.d ? (unsigned)(4 * ((long)row * p.v_ss + 4 * pc)) : kPastEnd;
+  }
+  // K tiles at lds, V tiles after both of them.
+  auto copy1 = [&](bool isv, int src, int s, int u) __attribute__((always_inline)) {
+    const int k0 = src * kKB, rows = min(kKB, S - k0);
+    const long ss = isv ? p.v_ss : p.k_ss;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)((isv ? V : K) + (long)k0 * ss), (short)0, (int)(4 * ((rows - 1) * ss + p.d)), 0x00020000);
+    const unsigned dst = opaque_lds_addr(lds) + (isv ? 2 * TILEB : 0) + (s & 1) * TILEB + (w * CPT + u) * 1024;
+    const unsigned o = crow[u] < rows ? off[isv ? CPT + u : u] : kPastEnd;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, lds_ptr(dst), 16, (int)o, 0, 0, 0);
+  };
+  auto copy = [&](bool isv, int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < CPT; ++u) copy1(isv, s, s, u);
+  };
+  // Every wavefront's LDS reads are done (its copies still in flight).
+  auto lds_done_barrier = [&]() __attribute__((always_inline)) {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));  // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  };
+  // Every wavefront's copies have landed and its LDS accesses are done.
+  auto step_barrier = [&]() __attribute__((always_inline)) {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_s_barrier();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  };
+
+  const int ns = (min(q0 + kQB, S) - 1) / kKB + 1;  // steps up to the diagonal
+  copy(false, 0);
+  copy(true, 0);
+  if (ns > 1) copy(false, 1);
+  // Q^T: lane (r, g) holds Q[qw + 16 hf + r][16 ks + 4 g + j].
+  floatx4 qf[2][NKS];
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf) {
+    const int q = qw + 16 * hf + r;
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) {
+      const int d = 16 * ks + 4 * g;
+      qf[hf][ks] = floatx4{0.f, 0.f, 0.f, 0.f};
+      if (q < S && d < p.d) qf[hf][ks] = *reinterpret_cast<const floatx4*>(Q + (long)q * p.q_ss + d);
+    }
+  }
+
+  float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};  // l: this lane's share
+  floatx4 o[2][NKS];
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+    for (int b = 0; b < NKS; ++b) o[hf][b] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+  const int krow = 16 * kg + r;  // this lane's K row of a step
+  const int swz = k_swz<D>(krow);
+  // Whether any key of this wavefront's step s is at or before its last query.
+  auto active = [&](int s) __attribute__((always_inline)) { return s < ns && s * kKB + 16 * kg <= qw + 31; };
+  // Scores of step s: sc[hf][i] for key s kKB + 16 kg + 4 g + i, query qw + 16 hf + r.
+  auto qk = [&](int s, int ks, floatx4 (&sc)[2]) __attribute__((always_inline)) {
+    const floatx4 a =
+        *reinterpret_cast<const floatx4*>(lds + (s & 1) * TILEB + krow * ROWB + (((4 * ks + g) ^ swz) << 4));
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf)
+        sc[hf] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], qf[hf][ks][j], sc[hf], 0, 0, 0);
+  };
+  float mx[2];
+  // Element i of both halves: scale, causal mask, running maximum of the step.
+  auto mask_max = [&](int s, int i, floatx4 (&sc)[2]) __attribute__((always_inline)) {
+    const int key = s * kKB + 16 * kg + 4 * g + i;
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      const float x = key > qw + 16 * hf + r ? -INFINITY : sc[hf][i] * p.c;
+      sc[hf][i] = x;
+      mx[hf] = i == 0 ? x : fmaxf(mx[hf], x);
+    }
+  };
+  float mu[2];  // the maximum the step's exponents are taken against
+  // The step's maxima over the wavefront's keys; O and the sum follow when one grew.
+  auto raise_max = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      const float mn = fmaxf(m[hf], max_xor32(max_xor16(mx[hf])));
+      if (__any(mn > m[hf])) {
+        // (no key yet: m is -inf, l and O are 0)
+        const float corr = m[hf] == -INFINITY ? 0.f : fast_exp2(m[hf] - mn);
+        l[hf] *= corr;
+#pragma unroll
+        for (int b = 0; b < NKS; ++b) o[hf][b] *= corr;
+        m[hf] = mn;
+      }
+      mu[hf] = mn == -INFINITY ? 0.f : mn;  // every key masked so far: p = 0
+    }
+  };
+
+  // Pipeline over steps: the exponentials of step s beside the QK^T MFMAs of
+  // step s + 1, then mask and maximum of step s + 1 beside the PV MFMAs of
+  // step s.  K tile s + 2 and V tile s + 1 are copied meanwhile, into the
+  // tiles read last in step s - 1.
+  const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+  floatx4 sc[2] = {zero, zero};
+  step_barrier();
+  if (active(0)) {
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) qk(0, ks, sc);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) mask_max(0, i, sc);
+    raise_max();
+  }
+  lds_done_barrier();
+#pragma unroll 1
+  for (int s = 0; s < ns; ++s) {
+    const bool next = active(s + 1);
+    floatx4 nx[2] = {zero, zero};
+    if (active(s)) {
+      auto exps = [&](int x0, int x1) __attribute__((always_inline)) {
+#pragma unroll
+        for (int x = x0; x < x1; ++x) {
+          const int hf = x & 1, i = x >> 1;
+          sc[hf][i] = fast_exp2(sc[hf][i] - mu[hf]);
+          l[hf] += sc[hf][i];
+        }
+      };
+      // Copies of the next tiles, CPT of V tile s + 1 and of K tile s + 2 (the
+      // last one again when there is none): spread over the MFMAs, as each
+      // holds the wavefront's issue for a while.
+      const int k2 = min(s + 2, ns - 1);
+      if (next) {
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) {
+          qk(s + 1, ks, nx);
+          exps(8 * ks / NKS, 8 * (ks + 1) / NKS);
+#pragma unroll
+          for (int u = 2 * CPT * ks / NKS; u < 2 * CPT * (ks + 1) / NKS; ++u)
+            u < CPT ? copy1(true, s + 1, s + 1, u) : copy1(false, k2, s + 2, u - CPT);
+        }
+      } else {
+        exps(0, 8);
+        if (s + 1 < ns) copy(true, s + 1);  // (that step is the last one)
+      }
+      typedef float vfrag __attribute__((ext_vector_type(NB)));
+      vfrag va[2][NH];
+      auto vread = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < NH; ++n)
+          va[i & 1][n] = *reinterpret_cast<const vfrag*>(lds + 2 * TILEB + (s & 1) * TILEB +
+                                                         (16 * kg + 4 * g + i) * ROWB + 64 * NB * n + 4 * NB * r);
+      };
+      vread(0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (i < 3) vread(i + 1);
+        __builtin_amdgcn_sched_barrier(0);  // a key's fragments are read one key ahead
+#pragma unroll
+        for (int n = 0; n < NH; ++n)
+#pragma unroll
+          for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int hf = 0; hf < 2; ++hf)
+              o[hf][n * NB + b] =
+                  __builtin_amdgcn_mfma_f32_16x16x4f32(va[i & 1][n][b], sc[hf][i], o[hf][n * NB + b], 0, 0, 0);
+        mask_max(s + 1, i, nx);
+      }
+      if (next) raise_max();
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) sc[hf] = nx[hf];
+    }
+    step_barrier();
+  }
+
+  // Merge the four key groups: states through LDS, then wavefront kg finishes
+  // every fourth run of 4 NB values of d per lane.
+  floatx4* ob = reinterpret_cast<floatx4*>(lds);
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf) {
+    l[hf] = sum_xor32(sum_xor16(l[hf]));
+    if (g == 0) ml[w][hf][r][0] = m[hf], ml[w][hf][r][1] = l[hf];
+#pragma unroll
+    for (int b = 0; b < NKS; ++b) ob[(w * 2 * NKS + hf * NKS + b) * 64 + lane] = o[hf][b];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < 2 * NH; ++t) {
+    if (t % 4 != kg) continue;
+    const int hf = t / NH, n = t % NH;
+    float wt[4], M = -INFINITY, L = 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) M = fmaxf(M, ml[2 * k + qg][hf][r][0]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      wt[k] = fast_exp2(ml[2 * k + qg][hf][r][0] - M);
+      L = fmaf(wt[k], ml[2 * k + qg][hf][r][1], L);
+    }
+    const float linv = 1.0f / L;
+    floatx4 acc[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      acc[b] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        acc[b] += wt[k] * ob[((2 * k + qg) * 2 * NKS + hf * NKS + n * NB + b) * 64 + lane];
+    }
+    const int q = qw + 16 * hf + r;
+    if (q < S) {
+      float* orow = O + (long)q * p.o_ss;
+#pragma unroll
+      for (int e = 0; e < 4; e += 4 / NB) {
+        // Row 4 g + e of the blocks: d = 16 NB n + NB (4 g + e) + b.
+        const int d = 16 * NB * n + NB * (4 * g + e);
+        float v[4];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) v[x] = acc[x % NB][e + x / NB] * linv;
+        if (d < p.d) store_vec<4>(orow + d, v);
+      }
+    }
+  }
+}
+
+int flash_f32_launch(const AttnArgs& a, hipStream_t st) {
+  const dim3 grid((unsigned)(((a.S + kQB - 1) / kQB) * (long)a.H));
+  if (a.d <= 32)
+    flash_f32_kernel<32><<<grid, dim3(512), 0, st>>>(a);
+  else if (a.d <= 64)
+    flash_f32_kernel<64><<<grid, dim3(512), 0, st>>>(a);
+  else
+    flash_f32_kernel<128><<<grid, dim3(512), 0, st>>>(a);
+  return check_launch("nkl_flash_attn_causal");
+}
+
+}  // namespace nkl

@@ -490,3 +490,56 @@ def test_gqa_bf16_every_kernel_and_schedule(rng, flash_cfg, kernel, qb, schedule
     out = _np(ops.attention(q, k, v))
     kr, vr = (t.repeat_interleave(H // Hkv, dim=0) for t in (k, v))
     assert_bf16_attention(out, q, kr, vr, (kernel, qb, schedule))
+
+
+@pytest.mark.parametrize("H,Hkv,S,d,scale", [
+    (1, 1, 1, 4, None), (3, 1, 16, 32, None), (2, 2, 63, 36, None), (2, 1, 64, 64, -0.3), (1, 1, 65, 100, None),
+    (4, 4, 127, 64, 4.0), (2, 2, 128, 128, None), (1, 1, 129, 128, -0.1), (6, 2, 191, 96, None),
+    (2, 2, 321, 128, 3.0), (1, 1, 1027, 64, None)])
+def test_flash_fp32_against_float64(H, Hkv, S, d, scale):
+    """The fp32 kernel at the edges of its blocks (64 queries, 64 keys in four
+    groups of 16), of its head-dim variants (32, 64, 128, padded ones between)
+    and with grouped heads, steep and negative scales, on head-split views of
+    wider rows full of NaN: within 5e-6 of the largest value of a float64
+    softmax (64-bit scores against sums of up to 128 products in 32 bits: below
+    1e-6 of a score of at most 130, exponentiated)."""
+    from nkilab import ops
+
+    g = torch.Generator(device="cuda").manual_seed(S * 131 + d)
+
+    def heads(n):
+        buf = torch.full((S, n * d + 8), float("nan"), device="cuda")
+        x = buf[:, 4:4 + n * d]
+        x.copy_(torch.randn(S, n * d, generator=g, device="cuda"))
+        return x.view(S, n, d).transpose(0, 1)
+
+    q, k, v = heads(H), heads(Hkv), heads(Hkv)
+    ob = torch.full((H, S + 1, d), 7.0, device="cuda")
+    ops.attention_into(q, k, v, ob[:, :S], scale=scale)
+    kd, vd = (t.double().repeat_interleave(H // Hkv, 0) for t in (k, v))
+    s = torch.matmul(q.double(), kd.transpose(1, 2).contiguous()) * (d ** -0.5 if scale is None else scale)
+    s.masked_fill_(torch.ones(S, S, dtype=torch.bool, device="cuda").triu(1), -float("inf"))
+    ref = torch.matmul(torch.softmax(s, -1), vd)
+    tol = 5e-6 * max(1.0, s[s > -1e300].abs().max().item() / 10)
+    assert (ob[:, :S].double() - ref).abs().max().item() <= tol * ref.abs().max().item()
+    assert (ob[:, S] == 7).all()
+
+
+def test_flash_fp32_with_infinite_scores():
+    """A key whose score is -inf for every query gets no weight, a query that
+    sees nothing else is NaN, and NaN stays in the queries that see it."""
+    from nkilab import ops
+
+    S, d = 200, 64
+    q = torch.rand(1, S, d, device="cuda") + 0.1
+    k = torch.randn(1, S, d, device="cuda")
+    v = torch.randn(1, S, d, device="cuda")
+    k[0, 0] = -float("inf")
+    k[0, 70] = -float("inf")
+    k[0, 150] = float("nan")
+    o = ops.attention(q, k, v)
+    assert torch.isnan(o[0, 0]).all() and torch.isnan(o[0, 150:]).all()
+    s = torch.matmul(q.double(), k.double().transpose(1, 2).contiguous()) * d ** -0.5
+    s.masked_fill_(torch.ones(S, S, dtype=torch.bool, device="cuda").triu(1), -float("inf"))
+    ref = torch.matmul(torch.softmax(s[:, :150, :150], -1), v[:, :150].double())
+    assert (o[:, 1:150].double() - ref[:, 1:]).abs().max().item() <= 1e-5
