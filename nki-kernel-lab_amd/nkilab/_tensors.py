@@ -19,6 +19,8 @@ try:  # bfloat16 NumPy arrays exist only when ml_dtypes is installed
 except ImportError:  # pragma: no cover - depends on the environment
     NP_BF16 = None
 
+_DTYPE_CODES = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16, torch.float16: _lib.F16}
+
 NUMPY, TORCH_CPU, TORCH_GPU = "numpy", "torch_cpu", "torch_gpu"
 
 
@@ -31,19 +33,17 @@ def device() -> torch.device:
 def dtype_code(dt: torch.dtype) -> int:
     """The C ABI's dtype code (float16 is an operand format of the GEMM, the
     RMSNorm output, the gate/up SwiGLU GEMM and the flash attention only)."""
-    if dt == torch.float32:
-        return _lib.F32
-    if dt == torch.bfloat16:
-        return _lib.BF16
-    if dt == torch.float16:
-        return _lib.F16
+    code = _DTYPE_CODES.get(dt)
+    if code is not None:
+        return code
     raise TypeError(f"unsupported dtype {dt}: float32, bfloat16 or float16 expected")
 
 
 def to_device(x) -> tuple[torch.Tensor, str]:
     """Return (GPU tensor, kind of the input)."""
     if isinstance(x, torch.Tensor):
-        dtype_code(x.dtype)
+        if x.dtype not in _DTYPE_CODES:
+            dtype_code(x.dtype)  # raises
         if x.is_cuda:
             return x, TORCH_GPU
         return x.to(device()), TORCH_CPU
@@ -70,8 +70,20 @@ def from_device(t: torch.Tensor, kind: str):
     return t.cpu().numpy()
 
 
-def stream_handle() -> int:
+def _stream_handle_slow() -> int:
     return torch.cuda.current_stream().cuda_stream
+
+
+def _stream_handle_raw() -> int:
+    return _raw_stream(_get_device())
+
+
+# torch's current stream of the current device, as a hipStream_t.  The raw
+# query takes 0.2 us where building a torch.cuda.Stream object takes 2.8, a
+# quarter of a small op's host time.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_get_device = getattr(torch._C, "_cuda_getDevice", None)
+stream_handle = _stream_handle_raw if _raw_stream and _get_device else _stream_handle_slow
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

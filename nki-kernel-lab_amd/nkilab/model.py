@@ -138,6 +138,19 @@ _DTYPES = {"float32": torch.float32, "bfloat16": torch.bfloat16, "float16": torc
 SPLIT = "split"
 
 
+def _weight(block: nn.Module, name: str) -> torch.Tensor:
+    """getattr(block, name).weight, read from the modules' own tables where it
+    is an ordinary parameter (nn.Module.__getattr__ costs a microsecond a call)."""
+    m = block._modules.get(name)
+    p = m._parameters.get("weight") if m is not None else None
+    return p if p is not None else getattr(block, name).weight
+
+
+def _heads(t: torch.Tensor, col: int, n: int, hd: int) -> torch.Tensor:
+    """Columns col .. col + n hd of a row-major t [S, cols] as [n, S, hd] (a view)."""
+    return t.as_strided((n, t.shape[0], hd), (hd, t.stride(0), 1), t.storage_offset() + col)
+
+
 def _device_param(block: nn.Module, name: str, p: torch.Tensor, dtype: torch.dtype, dev: torch.device):
     """Device copy of a parameter in `dtype`, cached until the parameter changes."""
     cache = block.__dict__.setdefault("_nkl_param_cache", {})
@@ -156,12 +169,13 @@ def _packed_gate_up(block: DecoderBlock, dev: torch.device, dtype: torch.dtype =
     either weight changes."""
     cache = block.__dict__.setdefault("_nkl_param_cache", {})
     key = ("gate_up", dtype, dev)
-    stamp = tuple((p.data_ptr(), p._version) for p in (block.wg.weight, block.wu.weight))
+    pg, pu = _weight(block, "wg"), _weight(block, "wu")
+    stamp = (pg.data_ptr(), pg._version, pu.data_ptr(), pu._version)
     hit = cache.get(key)
     if hit is not None and hit[0] == stamp:
         return hit[1]
-    wg = block.wg.weight.detach().to(device=dev, dtype=dtype)
-    wu = block.wu.weight.detach().to(device=dev, dtype=dtype)
+    wg = pg.detach().to(device=dev, dtype=dtype)
+    wu = pu.detach().to(device=dev, dtype=dtype)
     t = ops.pack_gate_up(wg, wu)
     cache[key] = (stamp, t)
     return t
@@ -256,26 +270,27 @@ def nki_forward(block: DecoderBlock, x, attention_variant: str = "flash_pipeline
         raise ValueError("nki_forward: fp32 compute on a bf16 residual stream is not supported")
     if cdt == torch.float16 and rdt != torch.float32:
         raise ValueError("nki_forward: compute_dtype='float16' needs an fp32 x")
-    W = {n: _device_param(block, n, getattr(block, n).weight, cdt, dev) for n in ("wqkv", "wo", "wg", "wu", "wd")}
-    g1 = _device_param(block, "norm1", block.norm1.weight, rdt, dev)
-    g2 = _device_param(block, "norm2", block.norm2.weight, rdt, dev)
+
+    def weight(n):
+        return _device_param(block, n, _weight(block, n), cdt, dev)
+
+    g1 = _device_param(block, "norm1", _weight(block, "norm1"), rdt, dev)
+    g2 = _device_param(block, "norm2", _weight(block, "norm2"), rdt, dev)
 
     h = torch.empty((S, d), dtype=cdt, device=dev)
     ops.rmsnorm_into(xt, g1, h, cfg.eps)
     Hkv = cfg.kv_heads
     kvd = Hkv * hd
     qkv = torch.empty((S, d + 2 * kvd), dtype=cdt, device=dev)
-    ops.linear_into(h, W["wqkv"], qkv)
-    q = qkv[:, :d].view(S, H, hd).transpose(0, 1)
-    k = qkv[:, d:d + kvd].view(S, Hkv, hd).transpose(0, 1)
-    v = qkv[:, d + kvd:].view(S, Hkv, hd).transpose(0, 1)
+    ops.linear_into(h, weight("wqkv"), qkv)
+    q, k, v = _heads(qkv, 0, H, hd), _heads(qkv, d, Hkv, hd), _heads(qkv, d + kvd, Hkv, hd)
     if cfg.rope_base is not None:  # in place on the q and k columns of qkv
         ops.rope_into(q, q, cfg.rope_base)
         ops.rope_into(k, k, cfg.rope_base)
     a = torch.empty((S, d), dtype=cdt, device=dev)
-    ops.attention_into(q, k, v, a.view(S, H, hd).transpose(0, 1), variant=attention_variant)
+    ops.attention_into(q, k, v, _heads(a, 0, H, hd), variant=attention_variant)
     x1 = torch.empty((S, d), dtype=rdt, device=dev)
-    ops.linear_into(a, W["wo"], x1, residual=xt)
+    ops.linear_into(a, weight("wo"), x1, residual=xt)
     h2 = torch.empty((S, d), dtype=cdt, device=dev)
     ops.rmsnorm_into(x1, g2, h2, cfg.eps)
     act = torch.empty((S, cfg.d_ff), dtype=cdt, device=dev)
@@ -285,9 +300,9 @@ def nki_forward(block: DecoderBlock, x, attention_variant: str = "flash_pipeline
     else:
         gate = torch.empty((S, cfg.d_ff), dtype=cdt, device=dev)
         up = torch.empty((S, cfg.d_ff), dtype=cdt, device=dev)
-        ops.linear_into(h2, W["wg"], gate)
-        ops.linear_into(h2, W["wu"], up)
+        ops.linear_into(h2, weight("wg"), gate)
+        ops.linear_into(h2, weight("wu"), up)
         ops.swiglu_into(gate, up, act)
     out = torch.empty((S, d), dtype=rdt, device=dev)
-    ops.linear_into(act, W["wd"], out, residual=x1)
+    ops.linear_into(act, weight("wd"), out, residual=x1)
     return from_device(out, kind)

@@ -56,8 +56,10 @@ _MATMUL_VARIANTS = {"blocked": _lib.GEMM_BLOCKED, "naive": _lib.GEMM_NAIVE}
 
 def _row_major(t: torch.Tensor, cols: int) -> tuple[torch.Tensor, int]:
     """(tensor, leading dim) with unit column stride."""
-    if t.dim() == 2 and (t.stride(1) == 1 or t.shape[1] == 1) and t.stride(0) >= cols and t.shape[0] > 0:
-        return t, t.stride(0)
+    if t.dim() == 2:
+        ld, cs = t.stride()
+        if (cs == 1 or t.shape[1] == 1) and ld >= cols and t.shape[0] > 0:
+            return t, ld
     t = t.contiguous()
     return t, max(cols, 1)
 
@@ -69,20 +71,22 @@ def _gemm(a: torch.Tensor, bmat: torch.Tensor, ldb: int, b_trans: bool, c: torch
     if a.dim() != 2 or bmat.dim() != 2 or c.dim() != 2:
         raise ValueError(f"gemm: 2-D operands expected, got {tuple(a.shape)}, {tuple(bmat.shape)}, {tuple(c.shape)}")
     M, K = a.shape
-    N = c.shape[1]
-    if c.shape[0] != M:
+    Mc, N = c.shape
+    if Mc != M:
         raise ValueError(f"gemm: output {tuple(c.shape)} does not have the {M} rows of a {tuple(a.shape)}")
-    want_b = (N, K) if b_trans else (K, N)
-    if tuple(bmat.shape) != want_b:
+    if bmat.shape != ((N, K) if b_trans else (K, N)):
+        want_b = (N, K) if b_trans else (K, N)
         raise ValueError(f"gemm: b {tuple(bmat.shape)} does not match [{'N, K' if b_trans else 'K, N'}] = {want_b}")
-    if residual is not None and tuple(residual.shape) != (M, N):
+    if residual is not None and residual.shape != (M, N):
         raise ValueError(f"gemm: residual {tuple(residual.shape)} does not match the output [{M}, {N}]")
     if a.dtype != bmat.dtype:
         raise TypeError(f"gemm: a and b must share a dtype, got {a.dtype} and {bmat.dtype}")
     a, lda = _row_major(a, K)
-    if c.dim() != 2 or (c.stride(1) != 1 and N > 1) or (M > 1 and c.stride(0) < N):
+    ldc, cs = c.stride()
+    if (cs != 1 and N > 1) or (M > 1 and ldc < N):
         raise ValueError("gemm: the output must be a row-major [M, N] tensor")
-    ldc = c.stride(0) if M > 1 else max(N, 1)
+    if M <= 1:
+        ldc = max(N, 1)
     ldr = 0
     if residual is not None:
         residual, ldr = _row_major(residual, N)
@@ -91,20 +95,22 @@ def _gemm(a: torch.Tensor, bmat: torch.Tensor, ldb: int, b_trans: bool, c: torch
     if K == 0:
         c.copy_(residual if residual is not None else torch.zeros_like(c))
         return c
-    pa, pb, pc, pr, st = ptr(a), ptr(bmat), ptr(c), ptr(residual), stream_handle()
+    pa, pb, pc, st = a.data_ptr(), bmat.data_ptr(), c.data_ptr(), stream_handle()
+    pr = None if residual is None else residual.data_ptr()
     dt_in, dt_out, bt = dtype_code(a.dtype), dtype_code(c.dtype), int(b_trans)
     if _MATMUL_VARIANTS[variant] == _lib.GEMM_NAIVE:
         _lib.call("nkl_gemm", pa, pb, pc, pr, M, N, K, lda, ldb, ldc, ldr, bt, 1, 0, 0, 0, 0, dt_in, dt_out,
                   _lib.GEMM_NAIVE, st)
         return c
     # Most shapes need no workspace; the call says so before it launches anything.
-    rc = _lib.lib().nkl_gemm_ws(pa, pb, pc, pr, None, 0, M, N, K, lda, ldb, ldc, ldr, bt, dt_in, dt_out, st)
+    L = _lib.lib()
+    rc = L.nkl_gemm_ws(pa, pb, pc, pr, None, 0, M, N, K, lda, ldb, ldc, ldr, bt, dt_in, dt_out, st)
     if rc == _lib.EWORKSPACE:
-        nbytes = _lib.lib().nkl_gemm_workspace_bytes(pa, pb, M, N, K, lda, ldb, bt, dt_in, dt_out)
+        nbytes = L.nkl_gemm_workspace_bytes(pa, pb, M, N, K, lda, ldb, bt, dt_in, dt_out)
         ws = workspace(nbytes, c.device)
-        rc = _lib.lib().nkl_gemm_ws(pa, pb, pc, pr, ptr(ws), nbytes, M, N, K, lda, ldb, ldc, ldr, bt, dt_in, dt_out,
-                                    st)
-    _lib.check("nkl_gemm_ws", rc)
+        rc = L.nkl_gemm_ws(pa, pb, pc, pr, ws.data_ptr(), nbytes, M, N, K, lda, ldb, ldc, ldr, bt, dt_in, dt_out, st)
+    if rc:
+        _lib.check("nkl_gemm_ws", rc)
     return c
 
 
@@ -114,8 +120,9 @@ def gemm_into(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, residual: torch
     A b stored column-major (e.g. ``w.t()`` of a row-major [N, K] weight) is
     read in place by the B^T kernel; no transpose copy is made."""
     K, N = b.shape
-    if N > 1 and K > 1 and b.stride(0) == 1 and b.stride(1) >= K:
-        return _gemm(a, b.t(), b.stride(1), True, c, residual, variant)
+    s0, s1 = b.stride()
+    if s0 == 1 and N > 1 and K > 1 and s1 >= K:
+        return _gemm(a, b.t(), s1, True, c, residual, variant)
     bm, ldb = _row_major(b, N)
     return _gemm(a, bm, ldb, False, c, residual, variant)
 
@@ -179,7 +186,7 @@ def matmul(a, b, variant: str = "blocked"):
     tb, _ = to_device(b)
     if ta.dtype != tb.dtype:
         raise TypeError(f"matmul operands must share a dtype, got {ta.dtype} and {tb.dtype}")
-    c = torch.empty((M, N), dtype=ta.dtype, device=ta.device)
+    c = ta.new_empty((M, N))
     gemm_into(ta, tb, c, variant=variant)
     return from_device(c, kind)
 
@@ -236,10 +243,14 @@ def _as_rows(t: torch.Tensor) -> tuple[torch.Tensor, int, int, int]:
     """View t as [rows, cols] with unit column stride: (t2d, rows, cols, ld)."""
     cols = t.shape[-1] if t.dim() > 0 else 1
     t2 = t.reshape(-1, cols) if t.dim() != 2 else t
-    if t2.dim() != 2 or (t2.stride(1) != 1 and cols > 1) or t2.stride(0) < cols:
+    if t2.dim() != 2:
         t2 = t2.contiguous()
-    ld = t2.stride(0) if t2.shape[0] > 1 else max(cols, 1)
-    return t2, t2.shape[0], cols, max(ld, cols)
+    ld, cs = t2.stride()
+    if (cs != 1 and cols > 1) or ld < cols:
+        t2 = t2.contiguous()
+        ld = t2.stride(0)
+    rows = t2.shape[0]
+    return t2, rows, cols, max(ld, cols) if rows > 1 else max(cols, 1)
 
 
 def softmax_into(x: torch.Tensor, y: torch.Tensor, fused: bool = True) -> torch.Tensor:
@@ -249,12 +260,14 @@ def softmax_into(x: torch.Tensor, y: torch.Tensor, fused: bool = True) -> torch.
     y2, _, _, ldy = _as_rows(y)
     dt = dtype_code(x2.dtype)
     if fused:
-        _lib.call("nkl_softmax", ptr(x2), ptr(y2), R, D, ldx, ldy, dt, stream_handle())
+        rc = _lib.lib().nkl_softmax(x2.data_ptr(), y2.data_ptr(), R, D, ldx, ldy, dt, stream_handle())
+        if rc:
+            _lib.check("nkl_softmax", rc)
     else:
         nbytes = _lib.lib().nkl_softmax_unfused_workspace_bytes(R, D)
         ws = workspace(nbytes, x2.device)
         _lib.call("nkl_softmax_unfused", ptr(x2), ptr(y2), ptr(ws), nbytes, R, D, ldx, ldy, dt, stream_handle())
-    if y2.data_ptr() != y.data_ptr():
+    if y2 is not y and y2.data_ptr() != y.data_ptr():
         y.copy_(y2.view_as(y))
     return y
 
@@ -263,8 +276,7 @@ def softmax(x, fused: bool = True):
     """Row softmax over the last dim (ops.py:55-57).  fused=True: one HBM pass
     (norm.py:65); fused=False: three passes through HBM (norm.py:22)."""
     t, kind = to_device(x)
-    y = torch.empty(t.shape, dtype=t.dtype, device=t.device)
-    return from_device(softmax_into(t, y, fused=fused), kind)
+    return from_device(softmax_into(t, t.new_empty(t.shape), fused=fused), kind)
 
 
 def rmsnorm_into(x: torch.Tensor, weight: torch.Tensor, y: torch.Tensor, eps: float = 1e-6) -> torch.Tensor:
@@ -279,10 +291,11 @@ def rmsnorm_into(x: torch.Tensor, weight: torch.Tensor, y: torch.Tensor, eps: fl
         raise ValueError(f"rmsnorm_into: weight has {weight.numel()} elements, x rows have {D}")
     if y.stride(-1) != 1 or not y.is_contiguous():
         raise ValueError("rmsnorm_into: output must be contiguous")
-    y2 = y.view(R, D)
     w = weight.contiguous()
-    _lib.call("nkl_rmsnorm_ex", ptr(x2), ptr(w), ptr(y2), R, D, ldx, D, float(eps), dtype_code(x2.dtype),
-              dtype_code(w.dtype), dtype_code(y2.dtype), stream_handle())
+    rc = _lib.lib().nkl_rmsnorm_ex(x2.data_ptr(), w.data_ptr(), y.data_ptr(), R, D, ldx, D, float(eps),
+                                   dtype_code(x2.dtype), dtype_code(w.dtype), dtype_code(y.dtype), stream_handle())
+    if rc:
+        _lib.check("nkl_rmsnorm_ex", rc)
     return y
 
 
@@ -290,8 +303,7 @@ def rmsnorm(x, weight, eps: float = 1e-6):
     """y = x * rsqrt(mean(x^2, -1) + eps) * weight (ops.py:60-61)."""
     t, kind = to_device(x)
     w, _ = to_device(weight)
-    y = torch.empty(t.shape, dtype=t.dtype, device=t.device)
-    return from_device(rmsnorm_into(t, w, y, eps), kind)
+    return from_device(rmsnorm_into(t, w, t.new_empty(t.shape), eps), kind)
 
 
 def swiglu_into(gate: torch.Tensor, up: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
@@ -303,7 +315,10 @@ def swiglu_into(gate: torch.Tensor, up: torch.Tensor, y: torch.Tensor) -> torch.
     g, u = gate.contiguous(), up.contiguous()
     if not y.is_contiguous():
         raise ValueError("swiglu_into: output must be contiguous")
-    _lib.call("nkl_swiglu", ptr(g), ptr(u), ptr(y), g.numel(), dtype_code(g.dtype), stream_handle())
+    rc = _lib.lib().nkl_swiglu(g.data_ptr(), u.data_ptr(), y.data_ptr(), g.numel(), dtype_code(g.dtype),
+                               stream_handle())
+    if rc:
+        _lib.check("nkl_swiglu", rc)
     return y
 
 
@@ -315,8 +330,7 @@ def swiglu(gate, up):
         raise ValueError(f"swiglu: gate {tuple(g.shape)} and up {tuple(u.shape)} differ in shape")
     if g.dtype != u.dtype:
         raise TypeError(f"swiglu: gate and up must share a dtype, got {g.dtype} and {u.dtype}")
-    y = torch.empty(g.shape, dtype=g.dtype, device=g.device)
-    return from_device(swiglu_into(g, u, y), kind)
+    return from_device(swiglu_into(g, u, g.new_empty(g.shape)), kind)
 
 
 # ------------------------------------------------------------ attention --
@@ -353,8 +367,9 @@ _FLASH_SCRATCH: dict = {}
 _FLASH_RETIRED: list = []
 
 
-def _flash_scratch(ws_bytes: int, counter_bytes: int, dev: torch.device) -> tuple[torch.Tensor, torch.Tensor]:
-    key = (dev, stream_handle())
+def _flash_scratch(ws_bytes: int, counter_bytes: int, dev: torch.device,
+                   stream: int) -> tuple[torch.Tensor, torch.Tensor]:
+    key = (dev, stream)
     ws, cnt = _FLASH_SCRATCH.get(key, (None, None))
     if ws is None or ws.numel() < ws_bytes:
         if ws is not None:
@@ -374,8 +389,9 @@ ATTN_MAX_HEAD_STRIDE, ATTN_MAX_ROW_STRIDE = 1 << 24, 1 << 21
 
 
 def _attn_strides_ok(t: torch.Tensor, E: int) -> bool:
-    return (t.stride(2) == 1 and t.data_ptr() % 16 == 0 and t.stride(0) % E == 0 and t.stride(1) % E == 0
-            and 0 <= t.stride(0) <= ATTN_MAX_HEAD_STRIDE and 0 <= t.stride(1) <= ATTN_MAX_ROW_STRIDE)
+    sh, ss, sd = t.stride()
+    return (sd == 1 and t.data_ptr() % 16 == 0 and sh % E == 0 and ss % E == 0
+            and 0 <= sh <= ATTN_MAX_HEAD_STRIDE and 0 <= ss <= ATTN_MAX_ROW_STRIDE)
 
 
 def _attn_operand(t: torch.Tensor, E: int) -> torch.Tensor:
@@ -397,38 +413,36 @@ def attention_into(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.T
     if o.shape != q.shape or o.dtype != q.dtype or not (q.dtype == k.dtype == v.dtype):
         raise ValueError(f"attention_into: o {tuple(o.shape)} {o.dtype} must match q {tuple(q.shape)} {q.dtype}, "
                          "and k, v share q's dtype")
-    if scale is None:
-        scale = 1.0 / math.sqrt(d)
+    return _attention(q, k, v, o, spec, H, Hkv, S, d, 1.0 / math.sqrt(d) if scale is None else float(scale))
+
+
+def _attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor, spec: AttentionVariant, H: int,
+               Hkv: int, S: int, d: int, scale: float) -> torch.Tensor:
+    """attention_into on shapes and dtypes already checked."""
     E = 8 if q.element_size() == 2 else 4
     q, k, v = (_attn_operand(t, E) for t in (q, k, v))
     o_ok = _attn_strides_ok(o, E)
     out = o if o_ok else torch.empty((H, S, d), dtype=o.dtype, device=o.device)
-    strides = (q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
-               out.stride(0), out.stride(1))
+    strides = (*q.stride()[:2], *k.stride()[:2], *v.stride()[:2], *out.stride()[:2])
     dt = dtype_code(q.dtype)
     gqa = Hkv != H
     if spec.path == "flash":
-        nbytes = _lib.lib().nkl_flash_attn_causal_workspace_bytes(H, S, d, dt)
-        if gqa:
-            ws = cnt = None
-            if nbytes:
-                ws, cnt = _flash_scratch(nbytes, _lib.lib().nkl_flash_attn_causal_counter_bytes(H, S, dt), q.device)
-            _lib.call("nkl_flash_attn_causal_gqa", ptr(q), ptr(k), ptr(v), ptr(out), ptr(ws),
-                      ws.numel() if ws is not None else 0, ptr(cnt), cnt.numel() * 4 if cnt is not None else 0,
-                      H, Hkv, S, d, *strides, float(scale), dt, stream_handle())
-        elif nbytes:
-            ws, cnt = _flash_scratch(nbytes, _lib.lib().nkl_flash_attn_causal_counter_bytes(H, S, dt), q.device)
-            _lib.call("nkl_flash_attn_causal_ws", ptr(q), ptr(k), ptr(v), ptr(out), ptr(ws), ws.numel(), ptr(cnt),
-                      cnt.numel() * 4, H, S, d, *strides, float(scale), dt, stream_handle())
-        else:
-            _lib.call("nkl_flash_attn_causal", ptr(q), ptr(k), ptr(v), ptr(out), H, S, d, *strides, float(scale), dt,
-                      stream_handle())
+        L, st = _lib.lib(), stream_handle()
+        nbytes = L.nkl_flash_attn_causal_workspace_bytes(H, S, d, dt)
+        pw, wb, pc, cb = None, 0, None, 0
+        if nbytes:
+            ws, cnt = _flash_scratch(nbytes, L.nkl_flash_attn_causal_counter_bytes(H, S, dt), q.device, st)
+            pw, wb, pc, cb = ws.data_ptr(), ws.numel(), cnt.data_ptr(), cnt.numel() * 4
+        rc = L.nkl_flash_attn_causal_gqa(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), pw, wb, pc, cb,
+                                         H, Hkv, S, d, *strides, scale, dt, st)
+        if rc:
+            _lib.check("nkl_flash_attn_causal_gqa", rc)
     else:
         nbytes = _lib.lib().nkl_attention_naive_workspace_bytes(H, S, dt)
         ws = workspace(nbytes, q.device)
         if gqa:
             _lib.call("nkl_attention_naive_gqa", ptr(q), ptr(k), ptr(v), ptr(out), ptr(ws), nbytes, H, Hkv, S, d,
-                      *strides, float(scale), dt, stream_handle())
+                      *strides, scale, dt, stream_handle())
         else:
             _lib.call("nkl_attention_naive", ptr(q), ptr(k), ptr(v), ptr(out), ptr(ws), nbytes, H, S, d, *strides,
                       float(scale), dt, stream_handle())
@@ -465,8 +479,8 @@ def attention(q, k, v, variant: str = "flash_pipelined", scale: float | None = N
     dp = -(-d // E) * E
     if dp != d:
         tq, tk, tv = (torch.nn.functional.pad(t, (0, dp - d)) for t in (tq, tk, tv))
-    o = torch.empty((H, S, dp), dtype=tq.dtype, device=tq.device)
-    attention_into(tq, tk, tv, o, variant=spec.name, scale=1.0 / math.sqrt(d) if scale is None else float(scale))
+    o = tq.new_empty((H, S, dp))
+    _attention(tq, tk, tv, o, spec, H, tk.shape[0], S, dp, 1.0 / math.sqrt(d) if scale is None else float(scale))
     if dp != d:
         o = o[:, :, :d].contiguous()
     return from_device(o, kind)
