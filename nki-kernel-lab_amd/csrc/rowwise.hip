@@ -123,8 +123,14 @@ __device__ __forceinline__ float row_sum(float v, float* red) {
 // ------------------------------------------------------------- softmax --
 // nkilab/kernels/norm.py:65-89: neg_max = -max(x); e = exp(x + neg_max) with
 // the row sum in fp32; rinv = 1 / sum; y = e * rinv rounded once.
+// Wavefronts per SIMD the compiler makes room for: two 1024-thread workgroups a
+// CU where their rows' registers (32 values a lane) allow it (1000 x 20000 fp32
+// softmax 35.4 -> 30.3 us).  The unaligned form would spill (500 x 20001 17.1
+// -> 19.0).
+constexpr int row_waves(int wpr, int nv, int e, bool al) { return al && wpr == 16 && nv * e <= 32 ? 8 : 1; }
+
 template <typename T, int WPR, int NV, bool AL>
-__global__ __launch_bounds__(WPR == 1 ? 256 : 64 * WPR) void softmax_vec_kernel(const T* __restrict__ x,
+__global__ __launch_bounds__(WPR == 1 ? 256 : 64 * WPR, row_waves(WPR, NV, VecE<T>::value, AL)) void softmax_vec_kernel(const T* __restrict__ x,
                                                                                 T* __restrict__ y, int rows, int cols,
                                                                                 long ldx, long ldy) {
   constexpr int E = VecE<T>::value;
@@ -294,7 +300,7 @@ __device__ __forceinline__ void load_w(const bf16* p, float (&v)[E]) {
 }
 
 template <typename TI, typename TW, typename TO, int WPR, int NV, bool AL>
-__global__ __launch_bounds__(WPR == 1 ? 256 : 64 * WPR) void rmsnorm_vec_kernel(
+__global__ __launch_bounds__(WPR == 1 ? 256 : 64 * WPR, row_waves(WPR, NV, VecE<TI>::value, AL)) void rmsnorm_vec_kernel(
     const TI* __restrict__ x, const TW* __restrict__ w, TO* __restrict__ y, int rows, int cols, long ldx, long ldy,
     float inv_d, float eps) {
   constexpr int E = VecE<TI>::value;
@@ -427,8 +433,9 @@ static bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 // four: softmax 1536 x 2048 bf16 5.2 / 4.7, RMSNorm 5.2 / 4.3, 2048 x 2048
 // fp32 -> fp16 6.3 / 5.7; past one round one wavefront is level or ahead: 3000
 // x 2048 bf16 softmax 5.7 / 6.3).  Sixteen vectors a lane turn at `deep_rows`
-// (fp32 softmax 1024 x 4096 7.6 / 6.0 but 1536 x 4096 9.0 / 9.7), and in 16
-// bits, 128 values a lane, always go to four (4096 x 8192 26.0 / 22.1).
+// (fp32 softmax 1024 x 4096 7.6 / 6.0 but 1536 x 4096 9.0 / 9.7).  128 values a
+// lane (16 vectors in 16 bits) always go to four times the wavefronts (4096 x
+// 8192 26.0 / 22.1; four / sixteen: 1000 x 32768 33.5 / 27.7).
 struct RowPlan {
   int wpr, nv;
 };
@@ -440,8 +447,8 @@ static RowPlan pick_row(int rows, int cols, int deep_rows) {
     const int cap = wpr == 16 ? 64 / E : 16;
     for (int nv = 1; nv <= cap; nv *= 2) {
       if (nvec > nv * 64 * wpr) continue;
-      if (wpr == 1 && nv >= 4 && (rows <= (nv == 16 ? deep_rows : 2048) || nv * E > 64)) return RowPlan{4, nv / 4};
-      return RowPlan{wpr, nv};
+      const bool more = nv * E > 64 || (wpr == 1 && nv >= 4 && rows <= (nv == 16 ? deep_rows : 2048));
+      return more ? RowPlan{4 * wpr, nv / 4} : RowPlan{wpr, nv};
     }
   }
   return RowPlan{16, 0};
@@ -458,9 +465,9 @@ static bool with_row_plan(RowPlan p, F f) {
   }
   NKL_ROW(1, 1) NKL_ROW(1, 2) NKL_ROW(1, 4) NKL_ROW(1, 8)
   if constexpr (VecE<T>::value == 4) { NKL_ROW(1, 16) }
-  NKL_ROW(4, 1) NKL_ROW(4, 2) NKL_ROW(4, 4) NKL_ROW(4, 8) NKL_ROW(4, 16)
+  NKL_ROW(4, 1) NKL_ROW(4, 2) NKL_ROW(4, 4) NKL_ROW(4, 8)
+  if constexpr (VecE<T>::value == 4) { NKL_ROW(4, 16) NKL_ROW(16, 16) } else { NKL_ROW(16, 4) }
   NKL_ROW(16, 8)
-  if constexpr (VecE<T>::value == 4) { NKL_ROW(16, 16) }
 #undef NKL_ROW
   return false;
 }
