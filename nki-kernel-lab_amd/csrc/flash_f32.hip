@@ -1,10 +1,10 @@
 // Causal flash attention in fp32: 16x16x4 fp32 MFMA, every sum, score and
 // probability in 32 bits.
 //
-// One 512-thread workgroup per 64-query block of a head (heaviest blocks
-// first: the dispatcher hands the light ones to the CUs that end early).  Its
-// eight wavefronts are 2 query groups x 4 key groups: wavefront (qg, kg) owns
-// queries 32 qg .. + 31 and keys 16 kg .. + 15 of every step of 64 keys, with a
+// One 512-thread workgroup per 64-query block (32-query on small grids) of a
+// head, heaviest blocks first: the dispatcher hands the light ones to the CUs
+// that end early.  Its eight wavefronts are 2 query groups x 4 key groups:
+// wavefront (qg, kg) owns queries 32 qg .. + 31 (16 qg .. + 15) and keys 16 kg .. + 15 of every step of 64 keys, with a
 // running state (max, sum, O) of its own; the four key groups of a query group
 // are merged through LDS at the end.  Each SIMD so holds two wavefronts, one's
 // softmax beside the other's MFMAs, on a grid of twice the 128-query blocks.
@@ -26,7 +26,7 @@
 //
 // Bound by the fp32 MFMAs (256 flop per clock and CU; a step is 8192 cycles of
 // them per SIMD, 3.5 of its 4.5 us): 16 x 2048 x 128 281 -> 171 us (101 TFLOP/s),
-// 8/2 x 4096 x 128 551 -> 320, 4 x 300 x 64 24.5 -> 17.8, against 64-query
+// 8/2 x 4096 x 128 551 -> 320, 4 x 300 x 64 24.5 -> 10.9, against 64-query
 // workgroups of four 16-query wavefronts that read one 4-byte operand per MFMA.
 // Of the rest, the copies take 0.3 us a step and the softmax, which the second
 // wavefront hides only in part, 0.3.
@@ -38,7 +38,7 @@ namespace nkl {
 
 namespace {
 
-constexpr int kQB = 64, kKB = 64;           // queries of a block, keys of a step
+constexpr int kKB = 64;                     // keys of a step
 constexpr unsigned kPastEnd = 0x80000000u;  // a buffer offset past every range: the lane reads zeros
 
 template <int D>
@@ -57,14 +57,16 @@ __device__ __forceinline__ float sum_xor16(float x) {
 
 }  // namespace
 
-template <int D>
+// NHF: 16-query halves of a query group (2: 64-query blocks, 1: 32-query ones).
+template <int D, int NHF>
 __global__ __launch_bounds__(512) void flash_f32_kernel(AttnArgs p) {
+  constexpr int kQB = 32 * NHF;
   constexpr int ROWB = D * 4, TILEB = kKB * ROWB, STAGEB = 2 * TILEB;  // K then V
   constexpr int CPT = TILEB / 1024 / 8;                                // copies per wavefront and tile
   constexpr int NKS = D / 16;                                          // K fragments (and 16-row blocks of O^T)
   constexpr int NB = D >= 64 ? 4 : 2, NH = NKS / NB;                   // blocks per V read, V reads per key
   __shared__ __align__(16) unsigned char lds[2 * STAGEB];
-  __shared__ float ml[8][2][16][2];  // (max, sum) per wavefront, half and query
+  __shared__ float ml[8][NHF][16][2];  // (max, sum) per wavefront, half and query
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -75,7 +77,7 @@ __global__ __launch_bounds__(512) void flash_f32_kernel(AttnArgs p) {
   const int nqb = (S + kQB - 1) / kQB;
   const int h = blockIdx.x % p.H;
   const int q0 = (nqb - 1 - blockIdx.x / p.H) * kQB;
-  const int qw = q0 + 32 * qg;  // first query of this wavefront
+  const int qw = q0 + 16 * NHF * qg;  // first query of this wavefront
   const float* Q = static_cast<const float*>(p.q) + (long)h * p.q_sh;
   const float* K = static_cast<const float*>(p.k) + (long)(h / p.group) * p.k_sh;  // shared K/V head (GQA)
   const float* V = static_cast<const float*>(p.v) + (long)(h / p.group) * p.v_sh;
@@ -127,9 +129,9 @@ __global__ __launch_bounds__(512) void flash_f32_kernel(AttnArgs p) {
   copy(true, 0);
   if (ns > 1) copy(false, 1);
   // Q^T: lane (r, g) holds Q[qw + 16 hf + r][16 ks + 4 g + j].
-  floatx4 qf[2][NKS];
+  floatx4 qf[NHF][NKS];
 #pragma unroll
-  for (int hf = 0; hf < 2; ++hf) {
+  for (int hf = 0; hf < NHF; ++hf) {
     const int q = qw + 16 * hf + r;
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {
@@ -139,43 +141,45 @@ __global__ __launch_bounds__(512) void flash_f32_kernel(AttnArgs p) {
     }
   }
 
-  float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};  // l: this lane's share
-  floatx4 o[2][NKS];
+  float m[NHF], l[NHF];  // l: this lane's share
+  floatx4 o[NHF][NKS];
 #pragma unroll
-  for (int hf = 0; hf < 2; ++hf)
+  for (int hf = 0; hf < NHF; ++hf) {
+    m[hf] = -INFINITY, l[hf] = 0.f;
 #pragma unroll
     for (int b = 0; b < NKS; ++b) o[hf][b] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
 
   const int krow = 16 * kg + r;  // this lane's K row of a step
   const int swz = k_swz<D>(krow);
   // Whether any key of this wavefront's step s is at or before its last query.
-  auto active = [&](int s) __attribute__((always_inline)) { return s < ns && s * kKB + 16 * kg <= qw + 31; };
+  auto active = [&](int s) __attribute__((always_inline)) { return s < ns && s * kKB + 16 * kg < qw + 16 * NHF; };
   // Scores of step s: sc[hf][i] for key s kKB + 16 kg + 4 g + i, query qw + 16 hf + r.
-  auto qk = [&](int s, int ks, floatx4 (&sc)[2]) __attribute__((always_inline)) {
+  auto qk = [&](int s, int ks, floatx4 (&sc)[NHF]) __attribute__((always_inline)) {
     const floatx4 a =
         *reinterpret_cast<const floatx4*>(lds + (s & 1) * TILEB + krow * ROWB + (((4 * ks + g) ^ swz) << 4));
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int hf = 0; hf < 2; ++hf)
+      for (int hf = 0; hf < NHF; ++hf)
         sc[hf] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], qf[hf][ks][j], sc[hf], 0, 0, 0);
   };
-  float mx[2];
+  float mx[NHF];
   // Element i of both halves: scale, causal mask, running maximum of the step.
-  auto mask_max = [&](int s, int i, floatx4 (&sc)[2]) __attribute__((always_inline)) {
+  auto mask_max = [&](int s, int i, floatx4 (&sc)[NHF]) __attribute__((always_inline)) {
     const int key = s * kKB + 16 * kg + 4 * g + i;
 #pragma unroll
-    for (int hf = 0; hf < 2; ++hf) {
+    for (int hf = 0; hf < NHF; ++hf) {
       const float x = key > qw + 16 * hf + r ? -INFINITY : sc[hf][i] * p.c;
       sc[hf][i] = x;
       mx[hf] = i == 0 ? x : fmaxf(mx[hf], x);
     }
   };
-  float mu[2];  // the maximum the step's exponents are taken against
+  float mu[NHF];  // the maximum the step's exponents are taken against
   // The step's maxima over the wavefront's keys; O and the sum follow when one grew.
   auto raise_max = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int hf = 0; hf < 2; ++hf) {
+    for (int hf = 0; hf < NHF; ++hf) {
       const float mn = fmaxf(m[hf], max_xor32(max_xor16(mx[hf])));
       if (__any(mn > m[hf])) {
         // (no key yet: m is -inf, l and O are 0)
@@ -194,7 +198,9 @@ __global__ __launch_bounds__(512) void flash_f32_kernel(AttnArgs p) {
   // step s.  K tile s + 2 and V tile s + 1 are copied meanwhile, into the
   // tiles read last in step s - 1.
   const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
-  floatx4 sc[2] = {zero, zero};
+  floatx4 sc[NHF];
+#pragma unroll
+  for (int hf = 0; hf < NHF; ++hf) sc[hf] = zero;
   step_barrier();
   if (active(0)) {
 #pragma unroll
@@ -207,12 +213,14 @@ __global__ __launch_bounds__(512) void flash_f32_kernel(AttnArgs p) {
 #pragma unroll 1
   for (int s = 0; s < ns; ++s) {
     const bool next = active(s + 1);
-    floatx4 nx[2] = {zero, zero};
+    floatx4 nx[NHF];
+#pragma unroll
+    for (int hf = 0; hf < NHF; ++hf) nx[hf] = zero;
     if (active(s)) {
       auto exps = [&](int x0, int x1) __attribute__((always_inline)) {
 #pragma unroll
         for (int x = x0; x < x1; ++x) {
-          const int hf = x & 1, i = x >> 1;
+          const int hf = x % NHF, i = x / NHF;
           sc[hf][i] = fast_exp2(sc[hf][i] - mu[hf]);
           l[hf] += sc[hf][i];
         }
@@ -225,13 +233,13 @@ __global__ __launch_bounds__(512) void flash_f32_kernel(AttnArgs p) {
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) {
           qk(s + 1, ks, nx);
-          exps(8 * ks / NKS, 8 * (ks + 1) / NKS);
+          exps(4 * NHF * ks / NKS, 4 * NHF * (ks + 1) / NKS);
 #pragma unroll
           for (int u = 2 * CPT * ks / NKS; u < 2 * CPT * (ks + 1) / NKS; ++u)
             u < CPT ? copy1(true, s + 1, s + 1, u) : copy1(false, k2, s + 2, u - CPT);
         }
       } else {
-        exps(0, 8);
+        exps(0, 4 * NHF);
         if (s + 1 < ns) copy(true, s + 1);  // (that step is the last one)
       }
       typedef float vfrag __attribute__((ext_vector_type(NB)));
@@ -252,14 +260,14 @@ __global__ __launch_bounds__(512) void flash_f32_kernel(AttnArgs p) {
 #pragma unroll
           for (int b = 0; b < NB; ++b)
 #pragma unroll
-            for (int hf = 0; hf < 2; ++hf)
+            for (int hf = 0; hf < NHF; ++hf)
               o[hf][n * NB + b] =
                   __builtin_amdgcn_mfma_f32_16x16x4f32(va[i & 1][n][b], sc[hf][i], o[hf][n * NB + b], 0, 0, 0);
         mask_max(s + 1, i, nx);
       }
       if (next) raise_max();
 #pragma unroll
-      for (int hf = 0; hf < 2; ++hf) sc[hf] = nx[hf];
+      for (int hf = 0; hf < NHF; ++hf) sc[hf] = nx[hf];
     }
     step_barrier();
   }
@@ -268,15 +276,15 @@ __global__ __launch_bounds__(512) void flash_f32_kernel(AttnArgs p) {
   // every fourth run of 4 NB values of d per lane.
   floatx4* ob = reinterpret_cast<floatx4*>(lds);
 #pragma unroll
-  for (int hf = 0; hf < 2; ++hf) {
+  for (int hf = 0; hf < NHF; ++hf) {
     l[hf] = sum_xor32(sum_xor16(l[hf]));
     if (g == 0) ml[w][hf][r][0] = m[hf], ml[w][hf][r][1] = l[hf];
 #pragma unroll
-    for (int b = 0; b < NKS; ++b) ob[(w * 2 * NKS + hf * NKS + b) * 64 + lane] = o[hf][b];
+    for (int b = 0; b < NKS; ++b) ob[(w * NHF * NKS + hf * NKS + b) * 64 + lane] = o[hf][b];
   }
   __syncthreads();
 #pragma unroll
-  for (int t = 0; t < 2 * NH; ++t) {
+  for (int t = 0; t < NHF * NH; ++t) {
     if (t % 4 != kg) continue;
     const int hf = t / NH, n = t % NH;
     float wt[4], M = -INFINITY, L = 0.f;
@@ -294,7 +302,7 @@ __global__ __launch_bounds__(512) void flash_f32_kernel(AttnArgs p) {
       acc[b] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int k = 0; k < 4; ++k)
-        acc[b] += wt[k] * ob[((2 * k + qg) * 2 * NKS + hf * NKS + n * NB + b) * 64 + lane];
+        acc[b] += wt[k] * ob[((2 * k + qg) * NHF * NKS + hf * NKS + n * NB + b) * 64 + lane];
     }
     const int q = qw + 16 * hf + r;
     if (q < S) {
@@ -312,14 +320,25 @@ __global__ __launch_bounds__(512) void flash_f32_kernel(AttnArgs p) {
   }
 }
 
-int flash_f32_launch(const AttnArgs& a, hipStream_t st) {
-  const dim3 grid((unsigned)(((a.S + kQB - 1) / kQB) * (long)a.H));
-  if (a.d <= 32)
-    flash_f32_kernel<32><<<grid, dim3(512), 0, st>>>(a);
-  else if (a.d <= 64)
-    flash_f32_kernel<64><<<grid, dim3(512), 0, st>>>(a);
+template <int D>
+static void launch(const AttnArgs& a, hipStream_t st) {
+  // 32-query blocks where 64-query ones leave half the CUs idle: half the MFMAs
+  // of a step per workgroup (us, 64 / 32: 4 x 300 x 64 17.8 / 10.9, 1 x 4096 x
+  // 128 290 / 161, 2 x 100 x 128 15.7 / 9.5).
+  const long n64 = (a.S + 63) / 64, n32 = (a.S + 31) / 32;
+  if (n64 * a.H <= 128)
+    flash_f32_kernel<D, 1><<<dim3((unsigned)(n32 * a.H)), dim3(512), 0, st>>>(a);
   else
-    flash_f32_kernel<128><<<grid, dim3(512), 0, st>>>(a);
+    flash_f32_kernel<D, 2><<<dim3((unsigned)(n64 * a.H)), dim3(512), 0, st>>>(a);
+}
+
+int flash_f32_launch(const AttnArgs& a, hipStream_t st) {
+  if (a.d <= 32)
+    launch<32>(a, st);
+  else if (a.d <= 64)
+    launch<64>(a, st);
+  else
+    launch<128>(a, st);
   return check_launch("nkl_flash_attn_causal");
 }
 

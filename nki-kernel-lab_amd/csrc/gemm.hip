@@ -139,7 +139,7 @@ typedef u32x4_t u32x4_al4 __attribute__((aligned(4)));
 // elements of K for four 32x32x2 MFMAs (lane group lg supplies k = 4 lg + j to
 // MFMA j, the same order in A and B), and B as [K, N] stays row-major in LDS
 // and is read 4 bytes at a time.  Its MFMAs take 64 cycles each, so the loop is
-// bound by them: 2048^3 222 -> 131 us (B^T; [K, N] 141) against 111 us of MFMA
+// bound by them: 2048^3 222 -> 131 us (B^T; [K, N] 133) against 111 us of MFMA
 // time, 128x128 tiles in two K groups; a 64 x 64 wavefront tile without the
 // copies, or without the fragment reads, takes 125 and 128.  The register-staged
 // kernel takes 150 to 160 there.
