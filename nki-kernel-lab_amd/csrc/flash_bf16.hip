@@ -1444,6 +1444,39 @@ Work plan(int H, int S, Config cfg) {
 // needs no partial states.
 // The overrides above replace the choice (tests, tuning); the
 // one-wavefront-per-SIMD kernels and kFwd take 64 < d <= 128 and fix the block.
+
+// The choice for d <= 64, whose tiles are short next to a workgroup's start,
+// hand-over and merge: 64-query blocks throughout, and no schedule that splits
+// a block once a round of workgroups is full.  Sweep over 1 to 64 heads x 64 to
+// 8192 positions, inputs rotated through twice the last-level cache, us at
+// d = 64 (d = 32), this rule / the 128-query rule above:
+//   up to 384 positions, or more than 640 blocks, or more than a round of
+//   blocks up to 1024 positions: one four-wavefront workgroup per block, two
+//   or more a CU, whose starts and ends hide each other's: 8 x 128 5.8 / 6.6
+//   (5.4 / 6.1), 4 x 300 7.9 / 8.3, 64 x 300 8.6 / 16.2 (7.6 / 14.6), 32 x 768
+//   13.2 / 17.0, 32 x 1024 16.5 / 17.9, 32 x 1537 24.6 / 33.9 (19.1 / 30.6),
+//   32 x 2048 33.6 / 38.3 (24.7 / 34.6), 16 x 4096 56 / 63 (42 / 58),
+//   32 x 4096 105 / 119 (74 / 113);
+//   other launches of more than a round: eight wavefronts per block, 8 x 3000
+//   25.9 / 29.0, 16 x 1537 20.6 / 22.5 (16.0 / 20.3); per pair of blocks when
+//   the pairs fill the CUs (d > 32), 16 x 2048 23.7 / 24.8, 8 x 4096 36.9 /
+//   37.7, where blocks take 26.4 and 40 (at d = 32 blocks lead, 19.4 / 22.7);
+//   within a round: eight wavefronts per block while the heaviest block
+//   exceeds a balanced range by at most 18 tiles, as in the rule above, else
+//   balanced ranges, 8 x 2048 17.4 / 19.0, 4 x 4096 24.5 / 25.4.
+Config choose_narrow(int H, int S, int d) {
+  const long cus = cu_count();
+  const long n64 = ((long)S + 63) / 64, blocks = (long)H * n64;
+  if (S <= 384 || blocks > cus * 5 / 2 || (blocks > cus && S <= 1024)) return Config{64, kBlock, kTeams4};
+  if (blocks > cus) {
+    const long pairs = (long)H * ((n64 + 1) / 2);
+    return Config{64, d > 32 && pairs <= cus && pairs * 5 >= cus * 4 ? kPairs : kBlock, kTeams};
+  }
+  const long units = (long)H * (n64 * (n64 - 1) + (S - 1) / BN + 1);
+  const long range = units / cus > kMinUnits ? units / cus : kMinUnits;
+  return Config{64, (S - 1) / BN + 1 <= range + 18 ? kBlock : kBalanced, kTeams};
+}
+
 Config choose(int H, int S, int d, bool f16) {
   const long cus = cu_count();
   const long nqb = (S + 127) / 128;
@@ -1497,6 +1530,7 @@ Config choose(int H, int S, int d, bool f16) {
   const bool tiny_fits = (long)H * nqb <= cus || units128 < kMinUnits * cus || S <= 64;
   if (d > 64 && d <= 128 && (S <= kTinyAutoS || (S <= kTinyMaxS && cfg.qb == 64)) && tiny_fits)
     cfg = Config{128, kBlock, kTiny};
+  if (d <= 64) cfg = choose_narrow(H, S, d);
   const Overrides& ov = overrides();
   if (ov.sched >= 0) cfg.sched = ov.sched;
   if (ov.qb >= 0) cfg.qb = ov.qb;
