@@ -127,6 +127,17 @@ int nkl_gemm_swiglu(const void* A, const void* Bgu, void* C, int M, int N,
                     void* stream);
 
 /*
+ * C = silu(A . Wg^T) * (A . Wu^T) in fp32, the two weights where they are: the
+ * gate and up GEMMs and the SwiGLU kernel in one launch.
+ *   A: [M, K] (lda >= K); Wg, Wu: [N, K] (ldg, ldu >= K); C: [M, N] (ldc >= N).
+ * dtype must be F32; pointers 16-byte aligned; N, K and the leading dimensions
+ * multiples of 4; operands under 2 GiB.
+ */
+int nkl_gemm_gate_up(const void* A, const void* Wg, const void* Wu, void* C,
+                     int M, int N, int K, long lda, long ldg, long ldu,
+                     long ldc, int dtype, void* stream);
+
+/*
  * The reference's PSUM block check (nkilab/kernels/matmul.py:58): returns
  * NKL_OK when a BM x BN block of fp32 accumulator tiles fits the 8-tile
  * budget, NKL_ELIMIT (with a message naming PSUM) otherwise.  Used by the

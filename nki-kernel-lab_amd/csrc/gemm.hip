@@ -38,6 +38,8 @@ struct GemmArgs {
   int Nc;   // columns stored: N, or fewer when packed operands pad N
   int Kall; // 0, or the whole K of a product split over the batch index: entry z takes K columns from z K
   int padded;  // rows along K hold zeros up to a multiple of 16 bytes past K
+  const void* B2;  // GU kernels: the up weight (B the gate weight; N their 32-row groups taken in turn)
+  long ldb2;
 };
 
 // Workgroup tile index -> (tile_m, tile_n).  Consecutive workgroup ids are
@@ -173,8 +175,12 @@ constexpr unsigned kOOB = 0x80000000u;  // a buffer offset past every range: the
 
 }  // namespace
 
-template <typename TI, typename TO, int BM, int BN, bool BT, int NS, int WGM = 2, int WGN = 2, int KG = 1>
+template <typename TI, typename TO, int BM, int BN, bool BT, int NS, int WGM = 2, int WGN = 2, int KG = 1,
+          bool GU = false>
 __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_dma_kernel(GemmArgs p) {
+  // GU: gate and up weights as two tensors (B, B2: [Nc, K] each); tile columns
+  // 64 j .. 64 j + 31 are rows 32 j .. of B, the next 32 those of B2, so that
+  // the SwiGLU epilogue finds each pair in adjacent accumulator tiles.
   // TI: the operand format (bf16, fp16 or fp32); operands move as raw 16-byte
   // chunks, the format only picks the MFMA.
   // KG > 1: KG groups of WGM x WGN wavefronts share the tile; group g takes
@@ -233,9 +239,30 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_dma_kernel(GemmArgs 
     aoff[u] = row < rows_a ? (unsigned)(SZ * ((long)row * p.lda + E * lc)) : kOOB;
   }
   __amdgpu_buffer_rsrc_t rb;
+  __amdgpu_buffer_rsrc_t rb2;  // GU: the up weight
   unsigned boff[B_PW];
-  int bkc[B_PW], brow[B_PW];
-  if constexpr (BT) {
+  int bkc[B_PW], brow[B_PW], bq[B_PW];  // (bq: the instruction's 1024 bytes of the tile)
+  if constexpr (GU) {
+    // Even copies take gate rows, odd ones up rows: the resource is a
+    // compile-time choice.  Instruction q covers 8 rows of one 32-row group.
+    static_assert(BT && B_PW % 2 == 0 && TN % 2 == 0, "gate/up pairs");
+    const int w0 = n0 / 2, rows_b = min(BN / 2, p.Nc - w0);
+    rb = __builtin_amdgcn_make_buffer_rsrc((void*)(B + (long)w0 * p.ldb), (short)0,
+                                           (int)min((long)SZ * ((rows_b - 1) * p.ldb + Kr), 0x7fffffffL), 0x00020000);
+    rb2 = __builtin_amdgcn_make_buffer_rsrc((void*)(static_cast<const TI*>(p.B2) + (long)w0 * p.ldb2), (short)0,
+                                            (int)min((long)SZ * ((rows_b - 1) * p.ldb2 + Kr), 0x7fffffffL), 0x00020000);
+#pragma unroll
+    for (int u = 0; u < B_PW; ++u) {
+      const int i = wid * (B_PW / 2) + u / 2;  // eighth rows of the weight this copy takes
+      const int q = (i / 4) * 8 + i % 4 + 4 * (u & 1);
+      const int row = 8 * q + dr, wrow = 8 * i + dr;
+      const int lc = dpc ^ g_swz(row);
+      bq[u] = q;
+      bkc[u] = E * lc;
+      brow[u] = 0;
+      boff[u] = wrow < rows_b ? (unsigned)(SZ * ((long)wrow * (u & 1 ? p.ldb2 : p.ldb) + E * lc)) : kOOB;
+    }
+  } else if constexpr (BT) {
     const int rows_b = min(BN, p.N - n0);
     rb = __builtin_amdgcn_make_buffer_rsrc((void*)(B + (long)n0 * p.ldb), (short)0,
                                            (int)min((long)SZ * ((rows_b - 1) * p.ldb + Kr), 0x7fffffffL), 0x00020000);
@@ -243,6 +270,7 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_dma_kernel(GemmArgs 
     for (int u = 0; u < B_PW; ++u) {
       const int row = 8 * (wid * B_PW + u) + dr;
       const int lc = dpc ^ g_swz(row);
+      bq[u] = wid * B_PW + u;
       bkc[u] = E * lc;
       brow[u] = 0;
       boff[u] = row < rows_b ? (unsigned)(SZ * ((long)row * p.ldb + E * lc)) : kOOB;
@@ -258,6 +286,7 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_dma_kernel(GemmArgs 
       const int q = wid * B_PW + u;
       const int sub = q / 8, row = F32 ? (256 * q + 4 * lane) / BN : 8 * (q % 8) + dr;
       const int col = F32 ? (256 * q + 4 * lane) % BN : 64 * sub + 8 * (dpc ^ g_swz(row));
+      bq[u] = q;
       brow[u] = row;
       bkc[u] = 0;
       boff[u] = col < cols_b ? (unsigned)(SZ * ((long)row * p.ldb + col)) : kOOB;
@@ -280,8 +309,8 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_dma_kernel(GemmArgs 
       else
         off = (boff[w] != kOOB && k0 + brow[w] < K) ? boff[w] + (unsigned)((long)SZ * k0 * p.ldb) : kOOB;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rb, (__attribute__((address_space(3))) void*)(sb + A_BYTES + (wid * B_PW + w) * 1024), 16, (int)off, 0, 0,
-          0);
+          GU && (w & 1) ? rb2 : rb, (__attribute__((address_space(3))) void*)(sb + A_BYTES + bq[w] * 1024), 16,
+          (int)off, 0, 0, 0);
     }
   };
   auto dma = [&](int s, int st) __attribute__((always_inline)) {
@@ -517,7 +546,7 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_dma_kernel(GemmArgs 
     const int wc = sw ? WN / 2 : WN;
     // Rows of the block go to rows m0 + wm WM ..; columns to c0 ...
     const int c0 = sw ? (n0 + wn * WN) / 2 : n0 + wn * WN;
-    const int ncols = sw ? p.N / 2 : p.Nc;
+    const int ncols = sw && !GU ? p.N / 2 : p.Nc;
     const int cpr = wc / OE;  // 16-byte chunks per staged row
 #pragma unroll
     for (int ip = 0; ip < TM / TP; ++ip) {
@@ -1091,6 +1120,29 @@ static void launch_f32(int t, const GemmArgs& g, int batch, hipStream_t st) {
   }
 }
 
+// The gate/up GEMM with SwiGLU in fp32 (nkl_gemm_gate_up): the tiles whose
+// wavefronts own 64 columns, by the rule of choose_f32_tile over both weights'
+// columns.  Bound by the fp32 MFMAs as the plain fp32 GEMM is; it saves two
+// launches and the passes over gate and up: two GEMMs and the SwiGLU kernel took
+// 17.1 us at 300 x 1024 x K 256, this 9.0; 16 x 768 x 256 16.6 -> 6.7, 1000 x
+// 2048 x 512 52 -> 37, 2048 x 3072 x 1024 235 -> 199, 2048 x 6144 x 2048 793 ->
+// 764.  The error against 64 bits is the same.
+static void launch_f32_gate_up(const GemmArgs& g, hipStream_t st) {
+  auto grid = [&](int bm, int bn) { return dim3((unsigned)tiles_of(g, bm, bn, 1)); };
+  auto rounds = [&](int bm, int bn) { return (double)((tiles_of(g, bm, bn, 1) + 255) / 256); };
+  if (tiles_of(g, 32, 64, 1) <= 256) {
+    gemm_dma_kernel<float, float, 32, 64, true, 3, 1, 1, 4, true><<<grid(32, 64), dim3(256), 0, st>>>(g);
+    return;
+  }
+  const double c64 = 0.69 * rounds(64, 64), c64x128 = 1.2 * rounds(64, 128), c128 = 2.0 * rounds(128, 128);
+  if (c128 <= c64x128 && c128 <= c64)
+    gemm_dma_kernel<float, float, 128, 128, true, 2, 2, 2, 2, true><<<grid(128, 128), dim3(512), 0, st>>>(g);
+  else if (c64x128 < c64)
+    gemm_dma_kernel<float, float, 64, 128, true, 3, 2, 2, 2, true><<<grid(64, 128), dim3(512), 0, st>>>(g);
+  else
+    gemm_dma_kernel<float, float, 64, 64, true, 2, 2, 1, 4, true><<<grid(64, 64), dim3(512), 0, st>>>(g);
+}
+
 // The LDS-DMA kernel takes 16-byte chunks at 32-bit buffer offsets.
 template <typename T, bool BT>
 static bool dma_ok(const GemmArgs& a) {
@@ -1385,6 +1437,28 @@ extern "C" int nkl_gemm_swiglu(const void* A, const void* Bgu, void* C, int M, i
   else
     launch_dma_cols<bf16, bf16, true>(t, a, 1, true, st);
   return check_launch("nkl_gemm_swiglu");
+}
+
+extern "C" int nkl_gemm_gate_up(const void* A, const void* Wg, const void* Wu, void* C, int M, int N, int K, long lda,
+                                long ldg, long ldu, long ldc, int dtype, void* stream) {
+  if (M < 0 || N < 0 || K < 0)
+    return set_error(NKL_EINVAL, "nkl_gemm_gate_up: negative shape M=%d N=%d K=%d", M, N, K);
+  if (dtype != NKL_F32) return set_error(NKL_EDTYPE, "nkl_gemm_gate_up: only fp32 is supported (dtype %d)", dtype);
+  if (M == 0 || N == 0) return NKL_OK;
+  if (!A || !Wg || !Wu || !C) return set_error(NKL_EINVAL, "nkl_gemm_gate_up: null operand pointer");
+  if (lda < K || ldg < K || ldu < K || ldc < N)
+    return set_error(NKL_EINVAL, "nkl_gemm_gate_up: leading dimension too small (lda=%ld ldg=%ld ldu=%ld ldc=%ld)", lda,
+                     ldg, ldu, ldc);
+  if (!aligned16(A) || !aligned16(Wg) || !aligned16(Wu) || !aligned16(C) || N % 4 || K % 4 || lda % 4 || ldg % 4 ||
+      ldu % 4 || ldc % 4)
+    return set_error(NKL_EINVAL, "nkl_gemm_gate_up: operands must be 16-byte aligned with N, K and leading dimensions "
+                     "multiples of 4");
+  const long lim = (1L << 31) / 4;
+  if ((M - 1) * lda + K >= lim || (N - 1) * ldg + K >= lim || (N - 1) * ldu + K >= lim || N > (1 << 29))
+    return set_error(NKL_EINVAL, "nkl_gemm_gate_up: operands must be under 2 GiB");
+  GemmArgs a{A, Wg, C, nullptr, M, 2 * ((N + 31) / 32 * 32), K, lda, ldg, ldc, 0, 0, 0, 0, 0, kEpiSwiglu, N, 0, 0, Wu, ldu};
+  launch_f32_gate_up(a, (hipStream_t)stream);
+  return check_launch("nkl_gemm_gate_up");
 }
 
 extern "C" int nkl_check_blocks(int BM, int BN) {

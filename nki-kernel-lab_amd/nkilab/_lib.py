@@ -13,7 +13,7 @@ LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
 
 F32, BF16, F16 = 0, 1, 2
 GEMM_BLOCKED, GEMM_NAIVE = 0, 1
-EWORKSPACE = -4
+EINVAL, EWORKSPACE = -1, -4
 ABI_VERSION = 1
 
 _c_int, _c_long, _c_float, _c_size = ctypes.c_int, ctypes.c_long, ctypes.c_float, ctypes.c_size_t
@@ -29,6 +29,8 @@ SIGNATURES = {
     "nkl_gemm_ws": (_c_int, [_vp, _vp, _vp, _vp, _vp, _c_size, _c_int, _c_int, _c_int, _c_long, _c_long, _c_long,
                              _c_long, _c_int, _c_int, _c_int, _vp]),
     "nkl_gemm_swiglu": (_c_int, [_vp, _vp, _vp, _c_int, _c_int, _c_int, _c_long, _c_long, _c_long, _c_int, _vp]),
+    "nkl_gemm_gate_up": (_c_int, [_vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _c_long, _c_long, _c_long, _c_long, _c_int,
+                                  _vp]),
     "nkl_check_blocks": (_c_int, [_c_int, _c_int]),
     "nkl_softmax": (_c_int, [_vp, _vp, _c_int, _c_int, _c_long, _c_long, _c_int, _vp]),
     "nkl_softmax_unfused_workspace_bytes": (_c_size, [_c_int, _c_int]),

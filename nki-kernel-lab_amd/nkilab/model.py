@@ -298,11 +298,7 @@ def nki_forward(block: DecoderBlock, x, attention_variant: str = "flash_pipeline
         # gate, up and SwiGLU in one GEMM over the packed weight (same values)
         ops.gemm_swiglu_into(h2, _packed_gate_up(block, dev, cdt), act)
     else:
-        gate = torch.empty((S, cfg.d_ff), dtype=cdt, device=dev)
-        up = torch.empty((S, cfg.d_ff), dtype=cdt, device=dev)
-        ops.linear_into(h2, weight("wg"), gate)
-        ops.linear_into(h2, weight("wu"), up)
-        ops.swiglu_into(gate, up, act)
+        ops.gate_up_into(h2, weight("wg"), weight("wu"), act)
     out = torch.empty((S, d), dtype=rdt, device=dev)
     ops.linear_into(act, weight("wd"), out, residual=x1)
     return from_device(out, kind)

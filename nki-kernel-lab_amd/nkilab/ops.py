@@ -174,6 +174,40 @@ def gemm_swiglu_into(a: torch.Tensor, w_gu: torch.Tensor, c: torch.Tensor) -> to
     return c
 
 
+def _splits_k(a: torch.Tensor, w: torch.Tensor, M: int, N: int, K: int) -> bool:
+    """Whether a @ w^T splits its K over workgroups.  The one gate/up GEMM does
+    not, and its longer sums cost precision there (16 x 4064 x 2048: 23.5 us
+    against 28.5, but 5.9e-7 against 4.2e-7 from 64 bits)."""
+    return _lib.lib().nkl_gemm_workspace_bytes(a.data_ptr(), w.data_ptr(), M, N, K, a.stride(0), w.stride(0), 1, _lib.F32,
+                                               _lib.F32) > 0
+
+
+def gate_up_into(a: torch.Tensor, wg: torch.Tensor, wu: torch.Tensor, c: torch.Tensor) -> torch.Tensor:
+    """c = silu(a @ wg^T) * (a @ wu^T) (model.py:88) for a [M, K], nn.Linear-layout
+    weights wg, wu [N, K] and c [M, N], all of one dtype: one fp32 GEMM where its
+    16-byte accesses fit the operands, else two ``linear_into`` and a SwiGLU."""
+    M, K = a.shape
+    N = c.shape[1]
+    if c.shape[0] != M or wg.shape != (N, K) or wu.shape != (N, K):
+        raise ValueError(f"gate_up_into: a {tuple(a.shape)}, Wg {tuple(wg.shape)}, Wu {tuple(wu.shape)} and output "
+                         f"{tuple(c.shape)} do not match")
+    if (a.dtype == wg.dtype == wu.dtype == c.dtype == torch.float32 and M > 0 and K > 0
+            and a.stride(1) == wg.stride(1) == wu.stride(1) == c.stride(1) == 1
+            and (K <= 1504 or not _splits_k(a, wg, M, N, K))):
+        rc = _lib.lib().nkl_gemm_gate_up(a.data_ptr(), wg.data_ptr(), wu.data_ptr(), c.data_ptr(), M, N, K, a.stride(0),
+                                         wg.stride(0), wu.stride(0), c.stride(0), _lib.F32, stream_handle())
+        if rc == 0:
+            return c
+        if rc != _lib.EINVAL:
+            _lib.check("nkl_gemm_gate_up", rc)
+    gate, up = (torch.empty((M, N), dtype=c.dtype, device=c.device) for _ in range(2))
+    linear_into(a, wg, gate)
+    linear_into(a, wu, up)
+    if not c.is_contiguous():
+        return c.copy_(swiglu_into(gate, up, torch.empty_like(gate)))
+    return swiglu_into(gate, up, c)
+
+
 def matmul(a, b, variant: str = "blocked"):
     """C = A @ B for any shapes (ops.py:38-52).  bf16 inputs accumulate in fp32 and
     C is rounded once; the output dtype is the input dtype."""

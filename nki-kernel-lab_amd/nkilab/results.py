@@ -390,7 +390,8 @@ def bench_block(quick: bool) -> dict:
         ref = block(x)
     out = nki_forward(block, x)
     err = float((out - ref).abs().max())
-    # per-op breakdown, each op timed alone on the GPU (the reference's parts)
+    # per-op breakdown, each op timed alone on the GPU (the reference's parts;
+    # the forward itself runs gate, up and SwiGLU as one launch)
     dev = torch.device("cuda")
     xs = x.to(dev)
     W = {n: getattr(block, n).weight.detach().to(dev) for n in ("wqkv", "wo", "wg", "wu", "wd")}
@@ -427,7 +428,7 @@ def bench_block(quick: bool) -> dict:
                       "latency_source": "measured"})
     return {"config": dataclasses.asdict(cfg), "seq_len": S, "dtype": "float32",
             "max_abs_err_vs_pytorch": err, "max_abs_ref": float(ref.abs().max()),
-            "total_instructions": None, "kernel_launches": 9, "parts": parts}
+            "total_instructions": None, "kernel_launches": 7, "parts": parts}
 
 
 def small_traces() -> dict:

@@ -233,6 +233,38 @@ def test_gemm_swiglu_equals_gate_up_then_swiglu(rng, M, K, N):
     assert rel_err(_np(fused), ref) < 2e-2
 
 
+@pytest.mark.parametrize("M,K,N,off", [
+    (1, 4, 4, 0), (33, 36, 28, 4), (32, 64, 32, 0), (65, 132, 100, 8), (300, 256, 1024, 0),  # one round: 32x64, 64x64
+    (1000, 96, 1028, 0), (700, 64, 4064, 4), (2049, 36, 2052, 0),                            # 64x64, 64x128, 128x128
+    (33, 35, 28, 0), (33, 36, 27, 0), (33, 36, 28, 3)])                                      # the two-GEMM path
+def test_gate_up_fp32(M, K, N, off):
+    """The fp32 gate/up GEMM over two weights, every tile and the operands it
+    leaves to two GEMMs, as views `off` elements into wider rows of NaN (so that
+    anything read past K would show), against float64: silu has a slope of at
+    most 1.1, and gate and up are within K roundings of 2^-24 of the sums of
+    |a b|; 2^-20 covers the exponential, the division and the product."""
+    from nkilab import ops
+
+    g = torch.Generator(device="cuda").manual_seed(M * 31 + K * 7 + N)
+
+    def operand(r, c):
+        buf = torch.full((r, c + (12 if off else 0)), float("nan"), device="cuda")
+        v = buf[:, off:off + c]
+        v.copy_(torch.randn(r, c, generator=g, device="cuda"))
+        return v
+
+    a, wg, wu = operand(M, K), operand(N, K), operand(N, K)
+    cb = torch.full((M, N + 8), 5.0, device="cuda")
+    c = cb[:, 4:N + 4]
+    ops.gate_up_into(a, wg, wu, c)
+    gate, up = (a.double() @ w.double().t() for w in (wg, wu))
+    eg, eu = ((K + 2) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().t()) for w in (wg, wu))
+    silu = gate * torch.sigmoid(gate)
+    bound = 1.1 * eg * (up.abs() + eu) + silu.abs() * eu + 2.0 ** -20 * (silu * up).abs() + 2.0 ** -126
+    assert ((c.double() - silu * up).abs() <= bound).all()
+    assert (cb[:, :4] == 5).all() and (cb[:, N + 4:] == 5).all()
+
+
 def test_gemm_swiglu_rejects_bad_shapes():
     from nkilab import ops
 

@@ -108,6 +108,22 @@ def test_gemm_swiglu_abi_checks():
     assert L.nkl_gemm_swiglu(None, None, None, 0, 64, 64, 64, 64, 64, 1, None) == 0   # empty
 
 
+def test_gemm_gate_up_abi_checks():
+    from nkilab import _lib
+
+    call = _lib.lib().nkl_gemm_gate_up
+    p = 1 << 20  # (refused before any pointer is used)
+    assert call(None, None, None, None, 0, 64, 64, 64, 64, 64, 64, 0, None) == 0    # empty
+    assert call(None, None, None, None, 4, 64, 64, 64, 64, 64, 64, 0, None) == -1   # null
+    assert call(p, p, p, p, 4, 64, 64, 64, 64, 64, 64, 1, None) == -2               # bf16
+    assert call(p, p, p, p, -1, 64, 64, 64, 64, 64, 64, 0, None) == -1
+    assert call(p, p, p, p, 4, 62, 64, 64, 64, 64, 64, 0, None) == -1               # N % 4
+    assert call(p, p, p, p, 4, 64, 62, 64, 64, 64, 64, 0, None) == -1               # K % 4
+    assert call(p, p, p + 4, p, 4, 64, 64, 64, 64, 64, 64, 0, None) == -1           # Wu off 16 bytes
+    assert call(p, p, p, p, 4, 64, 64, 64, 64, 60, 64, 0, None) == -1               # ldu < K
+    assert call(p, p, p, p, 4, 64, 64, 64, 1 << 24, 64, 64, 0, None) == -1          # Wg of 4 GiB
+
+
 def test_noalloc_attention_rejects_shapes_beyond_its_static_scratch():
     """The allocation-free entry holds 1 MiB of arrival counters (one per
     64-query block): a balanced launch over 2^24 + 64 positions needs one more
