@@ -630,8 +630,9 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_dma_kernel(GemmArgs 
 // Bound by the K-step's chain (LDS reads, stores and a barrier, ~0.4 us with one
 // workgroup on a CU) on small grids and by LDS traffic on large ones.  One
 // wavefront per tile reading elements from global memory, as before, took 74 us
-// at 1000 x 777 x 1301 bf16; this takes 14.5 (rows at an odd address cost ~20%:
-// 12.2 at 1000 x 784 x 1304).
+// at 1000 x 777 x 1301 bf16; this takes 13.6 on 64x64 tiles (rows at an odd
+// address cost ~20%) and 10.5 on 64x128 with eight wavefronts, whose 176 tiles
+// make one round where 336 make two.
 //
 // LDS tiles are the LDS-DMA kernel's: 128-byte rows (32 fp32 or 64 16-bit
 // elements of K; B as [K, N] in 16 bits in sub-tiles of 64 columns), 16-byte
@@ -1180,15 +1181,33 @@ static void gemm_launch(const GemmArgs& a, int batch, hipStream_t st) {
       launch_dma_cols<T, TO, BT>(choose_tile(a, batch), g, batch, false, st);
     return;
   }
-  // 128x128 from one such tile per CU (4001 x 4099 x 3999 bf16 225 us, 64x64
-  // 395; level at 1501 x 2049 x 2047); fp32 grids that 32x64 tiles of four K
-  // groups cover in one round take those (300 x 256 x 1024 7.2 us, 64x64 8.9).
-  if (tiles_of(a, 128, 128, batch) >= 256)
-    launch_reg<T, TO, BT, 128, 128, 2, 2, 1, 1>(a, batch, st);
-  else if (sizeof(T) == 4 && tiles_of(a, 32, 64, batch) <= 256)
-    launch_reg<T, TO, BT, 32, 64, 1, 2, 4, 2>(a, batch, st);
-  else
-    launch_reg<T, TO, BT, 64, 64, 2, 2, 1, 1>(a, batch, st);
+  // The tile with the least rounds of workgroups (one per CU) times the
+  // measured time of a round.  16 bits, relative to a K-step: 64x64 0.36, 64x128
+  // with eight wavefronts 0.55, 128x128 with sixteen 0.75 (us, bf16: 1000 x 777 x
+  // 1301 13.6 / 10.5 / 12.9; 700 x 777 x 1301 9.1 / 10.2 / 13.4; 1001 x 4097 x
+  // 1999 44.7 / 35.5 / 43.5; 1500 x 2049 x 2047 38.2 / 35.4 / 25.9; 4001 x 129 x
+  // 1001 10.6 / 9.2 / 8.1; four wavefronts on 128x128 take 20.5 to 66 there).
+  // fp32: 32x64 in four K groups where it makes one round (300 x 256 x 1024 7.2,
+  // 64x64 8.9); 64x128, two K-steps ahead, costs 1.87 rounds of 64x64 (1000 x
+  // 777 x 1301 31.4 with 64x64, 29.6 with 64x128; 1500 x 2049 x 2047 109 / 130;
+  // 4001 x 2001 x 2003 271 / 254); 128x128 takes 142 at 2047 x 1023 x 2049, 64x64 92.
+  auto rounds = [&](int bm, int bn) { return (double)((tiles_of(a, bm, bn, batch) + 255) / 256); };
+  if constexpr (sizeof(T) == 4) {
+    if (tiles_of(a, 32, 64, batch) <= 256)
+      launch_reg<T, TO, BT, 32, 64, 1, 2, 4, 2>(a, batch, st);
+    else if (1.87 * rounds(64, 128) < rounds(64, 64))
+      launch_reg<T, TO, BT, 64, 128, 2, 4, 1, 2>(a, batch, st);
+    else
+      launch_reg<T, TO, BT, 64, 64, 2, 2, 1, 1>(a, batch, st);
+  } else {
+    const double c64 = 0.36 * rounds(64, 64), c64x128 = 0.55 * rounds(64, 128), c128 = 0.75 * rounds(128, 128);
+    if (c128 < c64x128 && c128 < c64)
+      launch_reg<T, TO, BT, 128, 128, 4, 4, 1, 1>(a, batch, st);
+    else if (c64x128 < c64)
+      launch_reg<T, TO, BT, 64, 128, 2, 4, 1, 1>(a, batch, st);
+    else
+      launch_reg<T, TO, BT, 64, 64, 2, 2, 1, 1>(a, batch, st);
+  }
 }
 
 // -------------------------------------- workspace: packed operands, split K --
@@ -1247,8 +1266,9 @@ static WsPlan plan_ws(const GemmArgs& a) {
   w.kp = a.K;
   w.np = a.N;
   // Packing pays from two rounds of 128x128 tiles on (bf16 4001 x 4099 x 3999
-  // 225 -> 159 us; 1501 x 2049 x 2047, 192 tiles, 40 -> 44); the fp32 kernels
-  // are close enough to each other that it does not.
+  // 202 -> 146 us, 3001 x 1001 x 3003 45 -> 40; below that it depends on K: 4001 x
+  // 129 x 1001, 256 tiles, 9 -> 13, 2047 x 1023 x 2049, 272 tiles, 31 -> 28); the
+  // fp32 kernels are close enough to each other that it does not.
   if (sizeof(T) == 2 && !dma_ok<T, BT>(a) && tiles_of(a, 128, 128, 1) >= 512) {
     w.pack_a = !aligned16(a.A) || a.K % E || a.lda % E;  // (K off a vector: zeros in A, and in B^T)
     w.pack_b = !aligned16(a.B) || a.ldb % E || (BT ? a.K % E : a.N % E);

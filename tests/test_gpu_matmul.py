@@ -339,6 +339,12 @@ def test_gemm_any_shape_and_alignment(dt, M, K, N, off):
             assert torch.equal(again, c)
 
 
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,N", [(1001, 77, 1301), (1537, 65, 1999)])  # 64x128; 128x128 in 16 bits, 64x128 in fp32
+def test_gemm_unaligned_tiles(dt, M, K, N):
+    test_gemm_any_shape_and_alignment(dt, M, K, N, 1)
+
+
 def test_gemm_workspace_is_for_the_shapes_that_use_it():
     """No workspace where one launch serves (the common aligned shapes); the K
     split and the packed operands ask for one, and refuse a smaller one."""
