@@ -94,9 +94,10 @@ int nkl_gemm(const void* A, const void* B, void* C, const void* R,
  * needed), which some shapes use: products of few tiles split a long K over
  * workgroups (fp32 partial sums, added in a fixed order by a second launch),
  * and large unaligned 16-bit products first copy their operands into aligned
- * rows.  Where the size is 0 the call is nkl_gemm's and a null workspace will
- * do; a workspace that is too small gets NKL_EWORKSPACE and nothing launched.
- * The size depends on what it is given, the alignment of A and B included.
+ * rows (if both are then under 2 GiB).  Where the size is 0 the call is
+ * nkl_gemm's and a null workspace will do; a workspace that is too small gets
+ * NKL_EWORKSPACE and nothing launched.  The size depends on what it is given,
+ * the alignment of A and B included.
  */
 size_t nkl_gemm_workspace_bytes(const void* A, const void* B, int M, int N,
                                 int K, long lda, long ldb, int b_trans,

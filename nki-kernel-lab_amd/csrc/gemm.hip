@@ -905,7 +905,7 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_reg_kernel(GemmArgs 
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       const int col = n0 + wn * WN + j * 32 + lr;
-      if (col >= N) continue;
+      if (col >= p.Nc) continue;
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const int row = m0 + wm * WM + i * 32 + 8 * (e / 4) + 4 * lg + (e % 4);
@@ -1268,15 +1268,22 @@ static WsPlan plan_ws(const GemmArgs& a) {
   // Packing pays from two rounds of 128x128 tiles on (bf16 4001 x 4099 x 3999
   // 202 -> 146 us, 3001 x 1001 x 3003 45 -> 40; below that it depends on K: 4001 x
   // 129 x 1001, 256 tiles, 9 -> 13, 2047 x 1023 x 2049, 272 tiles, 31 -> 28); the
-  // fp32 kernels are close enough to each other that it does not.
+  // fp32 kernels are close enough to each other that it does not.  Nor does it
+  // where the copies would still not suit the LDS-DMA kernel (2 GiB or more).
   if (sizeof(T) == 2 && !dma_ok<T, BT>(a) && tiles_of(a, 128, 128, 1) >= 512) {
-    w.pack_a = !aligned16(a.A) || a.K % E || a.lda % E;  // (K off a vector: zeros in A, and in B^T)
-    w.pack_b = !aligned16(a.B) || a.ldb % E || (BT ? a.K % E : a.N % E);
-    w.pack = w.pack_a || w.pack_b;
-    w.kp = (a.K + E - 1) / E * E;
-    if (!BT) w.np = (a.N + E - 1) / E * E;
-    if (w.pack_a) w.a_off = w.bytes, w.bytes += up(sizeof(T) * (size_t)a.M * w.kp);
-    if (w.pack_b) w.b_off = w.bytes, w.bytes += up(sizeof(T) * (BT ? (size_t)a.N * w.kp : (size_t)a.K * w.np));
+    const bool pa = !aligned16(a.A) || a.K % E || a.lda % E;  // (K off a vector: zeros in A, and in B^T)
+    const bool pb = !aligned16(a.B) || a.ldb % E || (BT ? a.K % E : a.N % E);
+    const int kp = (int)(((long)a.K + E - 1) / E * E), np = BT ? a.N : (int)(((long)a.N + E - 1) / E * E);
+    GemmArgs g = a;  // the product over the packed operands (null: an aligned base)
+    if (pa) g.A = nullptr, g.lda = kp;
+    if (pb) g.B = nullptr, g.ldb = BT ? kp : np;
+    g.N = np, g.padded = 1;
+    if ((pa || pb) && dma_ok<T, BT>(g)) {
+      w.pack = true, w.pack_a = pa, w.pack_b = pb;
+      w.kp = kp, w.np = np;
+      if (pa) w.a_off = w.bytes, w.bytes += up(sizeof(T) * (size_t)a.M * kp);
+      if (pb) w.b_off = w.bytes, w.bytes += up(sizeof(T) * (BT ? (size_t)a.N : (size_t)a.K) * (BT ? kp : np));
+    }
   }
   // K is split over workgroups when their tiles leave half the CUs idle and K
   // is long: parts of at least 8 K-steps, up to one workgroup per CU (bf16

@@ -345,6 +345,36 @@ def test_gemm_unaligned_tiles(dt, M, K, N):
     test_gemm_any_shape_and_alignment(dt, M, K, N, 1)
 
 
+@pytest.mark.parametrize("M,K,N", [(1 << 20, 1024, 129), (130, 8192, 131073)])  # A, then B, of 2 GiB
+def test_gemm_odd_columns_past_2_gib(M, K, N):
+    """An operand of 2 GiB with N off a vector, with and without a residual:
+    every element against fp32 products of row ranges, nothing written past the
+    columns or the last row of C.  bf16 inputs are exact in fp32; both sides sum
+    K products in fp32 (K 2^-24 of the sum of |a b| each) and C is rounded once
+    to bf16."""
+    from nkilab import ops
+
+    free = torch.cuda.mem_get_info()[0]
+    if free < 16 << 30:
+        pytest.skip(f"needs 16 GiB of GPU memory, {free >> 30} free")
+    g = torch.Generator(device="cuda").manual_seed(7)
+    a, b = (torch.empty(s, dtype=torch.bfloat16, device="cuda").normal_(generator=g) for s in ((M, K), (K, N)))
+    r = torch.empty((M, N), dtype=torch.bfloat16, device="cuda").normal_(generator=g)
+    step = 1 << 17
+    bf = b.float()
+    for res in (None, r):
+        cb = torch.full((M + 1, N + 3), 5.0, dtype=torch.bfloat16, device="cuda")
+        ops.gemm_into(a, b, cb[:M, :N], residual=res)
+        assert (cb[:, N:] == 5).all() and (cb[M] == 5).all()
+        for m in range(0, M, step):
+            want = a[m:m + step].float() @ bf
+            if res is not None:
+                want += res[m:m + step].float()
+            mag = a[m:m + step].float().abs() @ bf.abs()
+            bound = 2 * (K + 2) * 2.0 ** -24 * (mag + want.abs()) + 2.0 ** -8 * want.abs()
+            assert ((cb[m:min(m + step, M), :N].float() - want).abs() <= bound).all(), (m, res is not None)
+
+
 def test_gemm_workspace_is_for_the_shapes_that_use_it():
     """No workspace where one launch serves (the common aligned shapes); the K
     split and the packed operands ask for one, and refuse a smaller one."""

@@ -124,6 +124,27 @@ def test_gemm_gate_up_abi_checks():
     assert call(p, p, p, p, 4, 64, 64, 64, 1 << 24, 64, 64, 0, None) == -1          # Wg of 4 GiB
 
 
+@pytest.mark.parametrize("dt", [1, 2])
+@pytest.mark.parametrize("M,N,K,b_trans", [
+    (131072, 50257, 8192, 0), (1 << 20, 129, 1024, 0),  # A is 2 GiB and aligned, B's rows are not
+    (4096, 131073, 8192, 0),                            # B is past 2 GiB
+    ((1 << 20) + 1, 129, 1023, 0), ((1 << 20) + 1, 129, 1023, 1),  # A is below 2 GiB, its padded copy is not
+    (129, (1 << 20) + 1, 1023, 1), (1 << 21, 129, 1023, 1)])
+def test_gemm_operands_of_2_gib_are_not_packed(dt, M, N, K, b_trans):
+    """Operands are copied into aligned rows for the kernel with 32-bit buffer
+    offsets only: where an operand, or its copy, is 2 GiB or more the product
+    needs no workspace (a null one is taken by nkl_gemm_ws).  Half the rows or
+    columns, and the copy fits."""
+    from nkilab import _lib
+
+    p = 1 << 20  # (an aligned address, never used)
+    need = lambda m, n, k: _lib.lib().nkl_gemm_workspace_bytes(  # noqa: E731
+        p, p, m, n, k, k, k if b_trans else n, b_trans, dt, dt)
+    assert need(M, N, K) == 0
+    m, n = (M, N // 2 + 1) if N > M else ((M - 1) // 2, N)
+    assert need(m, n, K) > 0
+
+
 def test_noalloc_attention_rejects_shapes_beyond_its_static_scratch():
     """The allocation-free entry holds 1 MiB of arrival counters (one per
     64-query block): a balanced launch over 2^24 + 64 positions needs one more
