@@ -1144,7 +1144,9 @@ static void launch_f32_gate_up(const GemmArgs& g, hipStream_t st) {
     gemm_dma_kernel<float, float, 64, 64, true, 2, 2, 1, 4, true><<<grid(64, 64), dim3(512), 0, st>>>(g);
 }
 
-// The LDS-DMA kernel takes 16-byte chunks at 32-bit buffer offsets.
+// The LDS-DMA kernel takes 16-byte chunks at 32-bit buffer offsets, and K >= 1:
+// at K = 0 the bytes of a [K, N] B, (K - 1) ldb + N elements, are negative, a
+// range that no copy's offset is past.
 template <typename T, bool BT>
 static bool dma_ok(const GemmArgs& a) {
   constexpr int E = VecE<T>::value;
@@ -1152,7 +1154,7 @@ static bool dma_ok(const GemmArgs& a) {
   const int K = a.Kall ? a.Kall : a.K;
   const long a_bytes = SZ * ((long)(a.M - 1) * a.lda + K),
              b_bytes = SZ * (BT ? (long)(a.N - 1) * a.ldb + K : (long)(K - 1) * a.ldb + a.N);
-  return aligned16(a.A) && aligned16(a.B) && (K % E == 0 || a.padded) && a.lda % E == 0 && a.ldb % E == 0 && a.sA % E == 0 &&
+  return K > 0 && aligned16(a.A) && aligned16(a.B) && (K % E == 0 || a.padded) && a.lda % E == 0 && a.ldb % E == 0 && a.sA % E == 0 &&
          a.sB % E == 0 && (BT || a.N % E == 0) && a_bytes < (1L << 31) && b_bytes < (1L << 31);
 }
 

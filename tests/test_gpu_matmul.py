@@ -345,6 +345,30 @@ def test_gemm_unaligned_tiles(dt, M, K, N):
     test_gemm_any_shape_and_alignment(dt, M, K, N, 1)
 
 
+@pytest.mark.parametrize("b_trans", [0, 1])
+@pytest.mark.parametrize("dt,dt_out", [(0, 0), (1, 1), (1, 0), (2, 2), (2, 0)])
+@pytest.mark.parametrize("M,N", [(40, 24), (300, 1024), (2048, 4096)])
+def test_gemm_abi_with_no_k(b_trans, dt, dt_out, M, N):
+    """K = 0 through the C entries: C is the residual, or zeros, on every tile."""
+    from nkilab import _lib
+    from nkilab._tensors import stream_handle
+
+    t = {0: torch.float32, 1: torch.bfloat16, 2: torch.float16}
+    a, b = (torch.full((r, 8), float("nan"), dtype=t[dt], device="cuda") for r in (M, N))
+    b = b if b_trans else b.view(8, N)
+    r = torch.randn((M, N), device="cuda").to(t[dt_out])
+    for res in (None, r):
+        c = torch.full((M, N + 8), 5.0, dtype=t[dt_out], device="cuda")
+        args = (a.data_ptr(), b.data_ptr(), c.data_ptr(), None if res is None else res.data_ptr())
+        _lib.call("nkl_gemm", *args, M, N, 0, 8, 8 if b_trans else N, N + 8, N, b_trans, 1, 0, 0, 0, 0, dt, dt_out, 0,
+                  stream_handle())
+        assert torch.equal(c[:, :N], torch.zeros_like(r) if res is None else r) and (c[:, N:] == 5).all()
+        c.fill_(5)
+        _lib.call("nkl_gemm_ws", *args, None, 0, M, N, 0, 8, 8 if b_trans else N, N + 8, N, b_trans, dt, dt_out,
+                  stream_handle())
+        assert torch.equal(c[:, :N], torch.zeros_like(r) if res is None else r) and (c[:, N:] == 5).all()
+
+
 @pytest.mark.parametrize("M,K,N", [(1 << 20, 1024, 129), (130, 8192, 131073)])  # A, then B, of 2 GiB
 def test_gemm_odd_columns_past_2_gib(M, K, N):
     """An operand of 2 GiB with N off a vector, with and without a residual:
