@@ -107,8 +107,14 @@ def _gemm(a: torch.Tensor, bmat: torch.Tensor, ldb: int, b_trans: bool, c: torch
     rc = L.nkl_gemm_ws(pa, pb, pc, pr, None, 0, M, N, K, lda, ldb, ldc, ldr, bt, dt_in, dt_out, st)
     if rc == _lib.EWORKSPACE:
         nbytes = L.nkl_gemm_workspace_bytes(pa, pb, M, N, K, lda, ldb, bt, dt_in, dt_out)
-        ws = workspace(nbytes, c.device)
-        rc = L.nkl_gemm_ws(pa, pb, pc, pr, ws.data_ptr(), nbytes, M, N, K, lda, ldb, ldc, ldr, bt, dt_in, dt_out, st)
+        try:
+            ws = workspace(nbytes, c.device)
+        except torch.OutOfMemoryError:  # a workspace only makes the product faster: run it without one
+            rc = L.nkl_gemm(pa, pb, pc, pr, M, N, K, lda, ldb, ldc, ldr, bt, 1, 0, 0, 0, 0, dt_in, dt_out,
+                            _lib.GEMM_BLOCKED, st)
+        else:
+            rc = L.nkl_gemm_ws(pa, pb, pc, pr, ws.data_ptr(), nbytes, M, N, K, lda, ldb, ldc, ldr, bt, dt_in, dt_out,
+                               st)
     if rc:
         _lib.check("nkl_gemm_ws", rc)
     return c

@@ -399,6 +399,23 @@ def test_gemm_odd_columns_past_2_gib(M, K, N):
             assert ((cb[m:min(m + step, M), :N].float() - want).abs() <= bound).all(), (m, res is not None)
 
 
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,N", [(2945, 137, 2947), (8, 8021, 64)])  # packed operands; K split
+def test_gemm_without_memory_for_a_workspace(dt, M, K, N, monkeypatch):
+    """A product whose workspace cannot be allocated is computed without one."""
+    from nkilab import ops
+
+    asked = []
+
+    def none_left(nbytes, dev):
+        asked.append(nbytes)
+        raise torch.OutOfMemoryError("no memory left")
+
+    monkeypatch.setattr(ops, "workspace", none_left)
+    test_gemm_any_shape_and_alignment(dt, M, K, N, 0)
+    assert asked or (dt == torch.float32 and N > 64)  # (fp32 operands are not packed)
+
+
 def test_gemm_workspace_is_for_the_shapes_that_use_it():
     """No workspace where one launch serves (the common aligned shapes); the K
     split and the packed operands ask for one, and refuse a smaller one."""
