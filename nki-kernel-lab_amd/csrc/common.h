@@ -350,6 +350,8 @@ __device__ __forceinline__ float load_frag(const float* p) { return *p; }
 namespace nkl {
 // Records `msg` as this thread's last error and returns `code`.
 int set_error(int code, const char* fmt, ...);
+// HIP takes fewer than 2^32 threads along x in one launch.
+constexpr long kMaxGridThreads = (1L << 32) - 1;
 // Checks hipGetLastError() after a launch; returns NKL_OK or NKL_ELAUNCH.
 int check_launch(const char* what);
 }  // namespace nkl

@@ -472,6 +472,17 @@ static bool with_row_plan(RowPlan p, F f) {
   return false;
 }
 
+// Calls f(first row, rows, grid) for the launches of a row kernel: one, unless
+// its threads pass HIP's limit (16.8M rows of 256 threads).
+template <typename F>
+static void for_row_launches(int rows, int rows_per_wg, int threads, F f) {
+  const long step = kMaxGridThreads / threads * rows_per_wg;
+  for (long r = 0; r < rows; r += step) {
+    const int n = (int)min(step, rows - r);
+    f(r, n, dim3((unsigned)(((long)n + rows_per_wg - 1) / rows_per_wg)));
+  }
+}
+
 template <typename T>
 static int softmax_launch_plan(RowPlan plan, const void* x, void* y, int rows, int cols, long ldx, long ldy,
                                hipStream_t st) {
@@ -480,14 +491,18 @@ static int softmax_launch_plan(RowPlan plan, const void* x, void* y, int rows, i
   T* yp = static_cast<T*>(y);
   const bool al = cols % E == 0 && ldx % E == 0 && ldy % E == 0 && aligned16(x) && aligned16(y);
   const bool done = with_row_plan<T>(plan, [&](auto W, auto N) {
-    constexpr int WPR = decltype(W)::value, NV = decltype(N)::value;
-    const dim3 grid(WPR == 1 ? (rows + kRowsPerBlock - 1) / kRowsPerBlock : rows), block(WPR == 1 ? 256 : 64 * WPR);
-    if (al)
-      softmax_vec_kernel<T, WPR, NV, true><<<grid, block, 0, st>>>(xp, yp, rows, cols, ldx, ldy);
-    else
-      softmax_vec_kernel<T, WPR, NV, false><<<grid, block, 0, st>>>(xp, yp, rows, cols, ldx, ldy);
+    constexpr int WPR = decltype(W)::value, NV = decltype(N)::value, NT = WPR == 1 ? 256 : 64 * WPR;
+    for_row_launches(rows, WPR == 1 ? kRowsPerBlock : 1, NT, [&](long r, int n, dim3 grid) {
+      if (al)
+        softmax_vec_kernel<T, WPR, NV, true><<<grid, dim3(NT), 0, st>>>(xp + r * ldx, yp + r * ldy, n, cols, ldx, ldy);
+      else
+        softmax_vec_kernel<T, WPR, NV, false><<<grid, dim3(NT), 0, st>>>(xp + r * ldx, yp + r * ldy, n, cols, ldx, ldy);
+    });
   });
-  if (!done) softmax_loop_kernel<T><<<dim3(rows), dim3(1024), 0, st>>>(xp, yp, cols, ldx, ldy);
+  if (!done)
+    for_row_launches(rows, 1, 1024, [&](long r, int, dim3 grid) {
+      softmax_loop_kernel<T><<<grid, dim3(1024), 0, st>>>(xp + r * ldx, yp + r * ldy, cols, ldx, ldy);
+    });
   return check_launch("nkl_softmax");
 }
 template <typename T>
@@ -506,16 +521,21 @@ static int rmsnorm_launch_plan(RowPlan plan, const void* x, const void* w, void*
   const float inv_d = (float)(1.0 / (double)cols);
   const bool al = cols % E == 0 && ldx % E == 0 && ldy % E == 0 && aligned16(x) && aligned16(w) && aligned16(y);
   const bool done = with_row_plan<TI>(plan, [&](auto W, auto N) {
-    constexpr int WPR = decltype(W)::value, NV = decltype(N)::value;
-    const dim3 grid(WPR == 1 ? (rows + kRowsPerBlock - 1) / kRowsPerBlock : rows), block(WPR == 1 ? 256 : 64 * WPR);
-    if (al)
-      rmsnorm_vec_kernel<TI, TW, TO, WPR, NV, true><<<grid, block, 0, st>>>(xp, wp, yp, rows, cols, ldx, ldy, inv_d,
-                                                                            eps);
-    else
-      rmsnorm_vec_kernel<TI, TW, TO, WPR, NV, false><<<grid, block, 0, st>>>(xp, wp, yp, rows, cols, ldx, ldy, inv_d,
-                                                                             eps);
+    constexpr int WPR = decltype(W)::value, NV = decltype(N)::value, NT = WPR == 1 ? 256 : 64 * WPR;
+    for_row_launches(rows, WPR == 1 ? kRowsPerBlock : 1, NT, [&](long r, int n, dim3 grid) {
+      if (al)
+        rmsnorm_vec_kernel<TI, TW, TO, WPR, NV, true><<<grid, dim3(NT), 0, st>>>(xp + r * ldx, wp, yp + r * ldy, n, cols,
+                                                                                 ldx, ldy, inv_d, eps);
+      else
+        rmsnorm_vec_kernel<TI, TW, TO, WPR, NV, false><<<grid, dim3(NT), 0, st>>>(xp + r * ldx, wp, yp + r * ldy, n,
+                                                                                  cols, ldx, ldy, inv_d, eps);
+    });
   });
-  if (!done) rmsnorm_loop_kernel<TI, TW, TO><<<dim3(rows), dim3(1024), 0, st>>>(xp, wp, yp, cols, ldx, ldy, inv_d, eps);
+  if (!done)
+    for_row_launches(rows, 1, 1024, [&](long r, int, dim3 grid) {
+      rmsnorm_loop_kernel<TI, TW, TO><<<grid, dim3(1024), 0, st>>>(xp + r * ldx, wp, yp + r * ldy, cols, ldx, ldy, inv_d,
+                                                                   eps);
+    });
   return check_launch("nkl_rmsnorm");
 }
 template <typename TI, typename TW, typename TO>

@@ -295,3 +295,35 @@ def test_softmax_of_infinite_and_masked_rows():
         assert (y[0, ::2] == 0).all() and abs(y[0].double().sum().item() - 1) < 1e-5
         assert y[1, 0] == 1 and (y[1, 1:] == 0).all()
         assert torch.isnan(y[2]).all() and torch.isnan(y[3, D // 2]) and torch.isnan(y[4]).all()
+
+
+def test_row_kernels_past_one_launch():
+    """More rows than one launch of a workgroup per row takes (HIP's limit of
+    2^32 threads, 16.8M rows of 256), in place: the rows on both sides of the
+    second launch, and one column of every other."""
+    from nkilab import ops
+
+    R, D = (1 << 24) + 5, 4104
+    torch.cuda.empty_cache()
+    free = torch.cuda.mem_get_info()[0]
+    if free < (R * D * 2) + (8 << 30):
+        pytest.skip(f"needs {(R * D * 2 >> 30) + 8} GiB of GPU memory, {free >> 30} free")
+    rows = [0, 1, (1 << 24) - 2, (1 << 24) - 1, 1 << 24, R - 1]
+    others = torch.ones(R, dtype=torch.bool, device="cuda")
+    others[rows] = False
+    x = torch.zeros(R, D, dtype=torch.bfloat16, device="cuda")
+    special = torch.randn(len(rows), D, device="cuda").bfloat16()
+    x[rows] = special
+    ops.softmax_into(x, x)
+    assert_within_bf16_ulps(_np(x[rows]), torch.softmax(special.double(), -1).cpu().numpy())
+    assert (x[others, 7] == torch.tensor(1 / D).bfloat16().cuda()).all()
+    x.fill_(2)
+    x[rows] = special
+    w = (torch.rand(D, device="cuda") + 0.5).bfloat16()
+    ops.rmsnorm_into(x, w, x)
+    s = special.double()
+    ref = s * torch.rsqrt(s.pow(2).mean(-1, keepdim=True) + 1e-6) * w.double()
+    assert_within_bf16_ulps(_np(x[rows]), ref.cpu().numpy())
+    assert (x[others, 7] == w[7]).all()
+    del x
+    torch.cuda.empty_cache()
