@@ -320,16 +320,40 @@ __global__ __launch_bounds__(512) void flash_f32_kernel(AttnArgs p) {
   }
 }
 
+// One launch over all heads, unless their threads pass HIP's limit: then
+// over ranges of heads, each of whole groups or within one group.
+template <int D, int NHF>
+static void launch_heads(const AttnArgs& a, hipStream_t st) {
+  const long nqb = ((long)a.S + 32 * NHF - 1) / (32 * NHF), fit = kMaxGridThreads / 512 / nqb;
+  for (long h = 0, n; h < a.H; h += n) {
+    n = min(fit > 1 ? fit : 1, a.H - h);
+    AttnArgs p = a;
+    if (n < a.H && a.group > 1) {
+      const long left = a.group - h % a.group;  // heads left of the group of head h
+      if (left < a.group || n < a.group)
+        n = min(n, left), p.group = (int)n;
+      else
+        n -= n % a.group;
+    }
+    p.H = (int)n;
+    p.q = static_cast<const float*>(a.q) + h * a.q_sh;
+    p.k = static_cast<const float*>(a.k) + h / a.group * a.k_sh;
+    p.v = static_cast<const float*>(a.v) + h / a.group * a.v_sh;
+    p.o = static_cast<float*>(a.o) + h * a.o_sh;
+    flash_f32_kernel<D, NHF><<<dim3((unsigned)(nqb * n)), dim3(512), 0, st>>>(p);
+  }
+}
+
 template <int D>
 static void launch(const AttnArgs& a, hipStream_t st) {
   // 32-query blocks where 64-query ones leave half the CUs idle: half the MFMAs
   // of a step per workgroup (us, 64 / 32: 4 x 300 x 64 17.8 / 10.9, 1 x 4096 x
   // 128 290 / 161, 2 x 100 x 128 15.7 / 9.5).
-  const long n64 = (a.S + 63) / 64, n32 = (a.S + 31) / 32;
+  const long n64 = ((long)a.S + 63) / 64;
   if (n64 * a.H <= 128)
-    flash_f32_kernel<D, 1><<<dim3((unsigned)(n32 * a.H)), dim3(512), 0, st>>>(a);
+    launch_heads<D, 1>(a, st);
   else
-    flash_f32_kernel<D, 2><<<dim3((unsigned)(n64 * a.H)), dim3(512), 0, st>>>(a);
+    launch_heads<D, 2>(a, st);
 }
 
 int flash_f32_launch(const AttnArgs& a, hipStream_t st) {

@@ -525,6 +525,19 @@ def test_flash_fp32_against_float64(H, Hkv, S, d, scale):
     assert (ob[:, S] == 7).all()
 
 
+@pytest.mark.parametrize("H,Hkv", [((1 << 23) + 3, (1 << 23) + 3), (3 * 2796204, 2796204), ((1 << 23) + 2, 2),
+                                   ((1 << 23) + 2, 1)])
+def test_flash_fp32_heads_past_one_launch(H, Hkv):
+    """More heads than one launch of 512 threads a head takes (HIP's limit of
+    2^32 threads), alone and in groups of 3, of half of them and of all: at one
+    position each query's output is its head's value."""
+    from nkilab import ops
+
+    q, k, v = (torch.randn(n, 1, 4, device="cuda") for n in (H, Hkv, Hkv))
+    o = ops.attention(q, k, v)
+    assert torch.equal(o, v.repeat_interleave(H // Hkv, 0))
+
+
 def test_flash_fp32_with_infinite_scores():
     """A key whose score is -inf for every query gets no weight, a query that
     sees nothing else is NaN, and NaN stays in the queries that see it."""
