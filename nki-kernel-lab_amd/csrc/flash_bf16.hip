@@ -1530,7 +1530,9 @@ Config choose(int H, int S, int d, bool f16) {
   const bool tiny_fits = (long)H * nqb <= cus || units128 < kMinUnits * cus || S <= 64;
   if (d > 64 && d <= 128 && (S <= kTinyAutoS || (S <= kTinyMaxS && cfg.qb == 64)) && tiny_fits)
     cfg = Config{128, kBlock, kTiny};
-  if (d <= 64) cfg = choose_narrow(H, S, d);
+  // (Past HIP's limit on threads a launch, the pairs of 128-query blocks above,
+  // which are up to half as many threads.)
+  if (d <= 64 && (long)H * (((long)S + 63) / 64) * 256 <= kMaxGridThreads) cfg = choose_narrow(H, S, d);
   const Overrides& ov = overrides();
   if (ov.sched >= 0) cfg.sched = ov.sched;
   if (ov.qb >= 0) cfg.qb = ov.qb;

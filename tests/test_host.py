@@ -472,6 +472,18 @@ def test_kernel_choice_rules():
     assert plan(16, 4096)[1] == 16 * 2112 // 2                      # 132 units per CU: ping-pong
 
 
+def test_narrow_head_launch_fits_the_thread_limit():
+    """Head dims up to 64: one four-wavefront workgroup per 64-query block up to
+    HIP's limit of 2^32 threads a launch (16.8M of those), then one
+    eight-wavefront workgroup per pair of 128-query blocks."""
+    from nkilab import _lib
+
+    _lib.flash_configure()
+    H = (1 << 24) // 3
+    assert _lib.flash_plan_check(H, 129, 8)[0] == 3 * H
+    assert _lib.flash_plan_check(H + 1, 129, 8)[0] == H + 1
+
+
 def test_merge_wait_rule():
     """The workgroup merging a split block waits (a bounded 256 polls) while
     blocks have few parts, and not at all when the longest block spans six or
