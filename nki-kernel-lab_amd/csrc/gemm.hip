@@ -969,7 +969,7 @@ static int forced_tile() {
 }
 
 static long tiles_of(const GemmArgs& a, int bm, int bn, int batch) {
-  return (long)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn) * batch;
+  return (((long)a.M + bm - 1) / bm) * (((long)a.N + bn - 1) / bn) * batch;
 }
 
 // Tile choice.  With a 128x128 tile or larger for every CU, the tile whose
@@ -1100,10 +1100,25 @@ static void launch_dma_cols(DmaTile t, const GemmArgs& g, int batch, bool swiglu
   launch_dma<TI, TO, BT>(pl.t2, g2, 1, st);
 }
 
+// One launch, unless its threads pass HIP's limit (a column of 1.1G rows is
+// 16.8M tiles of 256 threads): then over ranges of rows and columns.
 template <typename T, typename TO, bool BT, int BM, int BN, int WGM, int WGN, int KG, int PF>
 static void launch_reg(const GemmArgs& a, int batch, hipStream_t st) {
-  const dim3 grid((unsigned)tiles_of(a, BM, BN, 1), 1, (unsigned)batch);
-  gemm_reg_kernel<T, TO, BM, BN, BT, WGM, WGN, KG, PF><<<grid, dim3(64 * WGM * WGN * KG), 0, st>>>(a);
+  constexpr int NT = 64 * WGM * WGN * KG;
+  const long fit = kMaxGridThreads / NT, cols = min(tiles_of(a, a.M, BN, 1), fit) * BN, rows = fit / (cols / BN) * BM;
+  for (long m = 0; m < a.M; m += rows)
+    for (long n = 0; n < a.N; n += cols) {
+      GemmArgs g = a;
+      g.M = (int)min(rows, a.M - m);
+      g.N = (int)min(cols, a.N - n);
+      g.Nc = (int)min((long)g.N, a.Nc - n);
+      g.A = static_cast<const T*>(a.A) + m * a.lda;
+      g.B = static_cast<const T*>(a.B) + (BT ? n * a.ldb : n);
+      g.C = static_cast<TO*>(a.C) + m * a.ldc + n;
+      if (a.R) g.R = static_cast<const TO*>(a.R) + m * a.ldr + n;
+      const dim3 grid((unsigned)tiles_of(g, BM, BN, 1), 1, (unsigned)batch);
+      gemm_reg_kernel<T, TO, BM, BN, BT, WGM, WGN, KG, PF><<<grid, dim3(NT), 0, st>>>(g);
+    }
 }
 
 // fp32 tiles of the LDS-DMA kernel (two or four K groups each).

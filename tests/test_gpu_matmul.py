@@ -399,6 +399,36 @@ def test_gemm_odd_columns_past_2_gib(M, K, N):
             assert ((cb[m:min(m + step, M), :N].float() - want).abs() <= bound).all(), (m, res is not None)
 
 
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+@pytest.mark.parametrize("columns", [False, True])
+def test_gemm_tiles_past_one_launch(layout, columns):
+    """One column (or row) of more elements than the tiles of one launch hold
+    (HIP's limit of 2^32 threads): each an exact product of two bf16 values plus
+    the residual, rounded in fp32 and then to bf16, on both sides."""
+    from nkilab import ops
+
+    n = (1 << 30) + 65
+    torch.cuda.empty_cache()
+    free = torch.cuda.mem_get_info()[0]
+    if free < 24 << 30:
+        pytest.skip(f"needs 24 GiB of GPU memory, {free >> 30} free")
+    x = torch.empty(n, dtype=torch.bfloat16, device="cuda").normal_()
+    s = torch.full((1, 1), 1.75, dtype=torch.bfloat16, device="cuda")
+    r = torch.empty(n, dtype=torch.bfloat16, device="cuda").normal_()
+    c = torch.full((n + 8,), 5.0, dtype=torch.bfloat16, device="cuda")
+    shape = (1, n) if columns else (n, 1)
+    a, b = (s, x.view(shape)) if columns else (x.view(shape), s)
+    if layout == "nt":
+        ops.linear_into(a, b.view(b.shape[1], 1), c[:n].view(shape), residual=r.view(shape))
+    else:
+        ops.gemm_into(a, b, c[:n].view(shape), residual=r.view(shape))
+    step = 1 << 28
+    for i in range(0, n, step):
+        want = (x[i:i + step].float() * 1.75 + r[i:i + step].float()).bfloat16()
+        assert torch.equal(c[i:min(i + step, n)], want), i
+    assert (c[n:] == 5).all()
+
+
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M,K,N", [(2945, 137, 2947), (8, 8021, 64)])  # packed operands; K split
 def test_gemm_without_memory_for_a_workspace(dt, M, K, N, monkeypatch):
