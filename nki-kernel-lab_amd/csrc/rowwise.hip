@@ -140,11 +140,11 @@ __global__ __launch_bounds__(WPR == 1 ? 256 : 64 * WPR, row_waves(WPR, NV, VecE<
   if (row >= rows) return;  // WPR > 1: one row per workgroup, never taken
   const T* xr = x + (long)row * ldx;
   T* yr = y + (long)row * ldy;
-  const int head = AL ? 0 : row_head(yr, cols);
+  const int head = AL ? 0 : NV == 0 ? cols : row_head(yr, cols);
   const int nvec = (cols - head) / E, edge = AL ? 0 : cols - nvec * E;
   // Edge element of lane t < edge: the row's first head, then its last ones.
   const int te = t < head ? t : nvec * E + t;
-  float v[NV][E];
+  float v[NV > 0 ? NV : 1][E];
 #pragma unroll
   for (int n = 0; n < NV; ++n) {
     const int vi = n * 64 * WPR + t;
@@ -310,11 +310,12 @@ __global__ __launch_bounds__(WPR == 1 ? 256 : 64 * WPR, row_waves(WPR, NV, VecE<
   if (row >= rows) return;  // WPR > 1: one row per workgroup, never taken
   const TI* xr = x + (long)row * ldx;
   TO* yr = y + (long)row * ldy;
-  const int head = AL ? 0 : row_head(yr, cols);
+  const int head = AL ? 0 : NV == 0 ? cols : row_head(yr, cols);
   const int nvec = (cols - head) / E, edge = AL ? 0 : cols - nvec * E;
   // Edge element of lane t < edge: the row's first head, then its last ones.
   const int te = t < head ? t : nvec * E + t;
-  float v[NV][E];
+  const bool two = NV == 0 && t + kWave < cols;  // (a row of edge elements alone: two a lane)
+  float v[NV > 0 ? NV : 1][E];
 #pragma unroll
   for (int n = 0; n < NV; ++n) {
     const int vi = n * 64 * WPR + t;
@@ -325,9 +326,10 @@ __global__ __launch_bounds__(WPR == 1 ? 256 : 64 * WPR, row_waves(WPR, NV, VecE<
       for (int e = 0; e < E; ++e) v[n][e] = 0.f;
     }
   }
-  float tv = 0.f;
+  float tv = 0.f, tv2 = 0.f;
   if (t < edge) tv = to_f32(xr[te]);
-  float ssq = tv * tv;
+  if (two) tv2 = to_f32(xr[t + kWave]);
+  float ssq = fmaf(tv2, tv2, tv * tv);
 #pragma unroll
   for (int n = 0; n < NV; ++n)
 #pragma unroll
@@ -347,6 +349,7 @@ __global__ __launch_bounds__(WPR == 1 ? 256 : 64 * WPR, row_waves(WPR, NV, VecE<
     }
   }
   if (t < edge) yr[te] = from_f32<TO>((tv * rstd) * to_f32(w[te]));
+  if (two) yr[t + kWave] = from_f32<TO>((tv2 * rstd) * to_f32(w[t + kWave]));
 }
 
 // Rows too long for registers: one 1024-thread workgroup per row, two sweeps.
@@ -439,6 +442,14 @@ static bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 struct RowPlan {
   int wpr, nv;
 };
+// Short unaligned rows: one element a lane of one wavefront (RMSNorm: up to
+// two), no vectors.  300000 rows in the last-level cache, us, with vectors /
+// without: softmax bf16 x 3 54.3 / 39.7, x 17 62.0 / 43.0, x 64 62.6 / 45.8,
+// fp32 x 17 54.7 / 43.5, but 65536 x 64 12.5 / 13.8; RMSNorm bf16 x 17 53.3 / 39.1,
+// x 65 67.4 / 55.3, x 127 68.4 / 57.0, fp32 x 63 57.0 / 42.9; where y's rows all
+// start on 64 bytes and fill both elements, bf16 x 96 53.4 / 60.9.
+constexpr RowPlan kShortRow{1, 0};
+
 template <typename T>
 static RowPlan pick_row(int rows, int cols, int deep_rows) {
   constexpr int E = VecE<T>::value;
@@ -463,7 +474,7 @@ static bool with_row_plan(RowPlan p, F f) {
     f(std::integral_constant<int, W>{}, std::integral_constant<int, N>{});   \
     return true;                                                             \
   }
-  NKL_ROW(1, 1) NKL_ROW(1, 2) NKL_ROW(1, 4) NKL_ROW(1, 8)
+  NKL_ROW(1, 0) NKL_ROW(1, 1) NKL_ROW(1, 2) NKL_ROW(1, 4) NKL_ROW(1, 8)
   if constexpr (VecE<T>::value == 4) { NKL_ROW(1, 16) }
   NKL_ROW(4, 1) NKL_ROW(4, 2) NKL_ROW(4, 4) NKL_ROW(4, 8)
   if constexpr (VecE<T>::value == 4) { NKL_ROW(4, 16) NKL_ROW(16, 16) } else { NKL_ROW(16, 4) }
@@ -490,6 +501,7 @@ static int softmax_launch_plan(RowPlan plan, const void* x, void* y, int rows, i
   const T* xp = static_cast<const T*>(x);
   T* yp = static_cast<T*>(y);
   const bool al = cols % E == 0 && ldx % E == 0 && ldy % E == 0 && aligned16(x) && aligned16(y);
+  if (!al && cols * sizeof(T) <= 128) plan = kShortRow;
   const bool done = with_row_plan<T>(plan, [&](auto W, auto N) {
     constexpr int WPR = decltype(W)::value, NV = decltype(N)::value, NT = WPR == 1 ? 256 : 64 * WPR;
     for_row_launches(rows, WPR == 1 ? kRowsPerBlock : 1, NT, [&](long r, int n, dim3 grid) {
@@ -520,6 +532,7 @@ static int rmsnorm_launch_plan(RowPlan plan, const void* x, const void* w, void*
   // The multiplier 1/D is the fp32 value nearest the exact quotient.
   const float inv_d = (float)(1.0 / (double)cols);
   const bool al = cols % E == 0 && ldx % E == 0 && ldy % E == 0 && aligned16(x) && aligned16(w) && aligned16(y);
+  if (!al && cols * sizeof(TI) <= 256 && (cols <= kWave || ldy * sizeof(TO) % 64)) plan = kShortRow;
   const bool done = with_row_plan<TI>(plan, [&](auto W, auto N) {
     constexpr int WPR = decltype(W)::value, NV = decltype(N)::value, NT = WPR == 1 ? 256 : 64 * WPR;
     for_row_launches(rows, WPR == 1 ? kRowsPerBlock : 1, NT, [&](long r, int n, dim3 grid) {

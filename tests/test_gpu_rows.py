@@ -279,6 +279,15 @@ def test_row_kernels_at_every_plan(dt, R, D):
             assert (yb[:, :off_y] == 7).all() and (yb[:, off_y + D:] == 7).all()
 
 
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("D", [2, 31, 32, 33, 63, 64, 65, 96, 127, 128, 129])
+def test_short_unaligned_rows(dt, D):
+    """Rows at the limits of the kernels that hold one element a lane (64; 32
+    in fp32 softmax) or two (RMSNorm: 128 in bf16, 64 in fp32)."""
+    test_row_kernels_at_every_plan(dt, 70, D)
+    test_row_kernels_at_every_plan(dt, 1, D)
+
+
 def test_softmax_of_infinite_and_masked_rows():
     """Masked entries (-inf, the type's lowest value) get probability 0, a row
     of them and a row with +inf or NaN is NaN, at every plan."""
