@@ -668,8 +668,12 @@ __device__ __forceinline__ u32x4_t ld16_first(const T* p, int n) {
   return r;
 }
 
-template <typename TI, typename TO, int BM, int BN, bool BT, int WGM, int WGN, int KG, int PF>
+template <typename TI, typename TO, int BM, int BN, bool BT, int WGM, int WGN, int KG, int PF, int ACC = 1,
+          bool SHORT = false>
 __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_reg_kernel(GemmArgs p) {
+  // ACC = 2: even and odd K-steps are summed apart and added at the end, as two
+  // K groups do.  SHORT: a K-step or two, loaded with checks and without the
+  // sub-steps that hold zeros alone.
   constexpr bool F32 = sizeof(TI) == 4;
   constexpr bool H = std::is_same<TI, f16>::value;
   constexpr int E = VecE<TI>::value;  // elements per 16-byte chunk
@@ -776,22 +780,26 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_reg_kernel(GemmArgs 
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
   };
 
-  floatx16 acc[TM][TN];
+  floatx16 accs[ACC][TM][TN];
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+  for (int x = 0; x < ACC; ++x)
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) accs[x][i][j][e] = 0.f;
 
   const int nk = ((K + BK - 1) / BK + KG - 1) / KG;
-  // Every fragment of the K-step in stage st is read in flight together, then
-  // `mid` runs behind the reads, then the MFMAs.
-  auto compute = [&](int st, auto mid) __attribute__((always_inline)) {
+  // Every fragment of the K-step in stage st (its first nks sub-steps) is read
+  // in flight together, then `mid` runs behind the reads, then the MFMAs into
+  // acc.
+  auto compute = [&](int st, int nks, floatx16 (&acc)[TM][TN], auto mid) __attribute__((always_inline)) {
     const unsigned char* sb = lds + st * SSET + kg * STAGE;
     bf16x8 af[4][TM], bfr[4][TN];
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
+      if (ks >= nks) break;
 #pragma unroll
       for (int i = 0; i < TM; ++i)
         af[ks][i] = *reinterpret_cast<const bf16x8*>(sb + g_pos(wm * WM + lr, 2 * ks + lg) + 4096 * i);
@@ -819,6 +827,7 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_reg_kernel(GemmArgs 
     mid();
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
+      if (ks >= nks) break;
       if constexpr (F32) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
@@ -840,7 +849,7 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_reg_kernel(GemmArgs 
   // Leading steps (every group's K-step a leading one): no branch around a
   // load, so that each wait counts the loads issued after the one it waits
   // for.  The last steps' loads past nfast repeat the last leading step.
-  const int nfast = kfast / KG;
+  const int nfast = SHORT ? 0 : kfast / KG;
   if (nfast > 0) {
 #pragma unroll
     for (int u = 0; u < PF; ++u) gload(min(u, nfast - 1), rra[u], rrb[u]);
@@ -848,12 +857,12 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_reg_kernel(GemmArgs 
     gload(min(PF, nfast - 1), rra[0], rrb[0]);
     lds_barrier();
 #pragma unroll 1
-    for (int s0 = 0; s0 < nfast; s0 += PF)
+    for (int s0 = 0; s0 < nfast; s0 += max(PF, ACC))
 #pragma unroll
-      for (int u = 0; u < PF; ++u) {
+      for (int u = 0; u < max(PF, ACC); ++u) {
         const int s = s0 + u;
         if (s >= nfast) break;
-        compute(s & 1, [&]() __attribute__((always_inline)) {
+        compute(s & 1, 4, accs[u % ACC], [&]() __attribute__((always_inline)) {
           // The next K-step's LDS stores (its stage was read last in step
           // s - 1) and the global loads PF steps after it.
           lstore((s + 1) & 1, rra[(u + 1) % PF], rrb[(u + 1) % PF]);
@@ -867,8 +876,22 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_reg_kernel(GemmArgs 
     gload_checked(s, rra[0], rrb[0]);
     lstore(s & 1, rra[0], rrb[0]);
     lds_barrier();
-    compute(s & 1, []() {});
+    constexpr int SUB = BK / 4;  // K elements of a sub-step
+    const int nks = SHORT ? (K - (KG * s + kg) * BK + SUB - 1) / SUB : 4;
+    if (ACC == 1 || s % 2 == 0)
+      compute(s & 1, nks, accs[0], []() {});
+    else
+      compute(s & 1, nks, accs[ACC - 1], []() {});
     lds_barrier();
+  }
+  floatx16(&acc)[TM][TN] = accs[0];
+  if constexpr (ACC == 2) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] += accs[1][i][j][e];
   }
 
   if constexpr (KG > 1) {
@@ -1102,7 +1125,8 @@ static void launch_dma_cols(DmaTile t, const GemmArgs& g, int batch, bool swiglu
 
 // One launch, unless its threads pass HIP's limit (a column of 1.1G rows is
 // 16.8M tiles of 256 threads): then over ranges of rows and columns.
-template <typename T, typename TO, bool BT, int BM, int BN, int WGM, int WGN, int KG, int PF>
+template <typename T, typename TO, bool BT, int BM, int BN, int WGM, int WGN, int KG, int PF, int ACC = 1,
+          bool SHORT = false>
 static void launch_reg(const GemmArgs& a, int batch, hipStream_t st) {
   constexpr int NT = 64 * WGM * WGN * KG;
   const long fit = kMaxGridThreads / NT, cols = min(tiles_of(a, a.M, BN, 1), fit) * BN, rows = fit / (cols / BN) * BM;
@@ -1117,7 +1141,7 @@ static void launch_reg(const GemmArgs& a, int batch, hipStream_t st) {
       g.C = static_cast<TO*>(a.C) + m * a.ldc + n;
       if (a.R) g.R = static_cast<const TO*>(a.R) + m * a.ldr + n;
       const dim3 grid((unsigned)tiles_of(g, BM, BN, 1), 1, (unsigned)batch);
-      gemm_reg_kernel<T, TO, BM, BN, BT, WGM, WGN, KG, PF><<<grid, dim3(NT), 0, st>>>(g);
+      gemm_reg_kernel<T, TO, BM, BN, BT, WGM, WGN, KG, PF, ACC, SHORT><<<grid, dim3(NT), 0, st>>>(g);
     }
 }
 
@@ -1186,10 +1210,51 @@ static F32Tile choose_f32_tile(const GemmArgs& a, int batch) {
   return c128 <= c64x128 && c128 <= c64 ? kF128x128 : c64x128 < c64 ? kF64x128 : kF64x64;
 }
 
+template <typename T, typename TO, bool BT>
+static void launch_naive(const GemmArgs& a, int batch, hipStream_t st) {
+  gemm_naive_kernel<T, TO, BT><<<dim3((unsigned)((tiles_of(a, 32, 32, 1) + 3) / 4), 1, batch), dim3(256), 0, st>>>(a);
+}
+
+// Unaligned products with next to no K, which writing C bounds: one wavefront
+// per tile and nothing staged (us, this / the best staged form below, copies
+// of the operands included; 8192 x 3001, B as [K, N] and as [N, K]: bf16 K = 3
+// 17.1 / 23.5 and 15.7 / 23.4, K = 15 18.3 / 24.0 and 23.7 / 23.7; fp32 K = 3 20.6 /
+// 25, K = 15 26 / 30.6 and 30 / 32.6).  With a K of whole 32-byte sectors its
+// strided loads collide (fp32 K = 16 36 / 27.4).  Within a round of tiles the
+// staged kernels are level.
+template <typename T, bool BT>
+static bool unstaged(const GemmArgs& a, int batch) {
+  const int lim = BT ? (sizeof(T) == 4 ? 17 : 12) : 20;
+  return a.K <= lim && a.K > 0 && (a.K % 8 || (!BT && sizeof(T) == 2 && a.K == 8)) && !dma_ok<T, BT>(a) &&
+         tiles_of(a, sizeof(T) == 4 ? 32 : 64, 64, batch) > 256 && tiles_of(a, 32, 32, 1) * 64 < kMaxGridThreads - 256;
+}
+
 // One product (or a batch of them) into C, by the kernel its operands allow.
 template <typename T, typename TO, bool BT>
 static void gemm_launch(const GemmArgs& a, int batch, hipStream_t st) {
-  if (dma_ok<T, BT>(a)) {
+  if (unstaged<T, BT>(a, batch)) return launch_naive<T, TO, BT>(a, batch, st);
+  const bool dma = dma_ok<T, BT>(a);
+  if constexpr (sizeof(T) == 4) {
+    // fp32 with a short K and more than a round of tiles: the LDS-DMA kernel's
+    // one workgroup a CU leaves its prologue and stores bare, where up to five
+    // of the register-staged kernel's share one (us, DMA / this; B as [K, N]
+    // and [N, K], 8192 x 4096: K = 4 72 / 30 and 72 / 31, K = 16 73 / 34 and 72 /
+    // 34, K = 32 73 / 41 and 73 / 40, K = 48 74 / 66 and 73 / 63, K = 128 105 / 90
+    // and 104 / 88, K = 384 230 / 209 and 229 / 208).  Aligned products past 32 keep
+    // the LDS-DMA kernel's sums over even and odd K-steps.
+    if (tiles_of(a, 32, 64, batch) > 256 && a.K > 0) {
+      if (dma ? a.K <= 32 : a.K < 64 && (a.K - 1) % 32 < 24)
+        return launch_reg<T, TO, BT, 64, 64, 2, 2, 1, 1, 1, true>(a, batch, st);
+      if (dma && a.K <= 384) {
+        if (a.N <= 64)
+          launch_reg<T, TO, BT, 64, 64, 2, 2, 1, 1, 2>(a, batch, st);
+        else
+          launch_reg<T, TO, BT, 64, 128, 2, 4, 1, 2, 2>(a, batch, st);
+        return;
+      }
+    }
+  }
+  if (dma) {
     GemmArgs g = a;
     g.epi = staged_ok<TO>(a) ? kEpiStaged : kEpiElem;
     if constexpr (sizeof(T) == 4)
@@ -1286,8 +1351,11 @@ static WsPlan plan_ws(const GemmArgs& a) {
   // 202 -> 146 us, 3001 x 1001 x 3003 45 -> 40; below that it depends on K: 4001 x
   // 129 x 1001, 256 tiles, 9 -> 13, 2047 x 1023 x 2049, 272 tiles, 31 -> 28); the
   // fp32 kernels are close enough to each other that it does not.  Nor does it
-  // where the copies would still not suit the LDS-DMA kernel (2 GiB or more).
-  if (sizeof(T) == 2 && !dma_ok<T, BT>(a) && tiles_of(a, 128, 128, 1) >= 512) {
+  // where the copies would still not suit the LDS-DMA kernel (2 GiB or more), or
+  // where one row or column of tiles reads each copy once (65536 x 65 x 33 20.4
+  // with copies, 8.8 without; x 129 23.9 / 20.5, x 513 42.5 / 54.1).
+  if (sizeof(T) == 2 && !dma_ok<T, BT>(a) && tiles_of(a, 128, 128, 1) >= 512 && min(a.M, a.N) > 128 &&
+      !unstaged<T, BT>(a, 1)) {
     const bool pa = !aligned16(a.A) || a.K % E || a.lda % E;  // (K off a vector: zeros in A, and in B^T)
     const bool pb = !aligned16(a.B) || a.ldb % E || (BT ? a.K % E : a.N % E);
     const int kp = (int)(((long)a.K + E - 1) / E * E), np = BT ? a.N : (int)(((long)a.N + E - 1) / E * E);
@@ -1331,8 +1399,7 @@ struct Workspace {
 template <typename T, typename TO, bool BT>
 static int gemm_dispatch(const GemmArgs& a, int batch, int variant, Workspace ws, hipStream_t st) {
   if (variant == NKL_GEMM_NAIVE) {
-    const long tiles = (long)((a.M + 31) / 32) * ((a.N + 31) / 32);
-    gemm_naive_kernel<T, TO, BT><<<dim3((unsigned)((tiles + 3) / 4), 1, batch), dim3(256), 0, st>>>(a);
+    launch_naive<T, TO, BT>(a, batch, st);
     return check_launch("nkl_gemm(naive)");
   }
   if (ws.use) {  // (batch 1)

@@ -399,34 +399,34 @@ def test_gemm_odd_columns_past_2_gib(M, K, N):
             assert ((cb[m:min(m + step, M), :N].float() - want).abs() <= bound).all(), (m, res is not None)
 
 
-@pytest.mark.parametrize("layout", ["nt", "nn"])
+@pytest.mark.parametrize("K", [1, 13])  # nothing staged; staged through registers
 @pytest.mark.parametrize("columns", [False, True])
-def test_gemm_tiles_past_one_launch(layout, columns):
-    """One column (or row) of more elements than the tiles of one launch hold
-    (HIP's limit of 2^32 threads): each an exact product of two bf16 values plus
-    the residual, rounded in fp32 and then to bf16, on both sides."""
+def test_gemm_tiles_past_one_launch(K, columns):
+    """One column (or row) of more elements than the 64x64 tiles of one launch
+    hold (HIP's limit of 2^32 threads), with a residual: multiples of 1/8 below
+    16, whose products and sums fp32 holds exactly, rounded once to bf16."""
     from nkilab import ops
 
     n = (1 << 30) + 65
     torch.cuda.empty_cache()
     free = torch.cuda.mem_get_info()[0]
-    if free < 24 << 30:
-        pytest.skip(f"needs 24 GiB of GPU memory, {free >> 30} free")
-    x = torch.empty(n, dtype=torch.bfloat16, device="cuda").normal_()
-    s = torch.full((1, 1), 1.75, dtype=torch.bfloat16, device="cuda")
-    r = torch.empty(n, dtype=torch.bfloat16, device="cuda").normal_()
+    if free < 64 << 30:
+        pytest.skip(f"needs 64 GiB of GPU memory, {free >> 30} free")
+
+    def eighths(*shape):
+        return torch.empty(shape, dtype=torch.bfloat16, device="cuda").random_(-127, 128).mul_(0.125)
+
+    x, s, r = eighths(n, K), eighths(1, K), eighths(n)
     c = torch.full((n + 8,), 5.0, dtype=torch.bfloat16, device="cuda")
     shape = (1, n) if columns else (n, 1)
-    a, b = (s, x.view(shape)) if columns else (x.view(shape), s)
-    if layout == "nt":
-        ops.linear_into(a, b.view(b.shape[1], 1), c[:n].view(shape), residual=r.view(shape))
-    else:
-        ops.gemm_into(a, b, c[:n].view(shape), residual=r.view(shape))
-    step = 1 << 28
+    ops.linear_into(*((s, x) if columns else (x, s)), c[:n].view(shape), residual=r.view(shape))
+    step = 1 << 27
     for i in range(0, n, step):
-        want = (x[i:i + step].float() * 1.75 + r[i:i + step].float()).bfloat16()
-        assert torch.equal(c[i:min(i + step, n)], want), i
+        want = (x[i:i + step].float() * s.float()).sum(1) + r[i:i + step].float()
+        assert torch.equal(c[i:min(i + step, n)], want.bfloat16()), i
     assert (c[n:] == 5).all()
+    del x, c, r
+    torch.cuda.empty_cache()
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
@@ -444,6 +444,18 @@ def test_gemm_without_memory_for_a_workspace(dt, M, K, N, monkeypatch):
     monkeypatch.setattr(ops, "workspace", none_left)
     test_gemm_any_shape_and_alignment(dt, M, K, N, 0)
     assert asked or (dt == torch.float32 and N > 64)  # (fp32 operands are not packed)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,N", [
+    (1030, 1, 1301), (1030, 12, 1301), (1030, 13, 1300), (1030, 17, 1301), (1030, 20, 1301), (1030, 21, 1301),
+    (1030, 8, 1301), (1030, 16, 1301), (2050, 24, 2049), (1030, 32, 1300), (1030, 33, 1301), (1030, 57, 1301),  # fp32
+    (1030, 36, 1300), (1030, 64, 1300), (1030, 100, 1300), (1030, 384, 1300), (16500, 100, 60), (1030, 388, 1300),
+    (65540, 70, 129), (65540, 70, 128)])                                             # 16 bits: packed, not packed
+def test_gemm_short_k(dt, M, K, N):
+    """Short K over more than a round of tiles: the unstaged kernel, one or two
+    checked K-steps, two sums, and the K on both sides of each choice."""
+    test_gemm_any_shape_and_alignment(dt, M, K, N, 0)
 
 
 def test_gemm_workspace_is_for_the_shapes_that_use_it():
