@@ -1240,18 +1240,17 @@ static void gemm_launch(const GemmArgs& a, int batch, hipStream_t st) {
     // of the register-staged kernel's share one (us, DMA / this; B as [K, N]
     // and [N, K], 8192 x 4096: K = 4 72 / 30 and 72 / 31, K = 16 73 / 34 and 72 /
     // 34, K = 32 73 / 41 and 73 / 40, K = 48 74 / 66 and 73 / 63, K = 128 105 / 90
-    // and 104 / 88, K = 384 230 / 209 and 229 / 208).  Aligned products past 32 keep
-    // the LDS-DMA kernel's sums over even and odd K-steps.
-    if (tiles_of(a, 32, 64, batch) > 256 && a.K > 0) {
-      if (dma ? a.K <= 32 : a.K < 64 && (a.K - 1) % 32 < 24)
-        return launch_reg<T, TO, BT, 64, 64, 2, 2, 1, 1, 1, true>(a, batch, st);
-      if (dma && a.K <= 384) {
-        if (a.N <= 64)
-          launch_reg<T, TO, BT, 64, 64, 2, 2, 1, 1, 2>(a, batch, st);
-        else
-          launch_reg<T, TO, BT, 64, 128, 2, 4, 1, 2, 2>(a, batch, st);
-        return;
-      }
+    // and 104 / 88, K = 384 230 / 209 and 229 / 208; past 32 with more than a round
+    // of the larger tiles only, 777 x 300 x 1024 10.2 / 15.1).  Aligned products
+    // past 32 keep the LDS-DMA kernel's sums over even and odd K-steps.
+    if (tiles_of(a, 32, 64, batch) > 256 && a.K > 0 && (dma ? a.K <= 32 : a.K < 64 && (a.K - 1) % 32 < 24))
+      return launch_reg<T, TO, BT, 64, 64, 2, 2, 1, 1, 1, true>(a, batch, st);
+    if (dma && a.K > 32 && a.K <= 384 && tiles_of(a, 64, a.N <= 64 ? 64 : 128, batch) > 256) {
+      if (a.N <= 64)
+        launch_reg<T, TO, BT, 64, 64, 2, 2, 1, 1, 2>(a, batch, st);
+      else
+        launch_reg<T, TO, BT, 64, 128, 2, 4, 1, 2, 2>(a, batch, st);
+      return;
     }
   }
   if (dma) {

@@ -450,7 +450,7 @@ def test_gemm_without_memory_for_a_workspace(dt, M, K, N, monkeypatch):
 @pytest.mark.parametrize("M,K,N", [
     (1030, 1, 1301), (1030, 12, 1301), (1030, 13, 1300), (1030, 17, 1301), (1030, 20, 1301), (1030, 21, 1301),
     (1030, 8, 1301), (1030, 16, 1301), (2050, 24, 2049), (1030, 32, 1300), (1030, 33, 1301), (1030, 57, 1301),  # fp32
-    (1030, 36, 1300), (1030, 64, 1300), (1030, 100, 1300), (1030, 384, 1300), (16500, 100, 60), (1030, 388, 1300),
+    (1030, 36, 1300), (2050, 36, 1300), (2050, 64, 1300), (2050, 384, 1300), (16500, 100, 60), (2050, 388, 1300),
     (65540, 70, 129), (65540, 70, 128)])                                             # 16 bits: packed, not packed
 def test_gemm_short_k(dt, M, K, N):
     """Short K over more than a round of tiles: the unstaged kernel, one or two
