@@ -24,6 +24,8 @@
 // K rows are swizzled by 16-byte chunks (chunk c of row r at c ^ swz(r)), which
 // keeps the 16-row reads free of bank conflicts; V reads are whole rows.
 //
+// (A second kernel further down takes many short heads.)
+//
 // Bound by the fp32 MFMAs (256 flop per clock and CU; a step is 8192 cycles of
 // them per SIMD, 3.5 of its 4.5 us): 16 x 2048 x 128 281 -> 171 us (101 TFLOP/s),
 // 8/2 x 4096 x 128 551 -> 320, 4 x 300 x 64 24.5 -> 10.9, against 64-query
@@ -320,11 +322,161 @@ __global__ __launch_bounds__(512) void flash_f32_kernel(AttnArgs p) {
   }
 }
 
+// The kernel for many short heads: one 256-thread workgroup per 64-query block
+// of a head, heaviest blocks first, four wavefronts of 16 queries each, steps of
+// 32 keys staged through registers into two padded stages (68 KB at D = 128, 35
+// at 64, 18 at 32), so that two, three or five workgroups share a CU and hide
+// each other's starts, waits and ends, and a ragged last step is half as long.
+// S^T and O^T as in the kernel above, one 4-byte LDS read per MFMA; a block's
+// state stays with its wavefronts, nothing is merged.  O is summed over every
+// fourth group of 16 keys apart, as the other kernel's key groups do: one sum is
+// up to 5% faster, at 128 x 2048 x 32 with 3.7e-7 from 64 bits where four, and the
+// other kernel, have 2.5e-7.
+template <int D>
+__global__ __launch_bounds__(256, D == 128 ? 2 : D == 64 ? 3 : 5) void flash_f32_short_kernel(AttnArgs p) {
+  constexpr int NC = 4;  // sums of O
+  constexpr int kQB = 64, kKS = 32, CPR = D / 4, LD = D + 4, NCH = kKS * CPR / 256, ND = D / 16, NQF = D / 4;
+  __shared__ float Ks[2][kKS * LD];
+  __shared__ float Vs[2][kKS * LD];
+
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int g = lane >> 4, r = lane & 15;
+  const int S = p.S;
+
+  const int nqb = (S + kQB - 1) / kQB;
+  const int h = blockIdx.x % p.H;
+  const int q0 = (nqb - 1 - blockIdx.x / p.H) * kQB;
+  const int qw = q0 + 16 * w, q = qw + r;  // this wavefront's first query, this lane's query
+  const float* Q = static_cast<const float*>(p.q) + (long)h * p.q_sh;
+  const float* K = static_cast<const float*>(p.k) + (long)(h / p.group) * p.k_sh;  // shared K/V head (GQA)
+  const float* V = static_cast<const float*>(p.v) + (long)(h / p.group) * p.v_sh;
+  float* O = static_cast<float*>(p.o) + (long)h * p.o_sh;
+
+  // Q^T: lane (r, g) holds Q[q][4 f + g].
+  float qf[NQF];
+#pragma unroll
+  for (int f = 0; f < NQF; ++f) qf[f] = q < S && 4 * f + g < p.d ? Q[(long)q * p.q_ss + 4 * f + g] : 0.f;
+
+  uint4 rk[NCH], rv[NCH];
+  auto gload = [&](int k0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      const int c = tid + 256 * i, key = k0 + c / CPR, cc = (c % CPR) * 4;
+      rk[i] = ld16_or_zero(K, (long)key * p.k_ss + cc, key < S && cc < p.d);
+      rv[i] = ld16_or_zero(V, (long)key * p.v_ss + cc, key < S && cc < p.d);
+    }
+  };
+  auto lstore = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      const int c = tid + 256 * i, at = c / CPR * LD + (c % CPR) * 4;
+      *reinterpret_cast<uint4*>(&Ks[buf][at]) = rk[i];
+      *reinterpret_cast<uint4*>(&Vs[buf][at]) = rv[i];
+    }
+  };
+
+  float m = -INFINITY, l[2] = {0.f, 0.f};  // l: this lane's share
+  floatx4 o[NC][ND];
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int b = 0; b < ND; ++b) o[c][b] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+  const int ns = (min(q0 + kQB, S) - 1) / kKS + 1;  // steps up to the diagonal
+  const int q_last = qw + 15;
+  gload(0);
+  lstore(0);
+  __syncthreads();
+  auto step = [&](int s, int buf) __attribute__((always_inline)) {
+    const int k0 = s * kKS;
+    if (s + 1 < ns) gload(k0 + kKS);
+    // S^T = K . Q^T, element i of sc[kb] for key k0 + 16 kb + 4 g + i; the
+    // 16-key groups past the wavefront's last query are left out.
+    floatx4 sc[2];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      sc[kb] = floatx4{0.f, 0.f, 0.f, 0.f};
+      if (k0 + 16 * kb <= q_last) {
+#pragma unroll
+        for (int f = 0; f < NQF; ++f)
+          sc[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(Ks[buf][(16 * kb + r) * LD + 4 * f + g], qf[f], sc[kb], 0, 0, 0);
+      }
+    }
+    const bool diag = k0 + kKS - 1 > qw;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float x = diag && k0 + 16 * kb + 4 * g + i > q ? -INFINITY : sc[kb][i] * p.c;
+        sc[kb][i] = x;
+        mx = fmaxf(mx, x);
+      }
+    const float mn = fmaxf(m, max_xor32(max_xor16(mx)));
+    // (no key yet: m is -inf, l and O are 0; every key masked so far: p = 0)
+    const float mu = mn == -INFINITY ? 0.f : mn;
+    if (__any(mn > m)) {
+      const float corr = m == -INFINITY ? 0.f : fast_exp2(m - mn);
+      l[0] *= corr, l[1] *= corr;
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int b = 0; b < ND; ++b) o[c][b] *= corr;
+      m = mn;
+    }
+    float sum = 0.f;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        sc[kb][i] = fast_exp2(sc[kb][i] - mu);
+        sum += sc[kb][i];
+      }
+    l[buf] += sum;
+    // O^T += V^T . P^T
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      if (k0 + 16 * kb > q_last) continue;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int b = 0; b < ND; ++b)
+          o[2 * buf + kb][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              Vs[buf][(16 * kb + 4 * g + i) * LD + 16 * b + r], sc[kb][i], o[2 * buf + kb][b], 0, 0, 0);
+    }
+    if (s + 1 < ns) lstore(buf ^ 1);
+    __syncthreads();
+  };
+#pragma unroll 1
+  for (int s = 0; s < ns; s += 2) {
+    step(s, 0);
+    if (s + 1 < ns) step(s + 1, 1);
+  }
+
+  const float linv = 1.0f / sum_xor32(sum_xor16(l[0] + l[1]));
+  if (q < S) {
+    float* orow = O + (long)q * p.o_ss;
+#pragma unroll
+    for (int b = 0; b < ND; ++b) {
+      const int d = 16 * b + 4 * g;
+      float v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v[i] = o[0][b][i];
+#pragma unroll
+        for (int c = 1; c < NC; ++c) v[i] += o[c][b][i];
+        v[i] *= linv;
+      }
+      if (d < p.d) store_vec<4>(orow + d, v);
+    }
+  }
+}
+
 // One launch over all heads, unless their threads pass HIP's limit: then
 // over ranges of heads, each of whole groups or within one group.
-template <int D, int NHF>
-static void launch_heads(const AttnArgs& a, hipStream_t st) {
-  const long nqb = ((long)a.S + 32 * NHF - 1) / (32 * NHF), fit = kMaxGridThreads / 512 / nqb;
+template <typename F>
+static void launch_heads(const AttnArgs& a, int qb, int threads, F kernel, hipStream_t st) {
+  const long nqb = ((long)a.S + qb - 1) / qb, fit = kMaxGridThreads / threads / nqb;
   for (long h = 0, n; h < a.H; h += n) {
     n = min(fit > 1 ? fit : 1, a.H - h);
     AttnArgs p = a;
@@ -340,8 +492,30 @@ static void launch_heads(const AttnArgs& a, hipStream_t st) {
     p.k = static_cast<const float*>(a.k) + h / a.group * a.k_sh;
     p.v = static_cast<const float*>(a.v) + h / a.group * a.v_sh;
     p.o = static_cast<float*>(a.o) + h * a.o_sh;
-    flash_f32_kernel<D, NHF><<<dim3((unsigned)(nqb * n)), dim3(512), 0, st>>>(p);
+    kernel<<<dim3((unsigned)(nqb * n)), dim3(threads), 0, st>>>(p);
   }
+}
+
+// Whether the kernel for many short heads leads the 64-query one: by the heads,
+// which with short sequences are the rounds of workgroups, up to the length
+// where the 64-query kernel's steps win them back (heads x positions, us, short /
+// 64-query).
+// d <= 32: at any length from enough blocks on: 256 x 200 17.2 / 19.3, 1024 x 64
+// 11.1 / 12.1, 8192 x 16 31 / 68, 96 x 900 68 / 70, 128 x 2048 343 / 377, 32 x 6000
+// 714 / 766; but 256 x 128 9.7 / 8.8, 128 x 512 32 / 31, 32 x 4096 375 / 363.
+// d <= 64: 512 x 100 23 / 25, 384 x 200 44 / 46, 1024 x 384 231 / 236, 4096 x 16 31 /
+// 57, 640 x 64 15.6 / 17.5; but 320 x 200 level, 512 x 64 12.6 / 12.0, 1024 x 600 575
+// / 570.
+// d <= 128: 1024 x 16 18.5 / 34, 256 x 100 24 / 31, 144 x 200 42 / 47, 256 x 800 498 /
+// 524; but 128 x 100 19.4 / 16.6, 256 x 1024 level.  With somewhat fewer heads where
+// the 64-query kernel's last step would be half empty, and past 256: 128 x 200 35 /
+// 41, 128 x 300 52 / 59, but 128 x 256 41.7 / 40.9.
+template <int D>
+static bool many_short(int H, int S) {
+  const long blocks = (long)H * ((S - 1) / 64 + 1);
+  if (D == 32) return blocks >= (H >= 256 ? 768 : H >= 64 ? 1400 : 2200);
+  if (D == 64) return H >= 384 && S <= (H >= 512 ? 384 : 300) && (S <= 32 || S > 64 || H >= 640);
+  return (H >= 144 && S <= 800) || (H >= 112 && S > 128 && S <= 384 && ((S - 1) % 64 < 32 || S > 256));
 }
 
 template <int D>
@@ -351,9 +525,11 @@ static void launch(const AttnArgs& a, hipStream_t st) {
   // 128 290 / 161, 2 x 100 x 128 15.7 / 9.5).
   const long n64 = ((long)a.S + 63) / 64;
   if (n64 * a.H <= 128)
-    launch_heads<D, 1>(a, st);
+    launch_heads(a, 32, 512, flash_f32_kernel<D, 1>, st);
+  else if (many_short<D>(a.H, a.S))
+    launch_heads(a, 64, 256, flash_f32_short_kernel<D>, st);
   else
-    launch_heads<D, 2>(a, st);
+    launch_heads(a, 64, 512, flash_f32_kernel<D, 2>, st);
 }
 
 int flash_f32_launch(const AttnArgs& a, hipStream_t st) {

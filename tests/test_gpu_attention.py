@@ -525,10 +525,32 @@ def test_flash_fp32_against_float64(H, Hkv, S, d, scale):
     assert (ob[:, S] == 7).all()
 
 
-@pytest.mark.parametrize("H,Hkv", [((1 << 23) + 3, (1 << 23) + 3), (3 * 2796204, 2796204), ((1 << 23) + 2, 2),
-                                   ((1 << 23) + 2, 1)])
+@pytest.mark.parametrize("H,Hkv,S,d,scale", [
+    (130, 130, 1, 4, None), (135, 45, 16, 32, None), (70, 70, 65, 32, 4.0), (9, 3, 1027, 28, -0.3),
+    (132, 132, 63, 36, None), (130, 65, 64, 64, -0.3), (68, 68, 127, 64, 4.0), (46, 23, 129, 64, None),
+    (9, 9, 1027, 64, None), (66, 33, 65, 100, None), (70, 70, 128, 128, None), (45, 15, 191, 96, None),
+    (22, 22, 321, 128, 3.0), (33, 11, 256, 128, -0.1)])
+def test_flash_fp32_64_query_blocks(H, Hkv, S, d, scale):
+    """The same edges on launches of more than 128 blocks of 64 queries, which
+    keep them whole."""
+    test_flash_fp32_against_float64(H, Hkv, S, d, scale)
+
+
+@pytest.mark.parametrize("H,Hkv,S,d,scale", [
+    (1400, 1400, 1, 4, None), (1024, 512, 33, 32, None), (256, 128, 129, 28, 4.0), (256, 256, 192, 32, -0.3),
+    (384, 384, 31, 64, None), (640, 160, 63, 64, None), (384, 128, 100, 36, 4.0), (256, 256, 130, 64, -0.3),
+    (144, 48, 1, 128, None), (144, 48, 63, 128, None), (150, 50, 191, 96, 3.0), (112, 28, 200, 128, None),
+    (112, 112, 321, 100, -0.1)])
+def test_flash_fp32_many_short_heads(H, Hkv, S, d, scale):
+    """The same edges on launches of many short heads, whose kernel takes keys
+    in steps of 32."""
+    test_flash_fp32_against_float64(H, Hkv, S, d, scale)
+
+
+@pytest.mark.parametrize("H,Hkv", [((1 << 24) + 3, (1 << 24) + 3), (3 * 5592407, 5592407), ((1 << 24) + 2, 2),
+                                   ((1 << 24) + 2, 1)])
 def test_flash_fp32_heads_past_one_launch(H, Hkv):
-    """More heads than one launch of 512 threads a head takes (HIP's limit of
+    """More heads than one launch of 256 threads a head takes (HIP's limit of
     2^32 threads), alone and in groups of 3, of half of them and of all: at one
     position each query's output is its head's value."""
     from nkilab import ops
@@ -556,3 +578,23 @@ def test_flash_fp32_with_infinite_scores():
     s.masked_fill_(torch.ones(S, S, dtype=torch.bool, device="cuda").triu(1), -float("inf"))
     ref = torch.matmul(torch.softmax(s[:, :150, :150], -1), v[:, :150].double())
     assert (o[:, 1:150].double() - ref[:, 1:]).abs().max().item() <= 1e-5
+
+
+@pytest.mark.parametrize("H,d", [(65, 64), (65, 128), (520, 20), (400, 64), (112, 128)])
+def test_flash_fp32_with_infinite_scores_on_many_blocks(H, d):
+    """The same on 64-query blocks and in the kernel for many short heads (the
+    last three), with the first 40 keys at -inf: more than one step of it."""
+    from nkilab import ops
+
+    S = 200
+    q, k, v = (torch.randn(H, S, d, device="cuda") for _ in range(3))
+    q[-1].abs_().add_(0.1)  # (so that the scores below are infinite and of one sign)
+    k[-1, :40] = -float("inf")
+    k[-1, 150] = float("nan")
+    o = ops.attention(q, k, v)
+    s = torch.matmul(q.double(), k.double().transpose(1, 2).contiguous()) * d ** -0.5
+    s.masked_fill_(torch.ones(S, S, dtype=torch.bool, device="cuda").triu(1), -float("inf"))
+    ref = torch.matmul(torch.softmax(s[:, :150, :150], -1), v[:, :150].double())
+    assert torch.isnan(o[-1, :40]).all() and torch.isnan(o[-1, 150:]).all()
+    assert (o[:-1, :150].double() - ref[:-1]).abs().max().item() <= 1e-5
+    assert (o[-1, 40:150].double() - ref[-1, 40:]).abs().max().item() <= 1e-5
