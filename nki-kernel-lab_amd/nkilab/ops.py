@@ -180,6 +180,9 @@ def gemm_swiglu_into(a: torch.Tensor, w_gu: torch.Tensor, c: torch.Tensor) -> to
     return c
 
 
+FP32_SPLIT_K = 1505  # the shortest K nkl_gemm_ws splits over workgroups in fp32 (48 K-steps of 32, begun)
+
+
 def _splits_k(a: torch.Tensor, w: torch.Tensor, M: int, N: int, K: int) -> bool:
     """Whether a @ w^T splits its K over workgroups.  The one gate/up GEMM does
     not, and its longer sums cost precision there (16 x 4064 x 2048: 23.5 us
@@ -199,7 +202,7 @@ def gate_up_into(a: torch.Tensor, wg: torch.Tensor, wu: torch.Tensor, c: torch.T
                          f"{tuple(c.shape)} do not match")
     if (a.dtype == wg.dtype == wu.dtype == c.dtype == torch.float32 and M > 0 and K > 0
             and a.stride(1) == wg.stride(1) == wu.stride(1) == c.stride(1) == 1
-            and (K <= 1504 or not _splits_k(a, wg, M, N, K))):
+            and (K < FP32_SPLIT_K or not _splits_k(a, wg, M, N, K))):
         rc = _lib.lib().nkl_gemm_gate_up(a.data_ptr(), wg.data_ptr(), wu.data_ptr(), c.data_ptr(), M, N, K, a.stride(0),
                                          wg.stride(0), wu.stride(0), c.stride(0), _lib.F32, stream_handle())
         if rc == 0:

@@ -265,6 +265,13 @@ def test_gate_up_fp32(M, K, N, off):
     assert (cb[:, :4] == 5).all() and (cb[:, N + 4:] == 5).all()
 
 
+@pytest.mark.parametrize("M,K,N", [(16, 1504, 2048), (16, 1508, 2048), (16, 4064, 2048), (200, 2048, 1024)])
+def test_gate_up_fp32_around_the_k_split(M, K, N):
+    """The last K taken by one GEMM whatever the tiles, the first whose two
+    GEMMs split it, longer ones with and without a split."""
+    test_gate_up_fp32(M, K, N, 0)
+
+
 def test_gemm_swiglu_rejects_bad_shapes():
     from nkilab import ops
 

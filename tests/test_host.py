@@ -108,6 +108,18 @@ def test_gemm_swiglu_abi_checks():
     assert L.nkl_gemm_swiglu(None, None, None, 0, 64, 64, 64, 64, 64, 1, None) == 0   # empty
 
 
+def test_gate_up_knows_where_k_is_split():
+    """The shortest K that gate_up_into asks the library about is the shortest
+    that fp32 products split, aligned or not."""
+    from nkilab import _lib, ops
+
+    p = 1 << 20  # (an aligned address, never used)
+    need = lambda m, n, k: _lib.lib().nkl_gemm_workspace_bytes(p, p, m, n, k, k, k, 1, 0, 0)  # noqa: E731
+    for m, n in ((1, 64), (16, 2048), (100, 500), (128, 1024)):
+        assert all(need(m, n, k) == 0 for k in range(4, ops.FP32_SPLIT_K, 4)) and need(m, n, ops.FP32_SPLIT_K - 1) == 0
+        assert need(m, n, ops.FP32_SPLIT_K) > 0 and need(m, n, ops.FP32_SPLIT_K + 3) > 0
+
+
 def test_gemm_gate_up_abi_checks():
     from nkilab import _lib
 
