@@ -1446,35 +1446,55 @@ Work plan(int H, int S, Config cfg) {
 // one-wavefront-per-SIMD kernels and kFwd take 64 < d <= 128 and fix the block.
 
 // The choice for d <= 64, whose tiles are short next to a workgroup's start,
-// hand-over and merge: 64-query blocks throughout, and no schedule that splits
-// a block once a round of workgroups is full.  Sweep over 1 to 64 heads x 64 to
-// 8192 positions, inputs rotated through twice the last-level cache, us at
-// d = 64 (d = 32), this rule / the 128-query rule above:
-//   up to 384 positions, or more than 640 blocks, or more than a round of
-//   blocks up to 1024 positions: one four-wavefront workgroup per block, two
-//   or more a CU, whose starts and ends hide each other's: 8 x 128 5.8 / 6.6
-//   (5.4 / 6.1), 4 x 300 7.9 / 8.3, 64 x 300 8.6 / 16.2 (7.6 / 14.6), 32 x 768
-//   13.2 / 17.0, 32 x 1024 16.5 / 17.9, 32 x 1537 24.6 / 33.9 (19.1 / 30.6),
-//   32 x 2048 33.6 / 38.3 (24.7 / 34.6), 16 x 4096 56 / 63 (42 / 58),
-//   32 x 4096 105 / 119 (74 / 113);
-//   other launches of more than a round: eight wavefronts per block, 8 x 3000
-//   25.9 / 29.0, 16 x 1537 20.6 / 22.5 (16.0 / 20.3); per pair of blocks when
-//   the pairs fill the CUs (d > 32), 16 x 2048 23.7 / 24.8, 8 x 4096 36.9 /
-//   37.7, where blocks take 26.4 and 40 (at d = 32 blocks lead, 19.4 / 22.7);
-//   within a round: eight wavefronts per block while the heaviest block
-//   exceeds a balanced range by at most 18 tiles, as in the rule above, else
-//   balanced ranges, 8 x 2048 17.4 / 19.0, 4 x 4096 24.5 / 25.4.
-Config choose_narrow(int H, int S, int d) {
-  const long cus = cu_count();
-  const long n64 = ((long)S + 63) / 64, blocks = (long)H * n64;
-  if (S <= 384 || blocks > cus * 5 / 2 || (blocks > cus && S <= 1024)) return Config{64, kBlock, kTeams4};
-  if (blocks > cus) {
-    const long pairs = (long)H * ((n64 + 1) / 2);
-    return Config{64, d > 32 && pairs <= cus && pairs * 5 >= cus * 4 ? kPairs : kBlock, kTeams};
+// hand-over and merge: 64-query blocks, each a workgroup's own, unless the
+// heaviest ones outlast a balanced share of the work by more than splitting
+// costs; then `wide`, the rule above (us at d = 64, inputs rotated through twice
+// the last-level cache, this rule / the wide rule or the alternative named;
+// d = 32 in brackets).
+//   Up to 384 positions, or more than a round of blocks up to 1024: one
+//   four-wavefront workgroup per block, two or more a CU, whose starts and ends
+//   hide each other's: 8 x 128 5.8 / 6.6 (5.4 / 6.1), 4 x 300 7.9 / 8.3, 64 x 300
+//   8.6 / 16.2 (7.6 / 14.6), 32 x 768 13.2 / 17.0, 32 x 1024 16.5 / 17.9.
+//   Within a round: eight wavefronts per block while the heaviest block exceeds
+//   a balanced range by at most 18 tiles, as in the rule above, else balanced
+//   ranges, 8 x 2048 17.4 / 19.0, 4 x 4096 24.5 / 25.4, level at 1 x 12000 and for
+//   d > 32 wide past it, 1 x 16384 61 wide / 64 (58 / 57).
+//   From one round to two: eight wavefronts per block, 8 x 3000 26.4 / 29.9 (23.5 /
+//   25.3), 12 x 2112 22.8 / 25.5 (18.3 / 22.4).  The heaviest block, n64 tiles of 64
+//   keys, takes 0.4 us a tile where a CU's share is n64 blocks / (2 CUs) tiles and
+//   splitting costs 8 us, or 20 tiles: level at 7 x 2500 (18 tiles apart) 23.0 /
+//   22.7, past there 6 x 3000 (21) 24.7 wide, 26.1 blocks, 5 x 4096 (24) 30.3 / 33.0
+//   (27.1 / 30.4), 3 x 6000 36 / 44 (32 / 40), 1 x 20000 88 / 132 (84 / 120).
+//   d > 32, per pair of blocks when the pairs nearly fill the CUs: pairs / blocks
+//   12 x 2112, 204 pairs, 23.9 / 22.8, 16 x 1537, 208, 20.9 / 20.5, 14 x 1920, 210,
+//   22.7 / 22.9, 16 x 1800, 240, 22.6 / 23.8 (20.1 / 17.3); pairs / wide 9 x 3500,
+//   252, 33.1 / 36.4.  A pair takes 0.43 us a tile; from 6 us over the share on, 6 x
+//   4700 39.7 wide / 40.6 pairs, 5 x 5400 42.4 / 45.2, 4 x 8100 59.5 / 62.3, and at one
+//   pair a CU, 16 x 2048 23.1 / 23.7, 8 x 4096 35.2 / 36.6, 2 x 16384 111 / 120, wide
+//   leads (d = 32 keeps blocks: 16 x 2048 18.8 / 21.7, 4 x 8100 52 / 57); more pairs
+//   than CUs are blocks again, 24 x 1323 21.6 / 24.8 wide.
+//   From two rounds: four-wavefront workgroups again (d <= 32: from 640 blocks,
+//   eight wavefronts a block below, 17 x 2000 (19.4 / 23.5)), 18 x 2048 27.3 / 30.0,
+//   20 x 2040 28 / 31.5, 12 x 4096 51.2 / 52.7, 24 x 2048 29 / 35 (24 / 32), 8 x 8192 104
+//   / 110 (79 / 106).  At 0.7 us a tile, two to a CU, their heaviest block outlasts
+//   the share by more than 9.5 us at 9 x 4000 43.5 wide / 47.8, 5 x 8000 76 / 89, 6 x
+//   8192 89 / 95, 3 x 16384 165 / 185 (d = 32 leads there too, 78 / 86, 142 / 158).
+Config choose_narrow(int H, int S, int d, long cus, Config wide) {
+  const long n64 = ((long)S + 63) / 64, blocks = (long)H * n64, pairs = (long)H * ((n64 + 1) / 2);
+  if (S <= 384 || (blocks > cus && S <= 1024)) return Config{64, kBlock, kTeams4};
+  if (blocks <= cus) {
+    const long units = (long)H * (n64 * (n64 - 1) + (S - 1) / BN + 1);
+    const long range = units / cus > kMinUnits ? units / cus : kMinUnits;
+    if (d > 32 && n64 > cus * 3 / 4) return wide;
+    return Config{64, (S - 1) / BN + 1 <= range + 18 ? kBlock : kBalanced, kTeams};
   }
-  const long units = (long)H * (n64 * (n64 - 1) + (S - 1) / BN + 1);
-  const long range = units / cus > kMinUnits ? units / cus : kMinUnits;
-  return Config{64, (S - 1) / BN + 1 <= range + 18 ? kBlock : kBalanced, kTeams};
+  if (blocks <= 2 * cus) {
+    if (d > 32 && pairs * 5 >= cus * 4 && pairs <= cus)
+      return pairs < cus && n64 * (cus * 113 / 50 - blocks) < 32 * cus ? Config{64, kPairs, kTeams} : wide;
+    return n64 * (2 * cus - blocks) < 40 * cus ? Config{64, kBlock, kTeams} : wide;
+  }
+  if (d <= 32) return Config{64, kBlock, blocks > cus * 5 / 2 ? kTeams4 : kTeams};
+  return n64 * (cus * 92 / 25 - blocks) < 50 * cus ? Config{64, kBlock, kTeams4} : wide;
 }
 
 Config choose(int H, int S, int d, bool f16) {
@@ -1532,7 +1552,7 @@ Config choose(int H, int S, int d, bool f16) {
     cfg = Config{128, kBlock, kTiny};
   // (Past HIP's limit on threads a launch, the pairs of 128-query blocks above,
   // which are up to half as many threads.)
-  if (d <= 64 && (long)H * (((long)S + 63) / 64) * 256 <= kMaxGridThreads) cfg = choose_narrow(H, S, d);
+  if (d <= 64 && (long)H * (((long)S + 63) / 64) * 256 <= kMaxGridThreads) cfg = choose_narrow(H, S, d, cus, cfg);
   const Overrides& ov = overrides();
   if (ov.sched >= 0) cfg.sched = ov.sched;
   if (ov.qb >= 0) cfg.qb = ov.qb;
@@ -1617,7 +1637,9 @@ size_t flash_bf16_workspace_bytes(int H, int S, int d, bool f16) {
 // block) whenever some head dim takes the balanced schedule for this shape.
 size_t flash_bf16_counter_bytes(int H, int S) {
   if (H <= 0 || S <= 0) return 0;
-  if (choose(H, S, 32, false).sched != kBalanced && choose(H, S, 128, false).sched != kBalanced) return 0;
+  if (choose(H, S, 32, false).sched != kBalanced && choose(H, S, 64, false).sched != kBalanced &&
+      choose(H, S, 128, false).sched != kBalanced)
+    return 0;
   return (size_t)H * ((S + 63) / 64) * 4;
 }
 

@@ -484,6 +484,49 @@ def test_kernel_choice_rules():
     assert plan(16, 4096)[1] == 16 * 2112 // 2                      # 132 units per CU: ping-pong
 
 
+def test_narrow_head_choice_rules():
+    """Head dims up to 64 at the boundaries their rule was measured at (a 256-CU
+    device).  Workgroups and units (32-key tiles) tell 64-query blocks, one or a
+    pair of them a workgroup, from balanced 64- or 128-query ranges; d = 64 and 32
+    differ where noted.  The 128-query rule is that of d = 128."""
+    from nkilab import _lib
+
+    _lib.flash_configure()
+    _lib.flash_configure_polls()
+    plan = _lib.flash_plan_check
+
+    def kind(H, S, d):
+        n = -(-S // 64)
+        grid, units, split, _, polls = plan(H, S, d)
+        u64, nq = H * (n * (n - 1) + (S - 1) // 32 + 1), -(-S // 128)
+        u128 = H * (2 * (nq - 1) * nq + (S - 1) // 32 + 1)
+        if polls == -1:
+            return {H * n: "block", H * ((n + 1) // 2): "pairs"}[grid] if units == u64 else "wide pairs"
+        return {u64: "balanced", u128: "wide"}[units]
+
+    for d in (8, 32, 40, 64):
+        pair = "pairs" if d > 32 else "block"
+        assert kind(64, 300, d) == kind(32, 768, d) == kind(32, 1024, d) == "block"  # short, or short and many
+        assert kind(14, 1024, d) == "block" and kind(4, 4096, d) == "balanced"       # within a round
+        assert kind(8, 3000, d) == kind(12, 2112, d) == kind(7, 2500, d) == "block"  # one round to two: 192, 204 pairs
+        assert kind(16, 1537, d) == kind(14, 1920, d) == kind(9, 3500, d) == pair    # 208, 210, 252 pairs
+        assert kind(6, 3000, d) == kind(5, 4096, d) == kind(3, 6000, d) == kind(1, 20000, d) == "wide"
+        assert kind(6, 4700, d) == kind(5, 5400, d) == ("wide" if d > 32 else "block")
+        assert kind(1, 12000, d) == "balanced" and kind(1, 16384, d) == ("wide" if d > 32 else "balanced")
+        assert kind(24, 1323, d) == "block"                                            # 504 blocks, 264 pairs
+        full = "wide" if d > 32 else "block"
+        assert kind(16, 2048, d) == kind(8, 4096, d) == kind(4, 8100, d) == kind(2, 16384, d) == full
+        assert kind(32, 1100, d) == kind(18, 2048, d) == kind(20, 2040, d) == "block"  # two rounds and more
+        assert kind(12, 4096, d) == kind(24, 2048, d) == kind(8, 8192, d) == "block"
+        assert kind(9, 4000, d) == kind(5, 8000, d) == kind(6, 8192, d) == kind(3, 16384, d) == full
+    # Scratch and counters come together, whatever the head dim.
+    L = _lib.lib()
+    for H, S in ((1, 20000), (2, 16384), (4, 8100), (9, 4000), (6, 8192), (4, 4096), (16, 2048), (8, 3000)):
+        for d in (32, 64, 128):
+            if L.nkl_flash_attn_causal_workspace_bytes(H, S, d, 1):
+                assert L.nkl_flash_attn_causal_counter_bytes(H, S, 1) == H * -(-S // 64) * 4
+
+
 def test_narrow_head_launch_fits_the_thread_limit():
     """Head dims up to 64: one four-wavefront workgroup per 64-query block up to
     HIP's limit of 2^32 threads a launch (16.8M of those), then one
