@@ -75,12 +75,14 @@ const char* nkl_last_error_string(void);
  * dtype_out.  dtype_in in {F32, BF16, F16}; dtype_out in {F32, dtype_in}.
  * The LDS-DMA kernel takes operands of 16-byte chunks: A and B 16-byte
  * aligned, K, lda, ldb (and N when b_trans == 0) multiples of 8 (F32: 4), and
- * the operands under 2 GiB; others are staged through registers.  Variant
+ * the operands under 2 GiB; others, and fp32 products with a short K, are staged
+ * through registers, or not at all with next to no K.  Variant
  * NKL_GEMM_NAIVE takes a one-tile-per-wavefront kernel (the same fp32
  * accumulation).
- * The work is enqueued on `stream` as one kernel launch, or as two over
- * column ranges when the large tiles would leave a partial last round of
- * workgroups; nothing is allocated, and the call can be captured in a graph.
+ * The work is enqueued on `stream` as one kernel launch, as two over column
+ * ranges when the large tiles would leave a partial last round of workgroups,
+ * or as more over ranges of C when one would pass HIP's limit of 2^32 threads;
+ * nothing is allocated, and the call can be captured in a graph.
  */
 int nkl_gemm(const void* A, const void* B, void* C, const void* R,
              int M, int N, int K, long lda, long ldb, long ldc, long ldr,

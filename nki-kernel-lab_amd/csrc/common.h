@@ -352,6 +352,8 @@ namespace nkl {
 int set_error(int code, const char* fmt, ...);
 // HIP takes fewer than 2^32 threads along x in one launch.
 constexpr long kMaxGridThreads = (1L << 32) - 1;
+// CUs of the current device (256 on MI355X, and with no device).
+int cu_count();
 // Checks hipGetLastError() after a launch; returns NKL_OK or NKL_ELAUNCH.
 int check_launch(const char* what);
 }  // namespace nkl

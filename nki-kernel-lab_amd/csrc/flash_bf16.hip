@@ -1247,13 +1247,6 @@ void flash_bf16_w1_kernel(AttnArgs p, Work w) {
 
 namespace {
 
-int cu_count() {
-  int dev = 0, n = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 256;
-  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 256;
-  return n;
-}
-
 // Kernels: teams of wavefronts sharing SIMDs (8 wavefronts per workgroup, or
 // 4 with two workgroups per CU); the software-pipelined kernel with one
 // wavefront per SIMD and 32 queries (4 per workgroup) or 64 queries (2 or 4

@@ -2,15 +2,16 @@
 //
 // gemm_dma_kernel, the hot path: operands of 16-byte chunks (bf16, fp16 and
 // fp32) staged by the buffer unit, tiles from 32x32 to 256x256.
-// gemm_reg_kernel: any alignment, staged through registers.
+// gemm_reg_kernel: any alignment, staged through registers; fp32 products with
+// a short K too.
 // gemm_pack_kernel, gemm_reduce_kernel: with a workspace (nkl_gemm_ws), large
 // unaligned 16-bit products copy their operands into aligned rows for the
 // first kernel, and few-tile products with a long K split it over workgroups.
 //
-// Naive kernel (variant "naive"): each wavefront computes one 32x32 tile of C
+// Naive kernel (variant "naive", and unaligned products with next to no K):
+// each wavefront computes one 32x32 tile of C
 // reading its operands straight from global memory at every K step -- no
 // on-chip reuse, like the reference's matmul_naive.
-#include <atomic>
 #include <cstdlib>
 #include <cstring>
 #include <type_traits>
@@ -1023,20 +1024,6 @@ static DmaTile choose_tile(const GemmArgs& a, int batch) {
   return kT64x64K2;
 }
 
-// CUs of the current device (256 on MI355X), read once per device (threads
-// that race to read it store the same value).
-static int gemm_cus() {
-  static std::atomic<int> cus[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  int n = cus[dev].load(std::memory_order_relaxed);
-  if (n == 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cus[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
-}
-
 // Rows and columns of a tile.
 static void tile_dims(DmaTile t, int& bm, int& bn) {
   switch (t) {
@@ -1074,7 +1061,7 @@ struct TilePlan {
 static TilePlan plan_tiles(const GemmArgs& a, DmaTile t, int batch, bool swiglu) {
   TilePlan best{t, 0, t};
   if (batch != 1 || forced_tile() >= 0 || round_step_us(t) == 0.0) return best;
-  const long cus = gemm_cus();
+  const long cus = cu_count();
   const double nk = (a.K + 63) / 64;
   auto cost = [&](DmaTile x, int n) {
     int bm, bn;
