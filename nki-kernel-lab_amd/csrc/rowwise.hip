@@ -14,10 +14,12 @@
 // 16 bytes are read and written with the same 16-byte instructions at the
 // element's own alignment (gfx950 takes them at any address); the elements
 // ahead of the row's first 64-byte boundary and its last ones go one to a
-// lane.  One wavefront per row with element loads and three sweeps took 316 us
-// at 1000 x 20000 fp32 and 252 at 66 x 31363; sixteen wavefronts holding the
-// row take 35.3 (4.5 TB/s) and 6.8.  Rows past 65536 elements take the looped
-// kernels, which re-read the row (from L2) once per pass.
+// lane.  One wavefront per row with element loads and three sweeps took 315 us
+// for the softmax of 1000 x 20000 fp32 and 336 of 66 x 31363, inputs rotated
+// through twice the last-level cache (276 and 173 with them in the cache);
+// sixteen wavefronts holding the row take 26.8 (6.0 TB/s) and 7.7 (24.0 and 6.3).
+// Rows past 65536 elements take the looped kernels, which re-read the row (from
+// L2) once per pass.
 #include <math.h>
 
 #include <type_traits>
@@ -124,9 +126,10 @@ __device__ __forceinline__ float row_sum(float v, float* red) {
 // nkilab/kernels/norm.py:65-89: neg_max = -max(x); e = exp(x + neg_max) with
 // the row sum in fp32; rinv = 1 / sum; y = e * rinv rounded once.
 // Wavefronts per SIMD the compiler makes room for: two 1024-thread workgroups a
-// CU where their rows' registers (32 values a lane) allow it (1000 x 20000 fp32
-// softmax 35.4 -> 30.3 us).  The unaligned form would spill (500 x 20001 17.1
-// -> 19.0).
+// CU where their rows' registers (32 values a lane) allow it (softmax, rotated
+// inputs, us, in brackets inputs in the cache: 1000 x 20000 fp32 30.8 -> 26.8 (30.4
+// -> 24.0), 1000 x 32768 bf16 27.3 -> 22.7).  The unaligned form would spill (500 x
+// 20001 16.5 -> 18.3 (15.7 -> 18.2)).
 constexpr int row_waves(int wpr, int nv, int e, bool al) { return al && wpr == 16 && nv * e <= 32 ? 8 : 1; }
 
 template <typename T, int WPR, int NV, bool AL>
@@ -437,8 +440,9 @@ static bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 // fp32 -> fp16 6.3 / 5.7; past one round one wavefront is level or ahead: 3000
 // x 2048 bf16 softmax 5.7 / 6.3).  Sixteen vectors a lane turn at `deep_rows`
 // (fp32 softmax 1024 x 4096 7.6 / 6.0 but 1536 x 4096 9.0 / 9.7).  128 values a
-// lane (16 vectors in 16 bits) always go to four times the wavefronts (4096 x
-// 8192 26.0 / 22.1; four / sixteen: 1000 x 32768 33.5 / 27.7).
+// lane (16 vectors in 16 bits) always go to four times the wavefronts (bf16
+// softmax 4096 x 8192 25.2 / 21.0; four / sixteen: 1000 x 32768 24.1 / 22.7,
+// RMSNorm 31.8 / 22.2).
 struct RowPlan {
   int wpr, nv;
 };

@@ -540,7 +540,7 @@ def test_flash_fp32_64_query_blocks(H, Hkv, S, d, scale):
     (1400, 1400, 1, 4, None), (1024, 512, 33, 32, None), (256, 128, 129, 28, 4.0), (256, 256, 192, 32, -0.3),
     (384, 384, 31, 64, None), (640, 160, 63, 64, None), (384, 128, 100, 36, 4.0), (256, 256, 130, 64, -0.3),
     (144, 48, 1, 128, None), (144, 48, 63, 128, None), (150, 50, 191, 96, 3.0), (112, 28, 200, 128, None),
-    (112, 112, 321, 100, -0.1)])
+    (112, 112, 321, 100, -0.1), (64, 16, 1430, 20, None)])
 def test_flash_fp32_many_short_heads(H, Hkv, S, d, scale):
     """The same edges on launches of many short heads, whose kernel takes keys
     in steps of 32."""
