@@ -525,6 +525,29 @@ def test_flash_fp32_against_float64(H, Hkv, S, d, scale):
     assert (ob[:, S] == 7).all()
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,Hkv,S,d", [
+    (7, 7, 2500, 64), (16, 4, 1537, 64), (24, 8, 1323, 64), (18, 9, 2047, 40), (17, 17, 2000, 32),  # blocks, pairs
+    (6, 3, 3000, 64), (5, 5, 4096, 24), (3, 1, 6000, 64), (8, 8, 4050, 48), (9, 3, 4000, 64), (1, 1, 16384, 64)])
+def test_narrow_heads_at_every_schedule(dt, H, Hkv, S, d):
+    """Head dims up to 64 on both sides of the lines of their schedule rule (the
+    second row: the wider heads' rule), sampled queries of every head against
+    float64 on the same inputs."""
+    from nkilab import ops
+
+    g = torch.Generator(device="cuda").manual_seed(S + d)
+    q, k, v = (torch.randn(n, S, d, generator=g, device="cuda").to(dt) for n in (H, Hkv, Hkv))
+    o = ops.attention(q, k, v)
+    rows = torch.tensor(sorted({0, 1, 31, 63, 64, 127, 128, S // 3, S // 2, S - 65, S - 64, S - 2, S - 1}), device="cuda")
+    kd, vd = (t.double().repeat_interleave(H // Hkv, 0) for t in (k, v))
+    s = torch.matmul(q[:, rows].double(), kd.transpose(1, 2).contiguous()) * d ** -0.5
+    s.masked_fill_(torch.arange(S, device="cuda")[None, :] > rows[:, None], -float("inf"))
+    ref = torch.matmul(torch.softmax(s, -1), vd)
+    for h in range(H):
+        assert rel_err(_np(o[h, rows]), ref[h].cpu().numpy()) <= BF16_TOL, h
+    assert torch.isfinite(o).all()
+
+
 @pytest.mark.parametrize("H,Hkv,S,d,scale", [
     (130, 130, 1, 4, None), (135, 45, 16, 32, None), (70, 70, 65, 32, 4.0), (9, 3, 1027, 28, -0.3),
     (132, 132, 63, 36, None), (130, 65, 64, 64, -0.3), (68, 68, 127, 64, 4.0), (46, 23, 129, 64, None),
